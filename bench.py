@@ -274,17 +274,16 @@ def bc_bench(npa, ctx, args):
     G.free()
 
 
-COLOR_METRIC = "graph-color GTEPS + %HBM peak @R-MAT s20, dependency counting vs the reference's rounds, exact"
+COLOR_METRIC = "graph-color GTEPS + %HBM peak @R-MAT s20, dependency solve vs the reference's rounds, exact"
 
 
 def color_bench(npa, ctx, args):
     """--config color: GRAPH_COLOR_GPU on R-MAT scale 20 (1,048,576 vertices, 16,777,216 edges,
     ids permuted).  Modes: `rounds` = the reference's algorithm (every uncolored vertex re-checks
-    its smaller neighbours each round), `depcount` = the dependency-counting frontier; both are
+    its smaller neighbours each round), `depcount` = the dependency solve in id order; both are
     compared with the oracle (int32, exact).  GTEPS = m / step time.  Algorithmic bytes of
-    depcount = 8 per edge (col read by the count and the fill passes) + 12 per smaller-id edge
-    (its notify entry written and read, its counter decremented) + 40 per vertex (row bounds
-    twice 16, notify bounds twice 16, counter 4, color 4)."""
+    depcount = 4 per edge (col) + 4 per smaller-id edge (the neighbour's color) + 8 per vertex
+    (row bound, color)."""
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
     import oracle
     G = npa.Graph.rmat(ctx, 20, 16, wmin=1, wmax=1, seed=7)
@@ -316,7 +315,7 @@ def color_bench(npa, ctx, args):
                "sample": "oracle one-pass coloring (increasing ids) over the whole graph, one thread, %.2f s; "
                          "both GPU methods equal it: %s" % (tc, exact)}
     best = results["depcount"]
-    b_alg = 8.0 * G.m + 12.0 * m_small + 40.0 * G.n
+    b_alg = 4.0 * G.m + 4.0 * m_small + 8.0 * G.n
     achieved = b_alg / (best["device_ms"] * 1e-3) / 1e9
     line = {
         "metric": COLOR_METRIC, "value": round(best["gteps"], 3), "unit": "GTEPS", "n_gpus": 1, "steps": args.steps,
@@ -327,7 +326,7 @@ def color_bench(npa, ctx, args):
                    "smaller_id_edges": m_small, "colors": int(outs["depcount"].max())},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "k_color_count+k_color_fill+k_color_step (rounds captured in hipGraphs)", "bytes_per_launch": b_alg},
+                     "kernel": "k_color_tickets+k_color_solve (one launch in id order)", "bytes_per_launch": b_alg},
         "cpu_baseline": cpu, "exact": exact,
         "modes": {k: {kk: (round(vv, 4) if isinstance(vv, float) else vv) for kk, vv in v.items()}
                   for k, v in results.items()},

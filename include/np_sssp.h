@@ -398,9 +398,9 @@ int np_bc(np_ctx *ctx, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc
  * 14-35, 779-834)  The reference's rounds give every vertex v
  *     color[v] = 1 + max { color[u] : v -> u, u < v }   (1 when there is no such u),
  * whatever the thread timing; color_out[n] receives these int32 values (graph.colorArray).
- * method 0: dependency counting over the transposed smaller-neighbour lists, O(m) work;
+ * method 0: one launch that solves the recurrence in the order of the ids, O(m) work;
  * method 1: the reference's rounds as they are, O(rounds x m) (the baseline).
- * stats: iterations = rounds, kernel_ms = device time of the whole call. */
+ * stats: iterations = rounds (the largest color), kernel_ms = device time of the whole call. */
 int np_color(np_ctx *ctx, np_graph *g, int32_t method, int32_t *color_out, np_stats *stats);
 
 /* ---- PageRank: PAGERANK_GPU --------------------------------------------------------------

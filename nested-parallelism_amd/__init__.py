@@ -442,7 +442,7 @@ class Context:
         return out, st
 
     def color(self, g, method=0):
-        """Graph coloring of GRAPH_COLOR_GPU: method 0 dependency counting, 1 the reference's
+        """Graph coloring of GRAPH_COLOR_GPU: method 0 in the order of the ids, 1 the reference's
         rounds.  Returns (color int32[n], Stats)."""
         out = np.empty(g.n, np.int32)
         st = Stats()

@@ -9,14 +9,19 @@
 //     color[v] = 1 + max { color[u] : v -> u, u < v }   (1 when there is no such u),
 // the length of the longest path of decreasing ids that starts at v.
 //
-// MI355X mapping (method 0): the same values in O(m) work instead of O(rounds * m).  dep[v]
-// counts the edges v -> u with u < v; the transposed lists notify[u] = { v : v -> u, u < v }
-// are built once (count, rocPRIM scan, scatter; one wavefront per vertex).  Round c's frontier is the vertices of color
-// c; expanding it decrements dep[v] for every v in their notify lists, and a vertex whose count
-// reaches zero in round c gets color c + 1 and joins the next frontier.  There are as many
-// rounds as colors (about a thousand on R-MAT s20) and each is small, so no round waits on the
-// host: one kernel per round, one wavefront per frontier vertex, the frontier count read on the
-// device; rounds are captured 30 to a hipGraph and replayed until the frontier is empty.
+// MI355X mapping (method 0): the recurrence is a triangular solve in the order of the ids, so it
+// is solved without rounds.  The vertices are cut, in id order, into tickets of at most COL_EDGES
+// edges: runs of consecutive short rows, or one chunk of a long row.  A wavefront takes the next
+// ticket, reads its edges once into registers and looks up the colors of the smaller neighbours;
+// edges whose neighbour has no color yet are polled, and a vertex whose edges are all settled gets
+// its color with one store.  Every dependency has a smaller id (or is an earlier chunk of the same
+// row), so it belongs to the same wavefront or to a ticket taken earlier, and the wavefront that
+// holds the lowest unfinished ticket never waits for anything unstarted: the solve ends whatever
+// the number of resident wavefronts.  No transposed lists, no counters and no atomic per edge
+// (atomics run at 27 G/s on the whole chip).  R-MAT s20 (1,048,576 / 16,777,216, about 1,080
+// colors): 1.8 ms on the device, 1.7 us per hop of the longest chain, against 35.1 ms with one
+// launch per color over a frontier fed by per-edge counters; a 1000 x 1000 grid with 1 % long-range
+// edges (47,311 colors): 32 ms against 191.
 // Method 1 runs the reference's rounds as they are (every uncolored vertex re-checks its
 // smaller neighbours each round, one host readback per round): the baseline.
 #include <hip/hip_runtime.h>
@@ -33,92 +38,185 @@ static int col_grid(long long work, int cap) {
     return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
-// dep[v] = #{v -> u : u < v}; ncnt[u] += 1 for each such edge.  One wavefront per vertex, lanes
-// over its edges (a hub's edges would serialise in one thread).
-__global__ void k_color_count(const int *row, const int *col, int n, int *dep, long long *ncnt) {
-    const int lane = col_lane();
-    const long long nw = (long long)gridDim.x * (blockDim.x >> 6);
-    for (long long v = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); v < n; v += nw) {
-        int d = 0;
-        for (int k = row[v]; k < row[v + 1]; k += 64) {
-            const int e = k + lane;
-            const bool small = e < row[v + 1] && col[e] < v;
-            if (small) atomicAdd((unsigned long long *)&ncnt[col[e]], 1ull);
-            d += __popcll(__ballot(small));
-        }
-        if (lane == 0) dep[v] = d;
-    }
-}
+// One workgroup per CU and 256 edges per ticket: every wavefront that waits polls, and polls of a
+// color that many others wait for queue behind one another and behind its store.  R-MAT s20, ms:
+// 1.82 with 4 edges per lane and 1 workgroup per CU (2: 1.91), with 8 edges 2.21 (2: 2.30, 4: 2.53,
+// 8: 13.0); a pause between polls only adds to the hop (8 per CU 4.8, 2 per CU 2.32-2.53).
+constexpr int COL_UNR = 4;                 // edges per lane
+constexpr int COL_WGS = 1;                 // workgroups per CU
+constexpr int COL_EDGES = 64 * COL_UNR;    // edges per ticket at most
+constexpr int COL_BLOCK = 64;              // a run lies inside a block of this many vertices
+constexpr unsigned long long COL_SPIN_LIMIT = 1ull << 24;
 
-// notify lists: ncol[nrow[u] + k] = v for the edges v -> u, u < v (cursor[] starts at 0); one
-// wavefront per vertex, so a hub's slot reservations are issued 64 at a time.
-__global__ void k_color_fill(const int *row, const int *col, int n, const long long *nrow, int *cursor, int *ncol) {
-    const int lane = col_lane();
-    const long long nw = (long long)gridDim.x * (blockDim.x >> 6);
-    for (long long v = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); v < n; v += nw)
-        for (int k = row[v]; k < row[v + 1]; k += 64) {
-            const int e = k + lane;
-            if (e < row[v + 1]) {
-                const int u = col[e];
-                if (u < v) ncol[nrow[u] + atomicAdd(&cursor[u], 1)] = (int)v;
+// Tickets of one block of COL_BLOCK vertices, in id order: emit(first vertex, count) for a run of
+// rows with at most COL_EDGES edges together, emit(vertex, -1 - chunk) for chunk after chunk of a
+// longer row.
+template <class F>
+__device__ __forceinline__ void col_cut(const int *row, long long v0, long long v1, F emit) {
+    long long first = v0;
+    int acc = 0, r0 = row[v0];
+    for (long long v = v0; v < v1; ++v) {
+        const int r1 = row[v + 1], d = r1 - r0;
+        r0 = r1;
+        if (d > COL_EDGES || acc > COL_EDGES - d) {
+            if (v > first) emit((int)first, (int)(v - first));
+            first = v;
+            acc = 0;
+            if (d > COL_EDGES) {
+                for (int j = 0; j <= (d - 1) / COL_EDGES; ++j) emit((int)v, -1 - j);
+                first = v + 1;
+                continue;
             }
         }
+        acc += d;
+    }
+    if (v1 > first) emit((int)first, (int)(v1 - first));
 }
 
-// Appends v to q (wave-aggregated) when `take`; every lane of the wave calls it.
-__device__ __forceinline__ void col_append(bool take, int v, int *q, int *qn) {
-    const unsigned long long want = __ballot(take);
-    if (want == 0) return;
-    const int lane = col_lane();
-    const int leader = __ffsll((long long)want) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(qn, __popcll(want));
-    base = __shfl(base, leader);
-    if (take) q[base + __popcll(want & ((1ull << lane) - 1))] = v;
-}
-
-// Round 1: the vertices with no smaller out-neighbour.
-__global__ void k_color_init(const int *dep, int n, int *color, int *q, int *qn) {
-    for (long long base = (long long)blockIdx.x * blockDim.x; base < n; base += (long long)gridDim.x * blockDim.x) {
-        const long long v = base + threadIdx.x;
-        const bool take = v < n && dep[v] == 0;
-        if (v < n) color[v] = take ? 1 : 0;
-        col_append(take, (int)v, q, qn);
+// Tickets per block into cnt[block] (FILL false), or written from at[block] on (FILL true).
+template <bool FILL>
+__global__ void k_color_tickets(const int *row, int n, int *cnt, const int *at, int2 *tick) {
+    const long long nb = ((long long)n + COL_BLOCK - 1) / COL_BLOCK;
+    for (long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x; b <= nb; b += (long long)gridDim.x * blockDim.x) {
+        if (!FILL && b == nb) cnt[b] = 0;
+        if (b == nb) continue;
+        const long long v0 = b * COL_BLOCK, v1 = v0 + COL_BLOCK < n ? v0 + COL_BLOCK : n;
+        int k = FILL ? at[b] : 0;
+        col_cut(row, v0, v1, [&](int v, int what) {
+            if (FILL) tick[k] = make_int2(v, what);
+            ++k;
+        });
+        if (!FILL) cnt[b] = k;
     }
 }
 
-// Round r of the dependency-counting drive (every kernel of a captured chunk is one round):
-// the frontier q_in (count *qn_in, all of one color c) decrements the counters of its notify
-// lists; a vertex whose counter reaches zero gets c + 1 and joins q_out.  *qn_zero is the
-// output count of the next round: zeroed here (nothing reads it during this round).  A round
-// with an empty frontier does nothing else, so a chunk may run past the last color.
-__global__ __launch_bounds__(256) void k_color_step(const int *q_in, const int *qn_in, int *q_out, int *qn_out,
-                                                    int *qn_zero, const long long *nrow, const int *ncol, int *dep,
-                                                    int *color, int *rounds) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *qn_zero = 0;
-    const int ne = *qn_in;
-    if (ne == 0) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *rounds += 1;
-    const int c = color[q_in[0]];
+// One wavefront's ticket in LDS.
+struct ColWave {
+    int row[COL_BLOCK + 1];  // edge offsets of its vertices
+    int best[COL_BLOCK];     // largest settled neighbour color
+    int wait[COL_BLOCK];     // edges without one
+    int color[COL_BLOCK];    // color once stored, else 0
+};
+
+__device__ __forceinline__ int col_load(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void col_store(int *p, int v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// LDS of one wavefront: its lanes run in step, so only the compiler has to keep the order.
+__device__ __forceinline__ void col_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The solve: wavefronts take tickets until none is left (ntick = the number of tickets, on the
+// device).  What bounds it is the longest chain of dependencies (about as many hops as colors),
+// each hop one store and the poll that sees it; the edges themselves are read once.  The last
+// chunk of a long row waits for part[] of the other chunks (their largest color + 1).
+// ctl[0] = next ticket, ctl[1] = largest color, ctl[2] = set when a poll ran out of patience (the
+// launch then drains).
+__global__ __launch_bounds__(256) void k_color_solve(const int *row, const int *col, const int2 *tick, const int *ntick,
+                                                     int *part, int *color, int *ctl) {
+    __shared__ ColWave s_w[4];
+    ColWave &w = s_w[threadIdx.x >> 6];
     const int lane = col_lane();
-    const long long nw = (long long)gridDim.x * (blockDim.x >> 6);
-    for (long long o = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); o < ne; o += nw) {
-        const int u = q_in[o];
-        const long long e0 = nrow[u], e1 = nrow[u + 1];
-        for (long long k = e0; k < e1; k += 64) {  // one wavefront per frontier vertex
-            const long long i = k + lane;
-            bool take = false;
-            int v = 0;
-            if (i < e1) {
-                v = ncol[i];
-                if (atomicSub(&dep[v], 1) == 1) {  // its last smaller neighbour was colored now
-                    color[v] = c + 1;
-                    take = true;
+    const int nt = *ntick;
+    int top = 0;
+    for (;;) {
+        int t = 0;
+        if (lane == 0) t = atomicAdd(&ctl[0], 1);
+        t = __builtin_amdgcn_readfirstlane(t);
+        if (t >= nt) break;
+        const int2 tk = tick[t];
+        const int v0 = tk.x, nv = tk.y < 0 ? 1 : tk.y, chunk = tk.y < 0 ? -1 - tk.y : 0;
+        if (lane < nv) {
+            w.row[lane] = row[v0 + lane];
+            w.best[lane] = 0;
+            w.wait[lane] = 0;
+            w.color[lane] = 0;
+        }
+        if (lane == 0) w.row[nv] = row[v0 + nv];
+        col_order();
+        const int e0 = w.row[0] + chunk * COL_EDGES;
+        const int left = w.row[nv] - e0;                      // edges from this ticket's first on
+        const int ne = left < COL_EDGES ? left : COL_EDGES;
+        const bool leads = left <= COL_EDGES;                 // stores colors (else: its part only)
+        int next = leads ? t - chunk : t;                     // parts [next, t) still to be seen
+        int u[COL_UNR], sl[COL_UNR], c[COL_UNR];
+#pragma unroll
+        for (int k = 0; k < COL_UNR; ++k) u[k] = 64 * k + lane < ne ? col[e0 + 64 * k + lane] : -1;
+#pragma unroll
+        for (int k = 0; k < COL_UNR; ++k) {  // owner: the last vertex whose offset is at or before the edge
+            int o = 0;
+#pragma unroll
+            for (int step = COL_BLOCK / 2; step > 0; step >>= 1)
+                if (o + step < nv && w.row[o + step] - e0 <= 64 * k + lane) o += step;
+            sl[k] = o;
+            if (u[k] >= v0 + o) u[k] = -1;  // only smaller neighbours count
+        }
+#pragma unroll
+        for (int k = 0; k < COL_UNR; ++k) c[k] = u[k] >= 0 && u[k] < v0 ? col_load(color + u[k]) : 0;
+#pragma unroll
+        for (int k = 0; k < COL_UNR; ++k) {
+            if (u[k] < 0) continue;
+            if (c[k]) { atomicMax(&w.best[sl[k]], c[k]); u[k] = -1; }
+            else atomicAdd(&w.wait[sl[k]], 1);
+        }
+        bool mine = lane < nv;   // this lane's vertex (or part) is not stored yet
+        bool fresh = false;      // a vertex of the ticket got its color in the last round
+        unsigned long long spins = 0;
+        for (;;) {
+            col_order();
+            const bool ready = mine && next == t && w.wait[lane] == 0;
+            if (ready) {
+                const int cv = w.best[lane] + 1;
+                if (leads) {
+                    w.color[lane] = cv;
+                    col_store(color + v0 + lane, cv);
+                    top = cv > top ? cv : top;
+                } else {
+                    col_store(part + t, cv);
+                }
+                mine = false;
+            }
+            if (__ballot(mine) == 0) break;
+            fresh = __ballot(ready) != 0;
+            col_order();
+            // a color of the ticket's own vertices settles its successors from LDS; only without
+            // one are the other wavefronts' colors read again
+#pragma unroll
+            for (int k = 0; k < COL_UNR; ++k) {
+                c[k] = 0;
+                if (u[k] >= v0) c[k] = w.color[u[k] - v0];
+                else if (u[k] >= 0 && !fresh) c[k] = col_load(color + u[k]);
+            }
+            if (!fresh && next < t) {
+                const int p = next + lane < t ? col_load(part + next + lane) : 1;
+                if (__ballot(p == 0) == 0) {
+                    if (p > 1) atomicMax(&w.best[0], p - 1);
+                    next = next + 64 < t ? next + 64 : t;
                 }
             }
-            col_append(take, v, q_out, qn_out);
+#pragma unroll
+            for (int k = 0; k < COL_UNR; ++k) {
+                if (c[k] == 0) continue;
+                atomicMax(&w.best[sl[k]], c[k]);
+                atomicSub(&w.wait[sl[k]], 1);
+                u[k] = -1;
+            }
+            if (!fresh && (++spins & 1023) == 0) {
+                const int stop = __builtin_amdgcn_readfirstlane(col_load(&ctl[2]));
+                if (stop || spins > COL_SPIN_LIMIT) {
+                    if (lane == 0) col_store(&ctl[2], 1);
+                    return;
+                }
+            }
         }
+        col_order();
     }
+    for (int o = 32; o > 0; o >>= 1) { const int x = __shfl_xor(top, o); top = x > top ? x : top; }
+    if (lane == 0 && top) atomicMax(&ctl[1], top);
 }
 
 // The reference's round as it is (method 1): every uncolored vertex checks its smaller
@@ -141,36 +239,27 @@ __global__ void k_color_round(const int *row, const int *col, int n, int *color,
     }
 }
 
-hipError_t launch_color_count(const int *row, const int *col, int n, int *dep, long long *ncnt, hipStream_t s) {
-    hipLaunchKernelGGL(k_color_count, dim3(col_grid((long long)n * 64, 8192)), dim3(256), 0, s, row, col, n, dep, ncnt);
-    return hipGetLastError();
+long long color_blocks(int n) { return ((long long)n + COL_BLOCK - 1) / COL_BLOCK; }
+// a run or first chunk per vertex at most, and a further chunk per COL_EDGES edges
+long long color_ticket_cap(int n, long long m) { return (long long)n + m / COL_EDGES + 1; }
+hipError_t color_scan(void *temp, size_t *temp_bytes, const int *in, int *out, int n, hipStream_t s) {
+    return rocprim::exclusive_scan(temp, *temp_bytes, in, out, 0, (size_t)color_blocks(n) + 1, rocprim::plus<int>(), s);
 }
-hipError_t launch_color_fill(const int *row, const int *col, int n, const long long *nrow, int *cursor, int *ncol,
-                             hipStream_t s) {
-    hipLaunchKernelGGL(k_color_fill, dim3(col_grid((long long)n * 64, 8192)), dim3(256), 0, s, row, col, n, nrow,
-                       cursor, ncol);
-    return hipGetLastError();
-}
-hipError_t launch_color_init(const int *dep, int n, int *color, int *q, int *qn, hipStream_t s) {
-    hipLaunchKernelGGL(k_color_init, dim3(col_grid(n, 8192)), dim3(256), 0, s, dep, n, color, q, qn);
-    return hipGetLastError();
-}
-hipError_t launch_color_step(const int *q_in, const int *qn_in, int *q_out, int *qn_out, int *qn_zero,
-                             const long long *nrow, const int *ncol, int *dep, int *color, int *rounds, int num_cus,
-                             hipStream_t s) {
-    // frontiers average ~n / colors vertices: a small grid that strides, since a round that ends at
-    // once still pays for dispatching every workgroup
-    hipLaunchKernelGGL(k_color_step, dim3(num_cus * 2), dim3(256), 0, s, q_in, qn_in, q_out, qn_out, qn_zero, nrow, ncol,
-                       dep, color, rounds);
+hipError_t launch_color_solve(const int *row, const int *col, int n, long long m, const ColorBufs &b, int num_cus,
+                              hipStream_t s) {
+    const long long nb = color_blocks(n);
+    const dim3 tgrid(col_grid(nb + 1, 4096));
+    hipLaunchKernelGGL(k_color_tickets<false>, tgrid, dim3(256), 0, s, row, n, b.cnt, (const int *)nullptr, (int2 *)nullptr);
+    size_t tb = b.temp_bytes;
+    hipError_t e = color_scan(b.temp, &tb, b.cnt, b.at, n, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_color_tickets<true>, tgrid, dim3(256), 0, s, row, n, (int *)nullptr, b.at, b.tick);
+    hipLaunchKernelGGL(k_color_solve, dim3(col_grid((nb + m / COL_EDGES) * 64, num_cus * COL_WGS)), dim3(256), 0, s, row, col, b.tick, b.at + nb,
+                       b.part, b.color, b.ctl);
     return hipGetLastError();
 }
 hipError_t launch_color_round(const int *row, const int *col, int n, int *color, int c, int *nonstop, hipStream_t s) {
     hipLaunchKernelGGL(k_color_round, dim3(col_grid(n, 8192)), dim3(256), 0, s, row, col, n, color, c, nonstop);
     return hipGetLastError();
 }
-// Exclusive prefix of in[0..n] into out[0..n] (in[n] = 0 gives out[n] = total).
-hipError_t color_scan(void *temp, size_t *temp_bytes, const long long *in, long long *out, int n, hipStream_t s) {
-    return rocprim::exclusive_scan(temp, *temp_bytes, in, out, 0ll, (size_t)n + 1, rocprim::plus<long long>(), s);
-}
-
 }  // namespace np

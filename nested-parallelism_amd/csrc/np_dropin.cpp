@@ -336,7 +336,7 @@ void BC_GPU() {
 
 // GRAPH_COLOR_GPU (apps/graph-color/src/gpu/graph_color_wrapper.cu:662-699): solutions 0-12
 // differ in how the rounds assign vertices to threads and all give the same colors; each runs
-// np_color (dependency counting).  Other solution numbers compute nothing, as the reference's
+// np_color (method 0).  Other solution numbers compute nothing, as the reference's
 // switch does.  The caller's main allocates graph.colorArray (graph_color.cpp:99-105).
 void GRAPH_COLOR_GPU() {
     np_ctx *c = ctx_for_device();

@@ -181,16 +181,21 @@ hipError_t launch_bc_accum(const BcDev &b, const int *ent_v, const unsigned *ent
 hipError_t launch_bc_to_float(const double *bc, int n, float *out, hipStream_t s);
 
 // ---- color.hip: graph coloring (longest decreasing-id path labels) -----------------------
-hipError_t launch_color_count(const int *row, const int *col, int n, int *dep, long long *ncnt, hipStream_t s);
-hipError_t launch_color_fill(const int *row, const int *col, int n, const long long *nrow, int *cursor, int *ncol,
-                             hipStream_t s);
-hipError_t launch_color_init(const int *dep, int n, int *color, int *q, int *qn, hipStream_t s);
-// One dependency-counting round (graph-capturable: no host values depend on the frontier).
-hipError_t launch_color_step(const int *q_in, const int *qn_in, int *q_out, int *qn_out, int *qn_zero,
-                             const long long *nrow, const int *ncol, int *dep, int *color, int *rounds, int num_cus,
-                             hipStream_t s);
+// Dependency solve.  cnt, at: color_blocks(n) + 1 ints; tick, part: color_ticket_cap(n, m);
+// color: n; ctl: 3.  part, color and ctl hold zeros before it; after it ctl[1] = the largest
+// color, ctl[2] != 0 when a bounded wait expired.
+struct ColorBufs {
+    int *cnt, *at, *part, *color, *ctl;
+    int2 *tick;
+    void *temp;
+    size_t temp_bytes;  // of color_scan (temp null queries it)
+};
+long long color_blocks(int n);
+long long color_ticket_cap(int n, long long m);
+hipError_t color_scan(void *temp, size_t *temp_bytes, const int *in, int *out, int n, hipStream_t s);
+hipError_t launch_color_solve(const int *row, const int *col, int n, long long m, const ColorBufs &b, int num_cus,
+                              hipStream_t s);
 hipError_t launch_color_round(const int *row, const int *col, int n, int *color, int c, int *nonstop, hipStream_t s);
-hipError_t color_scan(void *temp, size_t *temp_bytes, const long long *in, long long *out, int n, hipStream_t s);
 
 // ---- pagerank.hip: PageRank over the in-edge CSR ------------------------------------------
 // Rows by length: < PR_HEAVY entries PR_GROUP lanes each; < PR_HUGE one wavefront each (med);

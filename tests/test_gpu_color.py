@@ -54,3 +54,48 @@ def test_gpu_graph_color_cli_matches_oracle(tmp_path, orc, solution):
     assert "Execution time:" in r.stderr
     ref = orc.color(g["row"], g["col"])
     assert out.read_text().splitlines() == ["Node %d: %d" % (i + 1, c) for i, c in enumerate(ref)]
+
+
+def _long_rows(n, lens, seed):
+    """n vertices of 3 edges each, except vertex n - 1 - k, which has lens[k] (most to smaller ids)."""
+    rng = np.random.default_rng(seed)
+    deg = np.full(n, 3, np.int64)
+    deg[n - len(lens):] = lens[::-1]
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(deg)
+    return row, rng.integers(0, n, int(row[-1])).astype(np.int32)
+
+
+@pytest.mark.parametrize("case", ["rows_at_ticket_edge", "long_rows", "long_rows_linked", "path", "path_down",
+                                  "one_block_minus", "one_block", "one_block_plus", "empty_rows", "one_hub"])
+def test_color_ticket_boundaries_match_oracle(npa, ctx, orc, case):
+    """Tickets hold at most 256 edges inside blocks of 64 vertices: rows just below, at and above
+    that, rows of many chunks, chunks that depend on one another, and the longest chains."""
+    if case == "rows_at_ticket_edge":
+        row, col = _long_rows(300, [255, 256, 257, 1, 0, 256, 511, 512, 513], 71)
+    elif case == "long_rows":
+        row, col = _long_rows(20000, [70000, 16385, 16384, 5000, 257], 72)
+    elif case == "long_rows_linked":                  # every long row reads the long rows before it
+        row, col = _long_rows(3000, [900] * 200, 73)
+        col[row[2800]:] = 2800 + col[row[2800]:] % 200
+    elif case in ("path", "path_down"):               # a chain of n dependencies, or none
+        n = 5000
+        row = np.minimum(np.arange(n + 1), n - 1).astype(np.int32)
+        col = np.arange(1, n, dtype=np.int32)
+        if case == "path":
+            row = np.maximum(np.arange(n + 1) - 1, 0).astype(np.int32)
+            col = np.arange(n - 1, dtype=np.int32)
+    elif case == "empty_rows":
+        row, col = np.zeros(1001, np.int32), np.zeros(0, np.int32)
+    elif case == "one_hub":                           # more chunks than one look at the parts covers
+        row, col = _long_rows(500, [256 * 150 + 1], 74)
+    else:
+        n = {"one_block_minus": 63, "one_block": 64, "one_block_plus": 65}[case]
+        row, col = _long_rows(n, [4], 75)
+    G = npa.Graph.from_csr(ctx, row, col, np.ones(len(col), np.int32))
+    ref = orc.color(row, col)
+    for _ in range(2):
+        got, st = ctx.color(G)
+        assert np.array_equal(got, ref), case
+        assert st.iterations == int(ref.max())
+    G.free()
