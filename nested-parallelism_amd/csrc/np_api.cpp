@@ -198,6 +198,7 @@ struct Pack {
     int kshift = 0;          // dist rows of 2^kshift sources
     std::vector<int> inst;   // batch instance of each lane
     Space sp;
+    bool unpacked = false;   // the batch's result buffer holds the last solve's distances
 };
 
 struct np_batch {
@@ -216,6 +217,8 @@ struct np_batch {
     int *row = nullptr, *col = nullptr, *w = nullptr;  // concatenated graphs (or borrowed)
     bool owns_graph = false;
     Space sp;
+    ConcatOut *parts = nullptr;         // per concatenated instance: where its result goes
+    bool unpermuted = false;            // `out` holds the last solve's renumbered instances
     int *out = nullptr;                 // results in original ids (unpacked / mapped back)
     long long out_total = 0;
 };
@@ -652,6 +655,7 @@ static void batch_release(np_batch *b) {
     for (Pack *pk : b->packs) { pk->sp.release(); delete pk; }
     b->packs.clear();
     if (b->owns_graph) { dfree(b->row); dfree(b->col); dfree(b->w); }
+    dfree(b->parts);
     dfree(b->out);
     b->nconcat = 0;
 }
@@ -1584,6 +1588,13 @@ static int build_concat(np_ctx *c, np_batch *b, const std::vector<int> &ids, np_
         HIPCHK(launch_fill_lut(s.lut, b->base[ids[t]] / G, ((long long)g->n + G - 1) / G, t, c->stream));
     }
     HIPCHK(hipMemcpyAsync(s.inst, inst.data(), sizeof(int2) * (size_t)cnt, hipMemcpyHostToDevice, c->stream));
+    std::vector<ConcatOut> parts(cnt);
+    for (int t = 0; t < cnt; ++t) {
+        const np_graph *g = uniq[gi[t]];
+        parts[t] = ConcatOut{b->out_off[ids[t]], g->rl.active ? g->rl.old2new : nullptr, inst[t].x, g->n};
+    }
+    HIPCHK(dalloc(&b->parts, (size_t)cnt));
+    HIPCHK(hipMemcpyAsync(b->parts, parts.data(), sizeof(ConcatOut) * (size_t)cnt, hipMemcpyHostToDevice, c->stream));
     if ((rc = ensure_src(c, s, cnt))) return rc;
     std::vector<int> slots(cnt);
     for (int t = 0; t < cnt; ++t) {
@@ -1733,6 +1744,8 @@ int np_batch_solve(np_ctx *c, np_batch *b, const np_sched *sched, np_stats *stat
     }
     const bool unit = b->unit != 0;
     const int inf = unit ? UNDEFINED : INF;
+    for (Pack *pk : b->packs) pk->unpacked = false;
+    b->unpermuted = false;
     np_stats acc;
     std::memset(&acc, 0, sizeof acc);
     acc.drive = -1;
@@ -1818,24 +1831,32 @@ int np_batch_solve(np_ctx *c, np_batch *b, const np_sched *sched, np_stats *stat
 }
 
 // Instance i's distances in original vertex ids: unpacked from its pack, or mapped back
-// when its graph is renumbered, into the batch's result buffer.
-static int batch_result(np_ctx *c, np_batch *b, int i, const int **res) {
+// when its graph is renumbered, into the batch's result buffer.  The first request after a
+// solve unpacks its whole pack (maps back every renumbered concatenated instance) in one
+// launch; *launched tells whether this one did.
+static int batch_result(np_ctx *c, np_batch *b, int i, const int **res, bool *launched) {
     const np_graph *g = b->graphs[i];
     const int *old2new = g->rl.active ? g->rl.old2new : nullptr;
     const int pk = b->pack_of[i];
+    *launched = false;
     if (pk < 0 && !old2new) {
         *res = b->sp.dist + b->base[i];
         return NP_OK;
     }
     if (!b->out) HIPCHK(dalloc(&b->out, (size_t)b->out_total));
-    int *dst = b->out + b->out_off[i];
-    if (pk >= 0) {
+    bool &have = pk >= 0 ? b->packs[pk]->unpacked : b->unpermuted;
+    if (!have && pk >= 0) {
         const Pack *p = b->packs[pk];
-        HIPCHK(launch_unpack(p->sp.dist, p->kshift, b->lane_of[i], old2new, g->n, dst, c->stream));
-    } else {
-        HIPCHK(launch_unpermute(b->sp.dist + b->base[i], old2new, g->n, dst, c->stream));
+        UnpackTo to{};
+        to.count = (int)p->inst.size();
+        for (int j = 0; j < to.count; ++j) to.off[j] = b->out_off[p->inst[j]];
+        HIPCHK(launch_unpack(p->sp.dist, p->kshift, to, old2new, g->n, b->out, c->stream));
+    } else if (!have) {
+        HIPCHK(launch_unpermute_parts(b->sp.dist, b->sp.lut, b->parts, b->sp.nslots, b->out, c->stream));
     }
-    *res = dst;
+    *launched = !have;
+    have = true;
+    *res = b->out + b->out_off[i];
     return NP_OK;
 }
 
@@ -1844,7 +1865,8 @@ int np_batch_get(np_ctx *c, np_batch *b, int32_t i, int32_t *dist_out) {
     if (b->ctx != c) { set_error("batch belongs to another context or its context was destroyed"); return NP_ERR_ARG; }
     HIPCHK(hipSetDevice(c->device));
     const int *d = nullptr;
-    int rc = batch_result(c, b, i, &d);
+    bool launched = false;
+    int rc = batch_result(c, b, i, &d, &launched);
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(dist_out, d, sizeof(int) * (size_t)b->nverts[i], hipMemcpyDeviceToHost, c->stream));
     return ctx_sync(c);
@@ -1853,8 +1875,9 @@ int np_batch_get(np_ctx *c, np_batch *b, int32_t i, int32_t *dist_out) {
 int np_batch_device_dist(np_batch *b, int32_t i, const int32_t **d_dist) {
     if (!b || !d_dist || i < 0 || i >= b->count) { set_error("bad argument"); return NP_ERR_ARG; }
     if (!b->ctx) { set_error("the batch's context was destroyed"); return NP_ERR_ARG; }
-    int rc = batch_result(b->ctx, b, i, d_dist);
-    if (rc) return rc;
+    bool launched = false;
+    int rc = batch_result(b->ctx, b, i, d_dist, &launched);
+    if (rc || !launched) return rc;
     return ctx_sync(b->ctx);
 }
 

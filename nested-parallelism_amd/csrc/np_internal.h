@@ -111,9 +111,16 @@ hipError_t launch_copy_cls(const unsigned char *src, unsigned char *dst, long lo
 // Source-packed state: dist rows set to inf, source i of srcs[] at lane i (nsrc <= 2^kshift);
 // delta > 0 starts a priority window at T = delta.
 hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, int delta, hipStream_t s);
-// out[v] = dist[(map(v) << kshift) + lane], map = old2new or identity (old2new null).
-hipError_t launch_unpack(const int *dist, int kshift, int lane, const int *old2new, int n, int *out,
+// out[to.off[j] + v] = dist[(map(v) << kshift) + j] for j < to.count, map = old2new or identity
+// (old2new null).
+struct UnpackTo { long long off[PACK_MAX]; int count; };
+hipError_t launch_unpack(const int *dist, int kshift, const UnpackTo &to, const int *old2new, int n, int *out,
                          hipStream_t s);
+// out[p.off + v] = dist[p.base + p.old2new[v]] for every instance p of a concatenated part whose
+// old2new is not null (lut: slot >> LUT_SHIFT -> index into parts).
+struct ConcatOut { long long off; const int *old2new; int base, n; };
+hipError_t launch_unpermute_parts(const int *dist, const int *lut, const ConcatOut *parts, long long nslots, int *out,
+                                  hipStream_t s);
 
 // Persistent drive: one cooperative launch.  `wgs` workgroups of 256 threads.  A state
 // with kshift >= 0 runs the source-packed kernels (here and in compact/expand).

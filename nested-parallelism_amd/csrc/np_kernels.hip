@@ -1630,11 +1630,43 @@ __global__ void k_pk_init_sources(DevState st, const int *srcs, int nsrc, int T0
     }
 }
 
-__global__ void k_unpack(const int *dist, int kshift, int lane, const int *old2new, int n, int *out) {
-    for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-         v += (long long)gridDim.x * blockDim.x) {
+// Every source's distances of a pack, in original vertex ids, in one pass over the rows: a thread
+// reads one vertex's row (2^KS consecutive distances, a random row when renumbered) and the wave
+// stores 64 consecutive vertices of one source after another.  One source at a time re-read every
+// row per source.  16 sources of 16.8 M vertices (1 GB of rows), solve and all results: 29.5 ms with
+// a pass per source, 26.5 with this one; 32 sources of 4.2 M vertices 39.0 -> 35.6.
+template <int KS>
+__global__ __launch_bounds__(WG) void k_unpack(const int *dist, UnpackTo to, const int *old2new, int n, int *out) {
+    for (long long v = (long long)blockIdx.x * WG + threadIdx.x; v < n; v += (long long)gridDim.x * WG) {
         const long long r = old2new ? old2new[v] : v;
-        out[v] = dist[(r << kshift) + lane];
+        const int *row = dist + (r << KS);
+        int d[1 << KS];
+        if (KS >= 2) {
+#pragma unroll
+            for (int q = 0; q < (1 << KS) / 4; ++q) {
+                const int4 x = ((const int4 *)row)[q];
+                d[4 * q] = x.x; d[4 * q + 1] = x.y; d[4 * q + 2] = x.z; d[4 * q + 3] = x.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < (1 << KS); ++j) d[j] = row[j];
+        }
+#pragma unroll
+        for (int j = 0; j < (1 << KS); ++j)
+            if (j < to.count) out[to.off[j] + v] = d[j];
+    }
+}
+
+// Results of a concatenated part's renumbered instances, in original vertex ids, in one launch (a
+// launch and a wait per instance cost more than small graphs' results): a workgroup's slots belong
+// to one instance (slots are padded to 2^LUT_SHIFT per instance).
+__global__ __launch_bounds__(WG) void k_unpermute_parts(const int *dist, const int *lut, const ConcatOut *parts,
+                                                        long long nslots, int *out) {
+    static_assert((1 << LUT_SHIFT) % WG == 0, "a workgroup must lie in one instance");
+    for (long long base = (long long)blockIdx.x * WG; base < nslots; base += (long long)gridDim.x * WG) {
+        const ConcatOut p = parts[lut[base >> LUT_SHIFT]];
+        const long long v = base + threadIdx.x - p.base;
+        if (p.old2new && v < p.n) out[p.off + v] = dist[p.base + p.old2new[v]];
     }
 }
 
@@ -2055,10 +2087,27 @@ hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, i
     hipLaunchKernelGGL(k_pk_init_sources, dim3(1), dim3(64), 0, s, st, d_srcs, nsrc, delta > 0 ? delta : NO_WINDOW);
     return hipGetLastError();
 }
-hipError_t launch_unpack(const int *dist, int kshift, int lane, const int *old2new, int n, int *out,
+hipError_t launch_unpack(const int *dist, int kshift, const UnpackTo &to, const int *old2new, int n, int *out,
                          hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_unpack, dim3(grid_for(n, 256)), dim3(256), 0, s, dist, kshift, lane, old2new, n, out);
+    const dim3 grid(grid_for(n, WG));
+#define NP_UNPACK(K) hipLaunchKernelGGL(k_unpack<K>, grid, dim3(WG), 0, s, dist, to, old2new, n, out)
+    switch (kshift) {
+    case 0: NP_UNPACK(0); break;
+    case 1: NP_UNPACK(1); break;
+    case 2: NP_UNPACK(2); break;
+    case 3: NP_UNPACK(3); break;
+    case 4: NP_UNPACK(4); break;
+    case 5: NP_UNPACK(5); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef NP_UNPACK
+    return hipGetLastError();
+}
+hipError_t launch_unpermute_parts(const int *dist, const int *lut, const ConcatOut *parts, long long nslots, int *out,
+                                  hipStream_t s) {
+    if (nslots <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_unpermute_parts, dim3(grid_for(nslots, WG)), dim3(WG), 0, s, dist, lut, parts, nslots, out);
     return hipGetLastError();
 }
 hipError_t launch_decide(const DevState &st, const SchedDev &sp, int it_off, hipStream_t s) {
