@@ -11,6 +11,9 @@ namespace np {
 constexpr int BAR_LEAVES = 32;
 struct alignas(128) BarLeaf { unsigned long long n; unsigned long long pad[15]; };
 
+// Largest number of sources packed into one distance row.
+constexpr int PACK_MAX = 32;
+
 // Device-side control block of one solve.
 struct Ctrl {
     BarLeaf leaf[BAR_LEAVES]; // grid barrier: cumulative arrivals per leaf (own cache lines)
@@ -29,6 +32,10 @@ struct Ctrl {
     long long pairs_total;    // source-packed: sum over iterations of queued (vertex, source) pairs
     long long edges_total;    // source-packed: sum over iterations of the queued vertices' out-degrees
     long long items_total;    // source-packed: ... of out-degree x queued sources ((edge, source) items)
+    int filt;                 // source-packed bound filter: 0 off, 1 the next compaction computes every
+                              // vertex's bound, 2 on (foff, fmask set)
+    unsigned fmask;           // sources that take part in the bounds
+    int foff[PACK_MAX];       // per source: its distance at the hub when the bounds were computed
 };
 
 // Everything an expansion / compaction touches.  Indices are "slots": the vertex ids of
@@ -67,10 +74,12 @@ struct DevState {
     // (once per flagging; bm[1] marks the held vertices); hold_cls 0 = never
     int hold_cls;
     int hold_min;
+    // source-packed bound filter (see pk_bound_code): one byte per vertex, null = off; a code step
+    // is 2^fshift, and at least fmin sources have to have reached the hub (solver id 0)
+    unsigned char *bound;
+    int fshift;
+    int fmin;
 };
-
-// Largest number of sources packed into one distance row.
-constexpr int PACK_MAX = 32;
 
 struct SchedDev {
     int learned;            // evaluate the MLP each iteration

@@ -306,8 +306,13 @@ __device__ __forceinline__ int find_class(const long long *pre, long long idx) {
     return c;
 }
 
+// Filtered packed expansions (pk_edge_tile): vertices of class c per tile, about 768 edges, for the
+// classes below PK_TILE_CLS.
+__device__ __forceinline__ int pk_tile_vertices(int c) { return c <= 4 ? 64 : 1024 >> c; }
+constexpr int PK_TILE_CLS = 11;
+
 // Thread 0 builds the tables from the frontier's class counts (already in tb.cnt).
-__device__ __noinline__ void build_tables(ItemTables &tb, const Cfg &cfg) {
+__device__ __noinline__ void build_tables(ItemTables &tb, const Cfg &cfg, bool filt = false) {
     long long acc[4] = {0, 0, 0, 0};
     for (int c = 0; c < NCLS; ++c) {
         for (int t = 0; t < 4; ++t) tb.pre[t][c] = acc[t];
@@ -315,7 +320,8 @@ __device__ __noinline__ void build_tables(ItemTables &tb, const Cfg &cfg) {
         if (c >= cfg.b3) acc[0] += n * grid_chunks(c);
         else if (c >= cfg.b2) acc[1] += n;
         else if (c >= cfg.b1) acc[2] += n;
-        else acc[3] += (n + 63) / 64;
+        else if (!filt) acc[3] += (n + 63) / 64;
+        else acc[3] += (n + pk_tile_vertices(c) - 1) / pk_tile_vertices(c);
     }
     for (int t = 0; t < 4; ++t) tb.pre[t][NCLS] = acc[t];
 }
@@ -688,6 +694,20 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
             else ctrl->error = NP_ERR_NOT_CONVERGED;
         }
         return;
+    }
+    if (st.bound && threadIdx.x < 64) {
+        // bound filter: one iteration after enough of the sources reached the hub (their first
+        // distances there are far from final) the bounds are computed and switched on
+        const int f = ld_coherent(&ctrl->filt);
+        const int j = threadIdx.x;
+        const int d = f < 2 && j < (1 << st.kshift) ? ld_coherent(st.dist + j) : st.inf;
+        const unsigned m = (unsigned)__ballot(d < st.inf);
+        if (f == 1) {
+            if (j < PACK_MAX) ctrl->foff[j] = d < st.inf ? d : 0;
+            if (j == 0) { ctrl->fmask = m; ctrl->filt = 2; }
+        } else if (f == 0 && j == 0 && __popc(m) >= st.fmin) {
+            ctrl->filt = 1;
+        }
     }
     Cfg cfg = decide(sp, s_cnt, ctrl->iters);
     if (threadIdx.x == 0) {
@@ -1112,19 +1132,74 @@ __device__ __forceinline__ void pk_relax_vertex(const DevState &st, int u, unsig
     }
 }
 
+// Bound filter of a pack on a skewed graph.  Once every source has reached the core, most edges a
+// packed expansion reads improve nothing (R-MAT s18, 16 sources, CPU model: 0.40 of 4.8 x m edge
+// rows improve), yet each costs a random row of distances and a lane per pending source.  The
+// sources' distances at a vertex differ mostly by one offset per source, its distance off[s] at the
+// hub: max over s of (dist[v][s] - off[s]) is a bound within a few units of every source's own
+// value.  An edge (u, v) with min over u's pending s of (dist[u][s] - off[s]) + w >= bound[v] can
+// improve no source, so it is dropped after reading one byte.  The bounds are upper bounds whatever
+// off[] is (any constants would do) and stay valid without upkeep, because distances only fall; a
+// vertex's bound is refreshed when it is expanded.  Sources that had not reached the hub when off[]
+// was taken (fmask clear) have no part in the bounds, and edges of a vertex pending for one of them
+// are never dropped.  16 sources of R-MAT s24, one solve: the four heaviest filtered expansions
+// 5.2 / 4.8 / 3.7 / 1.6 -> 4.1 / 3.2 / 2.4 / 1.1 ms, for 0.29 ms of bounds; what is left of them is
+// the stream of the rows themselves.
+// A byte holds ceil((bound - FBASE) / 2^fshift) with FBASE = -64 steps, 255 = no bound.
+constexpr int FBASE_STEPS = 64;
+constexpr int FNONE = 255;
+constexpr int FLOW = -(1 << 30), FHIGH = 1 << 30;  // below / above every normalised distance in use
+
+__device__ __forceinline__ int pk_bound_code(int b, int fshift) {
+    if (b >= FHIGH) return FNONE;
+    const int x = b + (FBASE_STEPS << fshift);
+    const int q = x <= 0 ? 0 : (x + (1 << fshift) - 1) >> fshift;
+    return q < FNONE ? q : FNONE;
+}
+// true when an edge with candidate value thr + w (relative to FBASE) may improve a source of the
+// vertex with bound code q
+__device__ __forceinline__ bool pk_may_improve(int q, int thr, int w, int fshift) {
+    return q == FNONE || thr + w < (q << fshift);
+}
+// One thread over vertex v's whole row: its bound (*hi) over the sources in `mask`, and the least
+// normalised distance (*lo) of the sources pending in m, FLOW when one of them is not in mask.
+__device__ __forceinline__ void pk_row_bound(const DevState &st, long long v, const int *off, unsigned mask, unsigned m,
+                                             int *hi, int *lo) {
+    const int *row = st.dist + (v << st.kshift);
+    int h = FLOW, l = (m & ~mask) ? FLOW : FHIGH;
+    for (int q = 0; q < (1 << st.kshift) / 4; ++q) {
+        const int4 x = ((const int4 *)row)[q];
+        const int d[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int y = d[k] >= st.inf ? FHIGH : d[k] - off[4 * q + k];
+            const bool in = (mask >> (4 * q + k)) & 1u;
+            h = in && y > h ? y : h;
+            l = in && ((m >> (4 * q + k)) & 1u) && y < l ? y : l;
+        }
+    }
+    *hi = h;
+    *lo = l;
+}
+// What an expansion needs of the filter, per lane: source lane & (row length - 1).
+struct PkFilt {
+    const int *off;   // [PACK_MAX] in LDS
+    unsigned mask;
+};
+
 // Wavefront-scope form of pk_relax_vertex (stride 64) with the neighbour tile staged in LDS: the
 // wavefront copies up to PK_TILE consecutive edges' col (and w) into its own LDS slice with
 // coalesced loads, one edge per lane per load, then takes the edges of its relaxation steps from
 // there.  Without staging every step re-reads col/w from global memory, q = 64 / P distinct edges
 // per load, and waits for them before its distance gathers.  tcol / tw: the wavefront's slice.
 constexpr int PK_TILE = 256;
-constexpr bool PK_STAGE = true;
 // a group of UNR steps spans up to UNR * 64 edges (one pending source): a tile must hold one,
 // or the rounded tile below would be empty and its loop would not advance
 static_assert(PK_TILE >= UNR * 64 && PK_TILE % 64 == 0, "PK_TILE must hold a step group of one source");
-template <bool UNIT>
-__device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, int u, unsigned M, int e0, int e1,
-                                                       int *tcol, int *tw) {
+constexpr int PK_SLICE = 2 * PK_TILE;  // LDS entries per wavefront
+template <bool UNIT, bool FILT>
+__device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, const PkFilt &pf, int u, unsigned M, int e0,
+                                                       int e1, bool first, int *tcol, int *tw) {
     M = (unsigned)__builtin_amdgcn_readfirstlane((int)M);
     const int P = __popc(M);
     if (P == 0 || e0 >= e1) return;
@@ -1134,13 +1209,35 @@ __device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, int u
     const int eo = lane / P, j = lane - eo * P;
     const bool on = eo < q;
     const int s = on ? nth_set_bit(M, j) : 0;
-    const int du = on ? ld_coherent(st.dist + (((unsigned)u << ks) + (unsigned)s)) : 0;
+    int du, thr = 0;
+    if (FILT) {
+        // u's whole row: its bound, the least pending normalised distance and every lane's du
+        const int sl = lane & ((1 << ks) - 1);
+        const int d = ld_coherent(st.dist + (((unsigned)u << ks) + (unsigned)sl));
+        const bool in = (pf.mask >> sl) & 1u;
+        const int nd = d >= st.inf ? FHIGH : d - pf.off[sl];
+        int hi = in ? nd : FLOW;
+        int lo = !((M >> sl) & 1u) ? FHIGH : in ? nd : FLOW;
+        for (int o = 1; o < (1 << ks); o <<= 1) {
+            const int x = __shfl_xor(hi, o), y = __shfl_xor(lo, o);
+            hi = x > hi ? x : hi;
+            lo = y < lo ? y : lo;
+        }
+        if (first && lane == 0) st.bound[u] = (unsigned char)pk_bound_code(hi, st.fshift);
+        thr = lo + (FBASE_STEPS << st.fshift);
+        du = __shfl(d, s);
+    } else {
+        du = on ? ld_coherent(st.dist + (((unsigned)u << ks) + (unsigned)s)) : 0;
+    }
     const int rs = lane - j > 0 ? lane - j : 0;
     const bool last = j == P - 1 || lane == 63;
     const int span = UNR * q;                  // edges of one group of UNR steps (<= PK_TILE)
-    const int tile = (PK_TILE / span) * span;  // whole groups per tile: no group straddles two tiles
+    // unfiltered: whole groups per tile, so that no group straddles two tiles; filtered: the edges
+    // that may improve gather in the slice until another tile might not fit
+    const int tile = FILT ? PK_TILE : (PK_TILE / span) * span;
+    int have = 0;
     for (int tb = e0; tb < e1; tb += tile) {
-        const int nt = e1 - tb < tile ? e1 - tb : tile;
+        int nt = e1 - tb < tile ? e1 - tb : tile;
         __builtin_amdgcn_wave_barrier();       // the previous tile's reads come first
         int c[PK_TILE / 64], wv[PK_TILE / 64];
 #pragma unroll
@@ -1148,12 +1245,32 @@ __device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, int u
             const int i = lane + 64 * r;
             const int ic = tb + (i < nt ? i : nt - 1);  // lanes past the tile re-read its last edge
             c[r] = st.col[ic];
-            if (!UNIT) wv[r] = st.w[ic];
+            wv[r] = UNIT ? 1 : st.w[ic];
         }
+        if (FILT) {
+            int b[PK_TILE / 64];
 #pragma unroll
-        for (int r = 0; r < PK_TILE / 64; ++r) {
-            tcol[lane + 64 * r] = c[r];
-            if (!UNIT) tw[lane + 64 * r] = wv[r];
+            for (int r = 0; r < PK_TILE / 64; ++r) b[r] = 64 * r < nt ? (int)st.bound[c[r]] : 0;
+#pragma unroll
+            for (int r = 0; r < PK_TILE / 64; ++r) {
+                const bool keep = lane + 64 * r < nt && pk_may_improve(b[r], thr, wv[r], st.fshift);
+                const unsigned long long m = __ballot(keep);
+                if (keep) {
+                    const int at = have + __popcll(m & __lanemask_lt());
+                    tcol[at] = c[r];
+                    if (!UNIT) tw[at] = wv[r];
+                }
+                have += __popcll(m);
+            }
+            if (have <= PK_SLICE - PK_TILE && tb + tile < e1) continue;
+            nt = have;
+            have = 0;
+        } else {
+#pragma unroll
+            for (int r = 0; r < PK_TILE / 64; ++r) {
+                tcol[lane + 64 * r] = c[r];
+                if (!UNIT) tw[lane + 64 * r] = wv[r];
+            }
         }
         __builtin_amdgcn_wave_barrier();
         for (int e = eo; __ballot(on && e < nt) != 0; e += span) {
@@ -1239,8 +1356,108 @@ __device__ __forceinline__ void pk_lane_tile(const DevState &st, const int *q, c
     }
 }
 
-template <bool UNIT>
-__device__ void pk_expansion(const DevState &st, const int *q, const unsigned *qm, ItemTables &tb) {
+// Filtered tile: up to 64 queued vertices of one out-degree class (pk_tile_vertices), about 768
+// edges in all (cl = the class: degrees below 2^cl).  A lane reads one vertex's row (bound, least
+// pending value); then the tile's edges are spread over the lanes, one lane per edge, and those that may improve are listed in LDS; a
+// listed edge gets one lane per source of the row (2^kshift), so the sources that improve are one
+// ballot.  One vertex per wavefront spent a chain of seven dependent accesses on about 40 edges.
+// The listed edges 0 .. nt of the wave's slice; u, M: lane i holds the tile's vertex i.
+__device__ __forceinline__ void pk_relax_listed(const DevState &st, int u, unsigned M, const int *tcol, const int *tw,
+                                                const unsigned char *town, int nt) {
+    const int ks = st.kshift;
+    const int lane = lane_id();
+    const int s = lane & ((1 << ks) - 1), rs = lane - s;
+    const int per = 64 >> ks;  // edges per step
+    const unsigned rowmask = ks == 5 ? ~0u : (1u << (1 << ks)) - 1u;
+    for (int base = 0; base < nt; base += UNR * per) {
+        int tv[UNR], alt[UNR], cur[UNR];
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            const int i = base + k * per + (lane >> ks);
+            const int ic = i < nt ? i : 0;
+            const int o = town[ic];
+            const unsigned uo = (unsigned)__shfl(u, o);
+            const unsigned Mo = (unsigned)__shfl((int)M, o);
+            tv[k] = tcol[ic];
+            const bool pend = i < nt && ((Mo >> s) & 1u);
+            // cached: a value older than the vertex's last improvement only repeats what its next
+            // expansion does again
+            alt[k] = pend ? st.dist[(uo << ks) + (unsigned)s] + tw[ic] : 0;
+            cur[k] = pend ? ld_coherent(st.dist + (((unsigned)tv[k] << ks) + (unsigned)s)) : 0;
+        }
+        unsigned prev[UNR];
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            prev[k] = 1u;
+            const bool imp = alt[k] < cur[k];
+            if (imp) atomicMin(st.dist + (((unsigned)tv[k] << ks) + (unsigned)s), alt[k]);
+            const unsigned mine = (unsigned)(__ballot(imp) >> rs) & rowmask;
+            if (s == 0 && mine) prev[k] = atomicOr(&st.mflag[tv[k]], mine);
+        }
+#pragma unroll
+        for (int k = 0; k < UNR; ++k)
+            if (prev[k] == 0) atomicOr(&st.bm[0][tv[k] >> 5], 1u << (tv[k] & 31));
+    }
+}
+
+__device__ __forceinline__ void pk_edge_tile(const DevState &st, const PkFilt &pf, const int *q, const unsigned *qm,
+                                             long long qidx, int nvalid, int cl, int *tcol, int *tw, unsigned char *town) {
+    const int lane = lane_id();
+    int u = 0, s0 = 0, d = 0, thr = 0;
+    unsigned M = 0;
+    if (lane < nvalid) {
+        u = ld_coherent(q + qidx + lane);
+        M = ld_coherent_u(qm + qidx + lane);
+        s0 = st.row[u];
+        d = M ? st.row[u + 1] - s0 : 0;
+        int hi, lo;
+        pk_row_bound(st, u, pf.off, pf.mask, M, &hi, &lo);
+        st.bound[u] = (unsigned char)pk_bound_code(hi, st.fshift);
+        thr = lo + (FBASE_STEPS << st.fshift);
+    }
+    // 2^cl slots per vertex (its degree is at least half of that): a slot's vertex and edge are its
+    // bits, where a prefix sum of the degrees needs a search of six dependent shuffles per edge
+    const int total = nvalid << cl;
+    int have = 0;
+    for (int base = 0; base < total; base += UNR * 64) {
+        int o[UNR], c[UNR], wv[UNR], b[UNR];
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            const int kk = base + k * 64 + lane;
+            o[k] = (kk >> cl) & 63;
+            const int i = kk & ((1 << cl) - 1);
+            const int e = __shfl(s0, o[k]) + i;
+            const bool ok = i < __shfl(d, o[k]) && kk < total;
+            c[k] = ok ? st.col[e] : -1;
+            wv[k] = ok ? st.w[e] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) b[k] = c[k] >= 0 ? (int)st.bound[c[k]] : 0;
+        __builtin_amdgcn_wave_barrier();  // the list's previous reads come first
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            const int t = __shfl(thr, o[k]);
+            const bool keep = c[k] >= 0 && pk_may_improve(b[k], t, wv[k], st.fshift);
+            const unsigned long long m = __ballot(keep);
+            if (keep) {
+                const int at = have + __popcll(m & __lanemask_lt());
+                tcol[at] = c[k];
+                tw[at] = wv[k];
+                town[at] = (unsigned char)o[k];
+            }
+            have += __popcll(m);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (have > PK_SLICE - UNR * 64 || base + UNR * 64 >= total) {
+            pk_relax_listed(st, u, M, tcol, tw, town, have);
+            have = 0;
+        }
+    }
+}
+
+template <bool UNIT, bool FILT>
+__device__ void pk_expansion(const DevState &st, const PkFilt &pf, const int *q, const unsigned *qm, ItemTables &tb,
+                             int *tcol, int *tw, unsigned char *town) {
     const long long G = tb.pre[0][NCLS], K = tb.pre[1][NCLS], W = tb.pre[2][NCLS],
                     T = tb.pre[3][NCLS];
     for (long long k = blockIdx.x; k < K; k += gridDim.x) {
@@ -1253,8 +1470,6 @@ __device__ void pk_expansion(const DevState &st, const int *q, const unsigned *q
     const long long NW = (long long)gridDim.x * WAVES;
     const long long gw = (long long)blockIdx.x * WAVES + (threadIdx.x >> 6);
     const long long U = G + W + T;
-    __shared__ int s_tcol[WAVES][PK_TILE], s_tw[WAVES][PK_TILE];
-    int *tcol = s_tcol[threadIdx.x >> 6], *tw = s_tw[threadIdx.x >> 6];
     for (long long x = gw; x < U; x += NW) {
         if (x < G) {
             int c = find_class(tb.pre[0], x);
@@ -1268,23 +1483,23 @@ __device__ void pk_expansion(const DevState &st, const int *q, const unsigned *q
             int e0 = s + (j << GRID_CHUNK_SHIFT);
             int e1 = e0 + (1 << GRID_CHUNK_SHIFT);
             if (e1 > e) e1 = e;
-            if (PK_STAGE) pk_relax_vertex_staged<UNIT>(st, u, M, e0, e1, tcol, tw);
-            else pk_relax_vertex<UNIT>(st, u, M, e0, e1, lane_id(), 64);
+            pk_relax_vertex_staged<UNIT, FILT>(st, pf, u, M, e0, e1, j == 0, tcol, tw);
         } else if (x < G + W) {
             long long i = x - G;
             int c = find_class(tb.pre[2], i);
             long long qi = tb.seg[c] + (i - tb.pre[2][c]);
             int u = ld_coherent(q + qi);
             unsigned M = ld_coherent_u(qm + qi);
-            if (PK_STAGE) pk_relax_vertex_staged<UNIT>(st, u, M, st.row[u], st.row[u + 1], tcol, tw);
-            else pk_relax_vertex<UNIT>(st, u, M, st.row[u], st.row[u + 1], lane_id(), 64);
+            pk_relax_vertex_staged<UNIT, FILT>(st, pf, u, M, st.row[u], st.row[u + 1], true, tcol, tw);
         } else {
             long long t = x - G - W;
             int c = find_class(tb.pre[3], t);
             long long ti = t - tb.pre[3][c];
-            long long first = ti * 64;
-            int nvalid = (int)((long long)tb.cnt[c] - first < 64 ? (long long)tb.cnt[c] - first : 64);
-            pk_lane_tile<UNIT>(st, q, qm, tb.seg[c] + first, nvalid);
+            const int tv = FILT ? pk_tile_vertices(c) : 64;
+            long long first = ti * tv;
+            int nvalid = (int)((long long)tb.cnt[c] - first < tv ? (long long)tb.cnt[c] - first : tv);
+            if (FILT) pk_edge_tile(st, pf, q, qm, tb.seg[c] + first, nvalid, c, tcol, tw, town);
+            else pk_lane_tile<UNIT>(st, q, qm, tb.seg[c] + first, nvalid);
         }
     }
 }
@@ -1454,15 +1669,23 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     if (T != NO_WINDOW || st.hold_cls) flush_deferred(my_dc, my_dm, &s_dc, &s_dm, defer_cnt, defer_min);
 }
 
-// Lane-bin bound of a packed expansion (see PACK_LANE_CLS); the other bins keep theirs.
-__device__ __forceinline__ Cfg pk_cfg(Cfg c) {
-    if (c.b1 > PACK_LANE_CLS) c.b1 = PACK_LANE_CLS;
+// Lane-bin bound of a packed expansion (see PACK_LANE_CLS); the other bins keep theirs.  A filtered
+// expansion takes every class below PK_TILE_CLS as tiles.
+__device__ __forceinline__ Cfg pk_cfg(Cfg c, bool filt) {
+    if (filt) {
+        c.b1 = PK_TILE_CLS;
+        if (c.b2 < c.b1) c.b2 = c.b1;
+        if (c.b3 < c.b1) c.b3 = c.b1;
+    } else if (c.b1 > PACK_LANE_CLS) {
+        c.b1 = PACK_LANE_CLS;
+    }
     return c;
 }
 
 template <bool UNIT>
 __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) {
     __shared__ ItemTables tb;
+    __shared__ int s_tcol[WAVES][PK_TILE], s_tw[WAVES][PK_TILE];
     __shared__ int s_total;
     Ctrl *ctrl = st.ctrl;
     unsigned long long gen = 0;
@@ -1523,13 +1746,13 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             return;
         }
         Cfg cfg = decide(sp, tb.cnt, it);
-        if (threadIdx.x == 0) build_tables(tb, pk_cfg(cfg));
+        if (threadIdx.x == 0) build_tables(tb, pk_cfg(cfg, false));
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
         }
         __syncthreads();
-        pk_expansion<UNIT>(st, q_cur, qm_cur, tb);
+        pk_expansion<UNIT, false>(st, PkFilt{}, q_cur, qm_cur, tb, s_tcol[threadIdx.x >> 6], s_tw[threadIdx.x >> 6], nullptr);
         if (!grid_sync(ctrl, nb, gen)) return;
     }
 }
@@ -1547,6 +1770,30 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     }
     pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T,
                   ctrl->defer_cnt + pass % 3, ctrl->defer_min + pass % 3);
+}
+
+// Every vertex's bound, once: between the compaction and the decision that records the offsets (no
+// distance changes in between, so every workgroup sees those offsets).  A launch of its own: inside
+// the compaction, behind an untaken branch, it cost every compaction about 65 us on 16.8 M vertices.
+__global__ __launch_bounds__(WG) void k_pk_bounds(DevState st) {
+    __shared__ int s_off[PACK_MAX];
+    __shared__ unsigned s_mask;
+    Ctrl *ctrl = st.ctrl;
+    if (ld_coherent(&ctrl->done) || ld_coherent(&ctrl->error) || ld_coherent(&ctrl->filt) != 1) return;
+    if (threadIdx.x < 64) {
+        const int j = threadIdx.x;
+        const int d = j < (1 << st.kshift) ? ld_coherent(st.dist + j) : st.inf;  // the hub's row
+        const unsigned m = (unsigned)__ballot(d < st.inf);
+        if (j < PACK_MAX) s_off[j] = d < st.inf ? d : 0;
+        if (j == 0) s_mask = m;
+    }
+    __syncthreads();
+    for (long long v = (long long)blockIdx.x * WG + threadIdx.x; v < st.nslots; v += (long long)gridDim.x * WG)
+    {
+        int hi, lo;
+        pk_row_bound(st, v, s_off, s_mask, 0u, &hi, &lo);
+        st.bound[v] = (unsigned char)pk_bound_code(hi, st.fshift);
+    }
 }
 
 // The packed expansion is a latency-bound gather: it is held to 64 VGPRs so that eight waves share
@@ -1594,12 +1841,19 @@ __global__ __launch_bounds__(WG) void k_pk_count(DevState st, int it_off) {
     }
 }
 
-template <bool UNIT>
+// BOUND: the state has a bound filter (one more set of bodies; without it the kernel stays as small
+// as it was, which the windowed grid's expansion shows: 2 % of its solve).
+template <bool UNIT, bool BOUND>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_pk_expand(DevState st, int it_off) {
     __shared__ ItemTables tb;
+    constexpr int SLICE = BOUND ? PK_SLICE : PK_TILE;
+    __shared__ int s_tcol[WAVES][SLICE], s_tw[WAVES][SLICE];
+    __shared__ unsigned char s_town[BOUND ? WAVES : 1][BOUND ? PK_SLICE : 1];
+    __shared__ int s_off[PACK_MAX];
     Ctrl *ctrl = st.ctrl;
     if (ld_coherent(&ctrl->done) || ld_coherent(&ctrl->error) || ld_coherent(&ctrl->skip)) return;
     const int it = ld_coherent(&ctrl->it_base) + it_off;
+    const bool filt = BOUND && ld_coherent(&ctrl->filt) == 2;
     if (threadIdx.x < NCLS) {
         tb.cnt[threadIdx.x] = ld_coherent(st.cnt + (it % 3) * NCLS + threadIdx.x);
         tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
@@ -1608,10 +1862,15 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     if (threadIdx.x == 0) {
         Cfg cfg = make_cfg(ld_coherent(&ctrl->cfg_level), ld_coherent(&ctrl->cfg_klo),
                            ld_coherent(&ctrl->cfg_khi));
-        build_tables(tb, pk_cfg(cfg));
+        build_tables(tb, pk_cfg(cfg, filt), filt);
     }
+    if (filt && threadIdx.x < PACK_MAX) s_off[threadIdx.x] = ld_coherent(ctrl->foff + threadIdx.x);
     __syncthreads();
-    pk_expansion<UNIT>(st, st.queue[it & 1], st.qmask[it & 1], tb);
+    const PkFilt pf{s_off, filt ? ld_coherent_u(&ctrl->fmask) : 0u};
+    int *tcol = s_tcol[threadIdx.x >> 6], *tw = s_tw[threadIdx.x >> 6];
+    unsigned char *town = s_town[BOUND ? threadIdx.x >> 6 : 0];
+    if (BOUND && filt) pk_expansion<UNIT, BOUND>(st, pf, st.queue[it & 1], st.qmask[it & 1], tb, tcol, tw, town);
+    else pk_expansion<UNIT, false>(st, pf, st.queue[it & 1], st.qmask[it & 1], tb, tcol, tw, town);
 }
 
 __global__ void k_pk_init_sources(DevState st, const int *srcs, int nsrc, int T0) {
@@ -2067,6 +2326,7 @@ hipError_t launch_compact(const DevState &st, int it_off, bool batch, int wgs, h
     int g = (int)(need < wgs ? (need < 1 ? 1 : need) : wgs);
     if (st.kshift >= 0) {
         hipLaunchKernelGGL(k_pk_compact, dim3(g), dim3(WG), 0, s, st, it_off);
+        if (st.bound) hipLaunchKernelGGL(k_pk_bounds, dim3(wgs), dim3(WG), 0, s, st);
         if (st.count_work) hipLaunchKernelGGL(k_pk_count, dim3(wgs), dim3(WG), 0, s, st, it_off);
     } else {
         hipLaunchKernelGGL(k_compact, dim3(g), dim3(WG), 0, s, st, it_off);
@@ -2080,6 +2340,7 @@ hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, i
     if ((e = launch_fill_u32(st.bm[0], st.nwords, 0u, s)) != hipSuccess) return e;
     if (st.hold_cls && (e = launch_fill_u32(st.bm[1], st.nwords, 0u, s)) != hipSuccess) return e;
     if ((e = launch_fill_u32(st.mflag, st.nslots, 0u, s)) != hipSuccess) return e;
+    if (st.bound && (e = launch_fill_u32((unsigned *)st.bound, (st.nslots + 3) / 4, ~0u, s)) != hipSuccess) return e;
     if ((e = launch_fill_i32(st.cnt, 3 * NCLS, 0, s)) != hipSuccess) return e;
     if (st.sbcnt && (e = launch_fill_i32(st.sbcnt, 3, 0, s)) != hipSuccess) return e;
     if ((e = launch_fill_i32((int *)st.ctrl, (long long)(sizeof(Ctrl) / sizeof(int)), 0, s)) != hipSuccess)
@@ -2153,8 +2414,11 @@ hipError_t launch_expand(const DevState &st, const SchedDev &sp, int it_off, boo
     if (sp.scheme != NP_SCHEME_CONSOLIDATE) return launch_scheme(st, sp, it_off, unit, wgs, s);
     const bool push = sp.push != 0;
     if (st.kshift >= 0) {
-        if (unit) hipLaunchKernelGGL(k_pk_expand<true>, dim3(wgs), dim3(WG), 0, s, st, it_off);
-        else hipLaunchKernelGGL(k_pk_expand<false>, dim3(wgs), dim3(WG), 0, s, st, it_off);
+#define NP_PK(U, B) hipLaunchKernelGGL((k_pk_expand<U, B>), dim3(wgs), dim3(WG), 0, s, st, it_off)
+        if (unit) NP_PK(true, false);
+        else if (st.bound) NP_PK(false, true);
+        else NP_PK(false, false);
+#undef NP_PK
         return hipGetLastError();
     }
 #define NP_EXP(B, U, P) hipLaunchKernelGGL((k_expand<B, U, P>), dim3(wgs), dim3(WG), 0, s, st, it_off)

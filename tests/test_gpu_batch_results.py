@@ -45,3 +45,43 @@ def test_every_row_width_and_request_order(npa, ctx, orc, k, relabel):
     b.free()
     for g in [G] + small:
         g.free()
+
+
+@pytest.mark.parametrize("kind", ["rmat", "rmat_hold", "zero_weights", "large_weights", "too_large_weights",
+                                  "cut_off_sources"])
+@pytest.mark.parametrize("k", [3, 4, 5, 16, 31, 32])
+def test_bound_filter_is_exact(npa, ctx, orc, k, kind):
+    """Packs of a renumbered graph on the per-iteration drives drop edges by the vertices' bounds: row
+    widths 4..32, rows in every class around the tile and grid bins, weights at the ends of the
+    codes' range, and sources that never reach the hub (no part in the bounds)."""
+    rng = np.random.default_rng(200 + k)
+    ctx.set_option(npa.CTX_RELABEL, 1)
+    wmax = {"zero_weights": 0, "large_weights": 1 << 22, "too_large_weights": 1 << 26}.get(kind, 255)
+    try:
+        g0 = npa.Graph.rmat(ctx, 12, 24, wmin=0 if wmax == 0 else 1, wmax=max(wmax, 1), seed=300 + k)
+        row, col, w = g0.download()
+        if kind == "zero_weights":
+            w[:] = 0
+        srcs = [int(s) for s in npa.pick_sources(row, k, 4)]
+        if kind == "cut_off_sources":                 # a path that never enters the R-MAT part
+            n = len(row) - 1
+            row = np.concatenate([row, row[-1] + np.arange(1, 41)]).astype(np.int32)
+            col = np.concatenate([col, n + np.minimum(np.arange(1, 41), 39)]).astype(np.int32)
+            w = np.concatenate([w, rng.integers(1, 255, 40)]).astype(np.int32)
+            srcs[0] = n + 3
+            if k > 8:
+                srcs[1] = n
+        G = npa.Graph.from_csr(ctx, row, col, w)
+    finally:
+        ctx.set_option(npa.CTX_RELABEL, 2)
+    b = npa.Batch(ctx, [G] * k, srcs)
+    ref = [orc.dijkstra(row, col, w, s)[0] for s in srcs]
+    hold = 6 if kind == "rmat_hold" else 0
+    for level, lo, hi, drive in ((2, 4, 10, npa.DRIVE_GRAPH), (2, 4, 6, npa.DRIVE_HOSTLOOP), (1, 6, 6, npa.DRIVE_GRAPH),
+                                 (0, 3, 3, npa.DRIVE_HOSTLOOP), (2, 6, 12, npa.DRIVE_PERSISTENT)):
+        b.solve(npa.Sched(level=level, log2_t_lo=lo, log2_t_hi=hi, drive=drive, pack_hold=hold))
+        for i in range(k):
+            assert np.array_equal(b.get(i), ref[i]), (kind, k, level, drive, i)
+    b.free()
+    G.free()
+    g0.free()
