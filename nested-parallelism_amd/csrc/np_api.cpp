@@ -95,6 +95,7 @@ struct Space {
     DevState gst{};
     int gchunk = 0, gwgs = 0;
     bool gbatch = false, gunit = false;
+    long long edges = 0;  // of the instances solved in this space
     // largest edge weight of the graph(s) solved in this space, and whether a distance could
     // reach INF: (largest vertex count - 1) x max_w >= INF (checked after every solve)
     int max_w = 0;
@@ -333,10 +334,16 @@ static SchedDev make_schedd(np_ctx *c, const np_sched &s, int n_feat) {
     return d;
 }
 
-static int persistent_wgs(np_ctx *c, const np_sched &s, bool batch, bool unit, bool packed) {
+// Workgroups of a persistent solve over `edges` edges.  Every workgroup more makes the two grid
+// barriers of an iteration dearer, so a graph whose iterations are short gets one per CU (ER 65,536
+// / 1 M: 0.59 ms with 1, 0.64 with 4; grid 512^2: 1.20 and 1.32), a middling one two (grid 2048^2,
+// 17 M edges: 3.77 with 2, 3.94 with 4; learned on R-MAT s20, 17 M: 1.20 and 1.22), and only large
+// ones all that fit (R-MAT s22, 67 M: 5.6, 4.5, 4.2, 4.1 ms with 1 to 4).
+static int persistent_wgs(np_ctx *c, const np_sched &s, bool batch, bool unit, bool packed, long long edges) {
     int occ = persistent_max_wgs_per_cu(batch, unit, s.frontier == NP_FRONTIER_PUSH, packed);
     if (occ < 1) occ = 1;
-    int per = s.wgs_per_cu > 0 ? std::min(s.wgs_per_cu, occ) : occ;
+    const int fit = packed ? occ : edges <= (4ll << 20) ? 1 : edges <= (32ll << 20) ? std::min(2, occ) : occ;
+    int per = s.wgs_per_cu > 0 ? std::min(s.wgs_per_cu, occ) : fit;
     return per * c->num_cus;
 }
 
@@ -345,9 +352,12 @@ static int read_ctrl(np_ctx *c) {
     return ctx_sync(c);
 }
 
-// Whether a solve over graphs of up to n vertices and largest weight max_w needs the
-// distance-range check.
-static void set_guard(Space &s, long long n, int max_w) {
+// Adds an instance of graph g to the space: its edges, and whether its vertices and largest weight
+// make the distance-range check needed.
+static void set_guard(Space &s, const np_graph *g) {
+    const long long n = g->n;
+    const int max_w = g->max_w;
+    s.edges += g->m;
     s.max_w = std::max(s.max_w, max_w);
     s.guard = s.guard || (n - 1) * (long long)max_w >= (long long)INF;
 }
@@ -421,7 +431,7 @@ static int run_drive(np_ctx *c, Space &s, const DevState &st, const np_sched &sc
     // the reference's other schedules are per-iteration launches
     if (sd.scheme != NP_SCHEME_CONSOLIDATE && drive == NP_DRIVE_PERSISTENT) drive = NP_DRIVE_HOSTLOOP;
     if (drive == NP_DRIVE_PERSISTENT) {
-        int wgs = persistent_wgs(c, sch, batch, unit, st.kshift >= 0);
+        int wgs = persistent_wgs(c, sch, batch, unit, st.kshift >= 0, s.edges);
         HIPCHK(hipEventRecord(c->ev0, c->stream));
         hipError_t e = launch_persistent(st, sd, batch, unit, wgs, c->stream);
         if (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge) {
@@ -490,7 +500,7 @@ static int graph_space(np_ctx *c, np_graph *g) {
     std::memcpy(s.hist, g->hist, sizeof(s.hist));
     s.cls = g->cls;
     s.own_cls = false;
-    set_guard(s, g->n, g->max_w);
+    set_guard(s, g);
     int rc = space_alloc(c, s, true);
     if (rc) { s.release(); return rc; }
     if ((rc = ensure_src(c, s, 1))) return rc;
@@ -1000,7 +1010,7 @@ int np_sssp_device_noalloc(np_ctx *c, np_graph *g, int32_t src, const np_sched *
     s.nslots = g->n;
     std::memcpy(s.hist, g->hist, sizeof(s.hist));
     s.cls = g->cls;
-    set_guard(s, g->n, g->max_w);
+    set_guard(s, g);
     int seg[NCLS + 1];
     seg_from_hist(s.hist, seg, &s.qcap);
     s.nwords = (s.nslots + 31) / 32;
@@ -1522,7 +1532,7 @@ static int build_pack(np_ctx *c, np_batch *b, np_graph *g, const std::vector<int
     std::memcpy(s.hist, g->hist, sizeof(s.hist));
     s.cls = g->cls;
     s.own_cls = false;
-    set_guard(s, g->n, g->max_w);
+    set_guard(s, g);
     int rc = space_alloc(c, s, false);
     if (rc) return rc;
     HIPCHK(dalloc(&s.dist, (size_t)g->n << ks));
@@ -1588,7 +1598,7 @@ static int build_concat(np_ctx *c, np_batch *b, const std::vector<int> &ids, np_
         b->base[ids[t]] = (int)acc;
         inst[t] = make_int2((int)acc, (int)VB[gi[t]]);
         for (int k = 0; k < NCLS; ++k) s.hist[k] += g->hist[k];
-        set_guard(s, g->n, g->max_w);
+        set_guard(s, g);
         acc += ((long long)g->n + G - 1) / G * G;
         if (acc > 0x7FFFFFFFll - G) { set_error("batch exceeds 2^31 vertex slots"); return NP_ERR_CAPACITY; }
     }

@@ -32,6 +32,7 @@ struct Ctrl {
     long long pairs_total;    // source-packed: sum over iterations of queued (vertex, source) pairs
     long long edges_total;    // source-packed: sum over iterations of the queued vertices' out-degrees
     long long items_total;    // source-packed: ... of out-degree x queued sources ((edge, source) items)
+    int solo;                 // persistent drive: iterations of the last solo visit
     int filt;                 // source-packed bound filter: 0 off, 1 the next compaction computes every
                               // vertex's bound, 2 on (foff, fmask set)
     unsigned fmask;           // sources that take part in the bounds

@@ -288,6 +288,42 @@ __device__ __forceinline__ void lane_tile(const DevState &st, const PushCtx &pc,
     }
 }
 
+// Shortest rows: a lane per queued vertex walks its edges, UNR loads in flight.  No owner search;
+// the rows of neighbouring vertices share cache lines.
+template <bool BATCH, bool UNIT, bool PUSH, bool GUARD>
+__device__ __forceinline__ void lane_serial(const DevState &st, const PushCtx &pc, const int *q, long long qidx,
+                                            int nvalid) {
+    const int lane = lane_id();
+    int B = 0, VB = 0, s = 0, d = 0, du = 0;
+    if (lane < nvalid) {
+        const int slot = ld_coherent(q + qidx + lane);
+        decode<BATCH>(st, slot, B, VB);
+        const int v = slot - B;
+        s = st.row[VB + v];
+        d = st.row[VB + v + 1] - s;
+        du = ld_coherent(st.dist + slot);
+        if (PUSH) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
+    }
+    for (int i = 0; __ballot(i < d) != 0; i += UNR) {
+        int tv[UNR], alt[UNR], cur[UNR];
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            const bool ok = i + k < d;
+            tv[k] = ok ? B + st.col[s + i + k] : 0;
+            alt[k] = ok ? du + (UNIT ? 1 : st.w[s + i + k]) : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) cur[k] = i + k < d ? ld_coherent(st.dist + tv[k]) : 0;
+#pragma unroll
+        for (int k = 0; k < UNR; ++k) {
+            bool want = false;
+            int c = 0;
+            if (alt[k] < cur[k]) want = relax_tail<PUSH>(st, pc, tv[k], alt[k], c);
+            if (PUSH) push_wave(st, pc, want, tv[k], c);
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------
 // one expansion (all threads of every workgroup call it)
 // ------------------------------------------------------------------------------------
@@ -296,6 +332,7 @@ struct ItemTables {
     long long pre[4][NCLS + 1];  // 0 grid chunks, 1 workgroup items, 2 wavefront items, 3 lane tiles
     int cnt[NCLS];
     int seg[NCLS];
+    int tv;                      // single source: vertices per lane tile
 };
 
 __device__ __forceinline__ int find_class(const long long *pre, long long idx) {
@@ -311,19 +348,57 @@ __device__ __forceinline__ int find_class(const long long *pre, long long idx) {
 __device__ __forceinline__ int pk_tile_vertices(int c) { return c <= 4 ? 64 : 1024 >> c; }
 constexpr int PK_TILE_CLS = 11;
 
-// Thread 0 builds the tables from the frontier's class counts (already in tb.cnt).
-__device__ __noinline__ void build_tables(ItemTables &tb, const Cfg &cfg, bool filt = false) {
-    long long acc[4] = {0, 0, 0, 0};
-    for (int c = 0; c < NCLS; ++c) {
-        for (int t = 0; t < 4; ++t) tb.pre[t][c] = acc[t];
-        long long n = c == 0 ? 0 : tb.cnt[c];
-        if (c >= cfg.b3) acc[0] += n * grid_chunks(c);
-        else if (c >= cfg.b2) acc[1] += n;
-        else if (c >= cfg.b1) acc[2] += n;
-        else if (!filt) acc[3] += (n + 63) / 64;
-        else acc[3] += (n + pk_tile_vertices(c) - 1) / pk_tile_vertices(c);
+// Single-source work items.
+// Lane bin: vertices of degree below 2^SERIAL_CLS are walked one per lane; longer rows go to tiles
+// whose edges are spread over the lanes, of as many vertices (8 to 64) as give every wavefront a
+// tile (64 always: the widest ER 65,536 / 1 M frontier, 43 K vertices, filled 670 of 4,096
+// wavefronts; the tables, tiles and serial rows together: 0.82 -> 0.63 ms).
+constexpr int SERIAL_CLS = 3;
+
+enum TableKind { TABLES_SINGLE = 0, TABLES_PACKED = 1, TABLES_FILTERED = 2 };
+
+// The first wavefront builds the tables from the frontier's class counts (already in tb.cnt),
+// lane c for class c; nwaves = wavefronts of the expansion.
+__device__ __forceinline__ void build_tables(ItemTables &tb, const Cfg &cfg, TableKind kind, long long nwaves) {
+    const int c = lane_id();
+    const long long n = c >= 1 && c < NCLS ? tb.cnt[c] : 0;
+    int tv = 64;
+    if (kind == TABLES_SINGLE) {
+        long long lanes = c > SERIAL_CLS && c < cfg.b1 ? n : 0;
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) lanes += __shfl_xor(lanes, o);
+        lanes = __shfl(lanes, 0);
+        while (tv > 8 && lanes <= (tv >> 1) * nwaves) tv >>= 1;
+        if (c == 0) tb.tv = tv;
+        if (c <= SERIAL_CLS) tv = 64;
+    } else if (kind == TABLES_FILTERED) {
+        tv = c < PK_TILE_CLS ? pk_tile_vertices(c) : 1;
     }
-    for (int t = 0; t < 4; ++t) tb.pre[t][NCLS] = acc[t];
+    long long item[4];
+    item[0] = c >= cfg.b3 ? n * grid_chunks(c & 31) : 0;
+    item[1] = c >= cfg.b2 && c < cfg.b3 ? n : 0;
+    item[2] = c >= cfg.b1 && c < cfg.b2 ? n : 0;
+    item[3] = c < cfg.b1 ? (n + tv - 1) / tv : 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        long long x = item[t];
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+            const long long y = __shfl_up(x, o);
+            if (c >= o) x += y;
+        }
+        if (c < NCLS) tb.pre[t][c] = x - item[t];
+        if (c == NCLS - 1) tb.pre[t][NCLS] = x;
+    }
+}
+
+// Vertices of a frontier from its class counts (the first wavefront; the result in every lane).
+__device__ __forceinline__ long long frontier_size(const int *cnt) {
+    const int c = lane_id();
+    long long x = c >= 1 && c < NCLS ? cnt[c] : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
 }
 
 template <bool BATCH, bool UNIT, bool PUSH, bool GUARD>
@@ -383,9 +458,11 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
             long long t = u - G - W;
             int c = find_class(tb.pre[3], t);
             long long ti = t - tb.pre[3][c];
-            long long first = ti * 64;
-            int nvalid = (int)((long long)tb.cnt[c] - first < 64 ? (long long)tb.cnt[c] - first : 64);
-            lane_tile<BATCH, UNIT, PUSH, GUARD>(st, pc, q, tb.seg[c] + first, nvalid);
+            const int tv = c <= SERIAL_CLS ? 64 : tb.tv;
+            long long first = ti * tv;
+            int nvalid = (int)((long long)tb.cnt[c] - first < tv ? (long long)tb.cnt[c] - first : tv);
+            if (c <= SERIAL_CLS) lane_serial<BATCH, UNIT, PUSH, GUARD>(st, pc, q, tb.seg[c] + first, nvalid);
+            else lane_tile<BATCH, UNIT, PUSH, GUARD>(st, pc, q, tb.seg[c] + first, nvalid);
         }
     }
 }
@@ -398,8 +475,8 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
 // least distance among them to defer_cnt / defer_min.  T = INT_MAX queues every flag.
 constexpr int NO_WINDOW = 0x7FFFFFFF;
 
-// Single-source frontiers, and source-packed ones without a window, are sparse: a thread scans
-// one bitmap word and visits its set bits, so empty words cost one load.  With a priority window
+// Source-packed frontiers without a window are sparse: a thread scans one bitmap word and visits
+// its set bits, so empty words cost one load (single-source ones: see compaction_impl).  With a priority window
 // a source-packed frontier is dense (deferred vertices stay flagged and are re-read every pass):
 // there each thread owns CPT vertices of a tile of WG * CPT consecutive ones, so the lanes of a
 // wave read the class bytes, masks and distance rows of consecutive vertices and the 32 lanes of
@@ -439,50 +516,77 @@ __device__ __forceinline__ void flush_deferred(int my_dc, int my_dm, int *s_dc, 
     if (threadIdx.x == 0 && *s_dc) { atomicAdd(defer_cnt, *s_dc); atomicMin(defer_min, *s_dm); }
 }
 
+// A wave loads up to 64 words at once and takes the nonzero ones two at a time, a lane per vertex,
+// COMPACT_UNR pairs in flight; the vertices to queue gather in LDS as (offset, class).  A thread
+// per word, walking its bits, left all but n / 8192 workgroups idle and waited for every class: one
+// solve on the persistent drive, ER 65,536 / 1 M 0.94 -> 0.82 ms, grid 2048^2 5.12 -> 4.13.
+constexpr int COMPACT_UNR = 4;
 __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const unsigned char *cls, const int *seg_off,
                                                 long long nwords, int *cnt_out, int *q_out, const int *dist,
                                                 int T, int *defer_cnt, int *defer_min) {
+    __shared__ unsigned short s_list[WAVES][64 * 32];
     __shared__ int s_lc[NCLS], s_lb[NCLS];
     __shared__ int s_dc, s_dm;
+    static_assert(NCLS <= 32, "an entry holds 11 bits of offset and 5 of class");
     if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; }
     int my_dc = 0, my_dm = NO_WINDOW;
-    for (long long wb = (long long)blockIdx.x * WG; wb < nwords; wb += (long long)gridDim.x * WG) {
+    const int lane = lane_id(), half = lane & 31;
+    unsigned short *list = s_list[threadIdx.x >> 6];
+    // words per wave: all workgroups take part, but a tile is worth its counter reservations
+    const long long share = (nwords + (long long)gridDim.x * WAVES - 1) / ((long long)gridDim.x * WAVES);
+    const int wt = share < 8 ? 8 : share < 64 ? (int)share : 64;
+    const long long tile = (long long)WAVES * wt;
+    for (long long wb = (long long)blockIdx.x * tile; wb < nwords; wb += (long long)gridDim.x * tile) {
         if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;
-        __syncthreads();
-        const long long wi = wb + threadIdx.x;
-        const unsigned word0 = wi < nwords ? ld_coherent_u(bm + wi) : 0u;
-        unsigned word = word0, take = 0, drop = 0;
-        while (word) {
-            int b = __ffs(word) - 1;
-            word &= word - 1;
-            const long long slot = wi * 32 + b;
-            int c = cls[slot];
-            if (!c) { drop |= 1u << b; continue; }  // no out-edges: nothing to propagate
-            if (T != NO_WINDOW) {
-                int d = ld_coherent(dist + slot);
-                if (d >= T) { my_dc++; my_dm = d < my_dm ? d : my_dm; continue; }
+        const long long w0 = wb + (threadIdx.x >> 6) * wt;
+        const unsigned word = lane < wt && w0 + lane < nwords ? ld_coherent_u(bm + w0 + lane) : 0u;
+        unsigned long long nz = __ballot(word != 0);
+        int n = 0;
+        while (nz) {
+            int idx[COMPACT_UNR], c[COMPACT_UNR], d[COMPACT_UNR];
+            unsigned x[COMPACT_UNR];
+#pragma unroll
+            for (int k = 0; k < COMPACT_UNR; ++k) {
+                const int ia = __ffsll((long long)nz) - 1;
+                nz &= nz - 1;
+                const int ib = __ffsll((long long)nz) - 1;
+                nz &= nz - 1;
+                idx[k] = lane < 32 ? ia : ib;  // -1: none left
+                x[k] = __shfl(word, idx[k] < 0 ? 0 : idx[k]);
+                if (idx[k] < 0) x[k] = 0u;
+                c[k] = (x[k] >> half) & 1u ? (int)cls[(w0 + idx[k]) * 32 + half] : 0;
             }
-            take |= 1u << b;
-            atomicAdd(&s_lc[c], 1);
+            if (T != NO_WINDOW) {
+#pragma unroll
+                for (int k = 0; k < COMPACT_UNR; ++k)
+                    d[k] = c[k] ? ld_coherent(dist + (w0 + idx[k]) * 32 + half) : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < COMPACT_UNR; ++k) {
+                const bool defer = T != NO_WINDOW && c[k] && d[k] >= T;
+                if (defer) { my_dc++; my_dm = d[k] < my_dm ? d[k] : my_dm; }
+                const bool take = c[k] && !defer;  // no out-edges (class 0): dropped
+                const unsigned long long m = __ballot(take), kept = __ballot(defer);
+                if (take) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
+                n += __popcll(m);
+                const unsigned nw = (unsigned)(kept >> (lane & 32));
+                if (half == 0 && nw != x[k]) st_coherent_u(bm + w0 + idx[k], nw);
+            }
         }
+        if (!__syncthreads_or(n)) continue;  // s_lc is clear, nothing was counted
+        for (int i = lane; i < n; i += 64) atomicAdd(&s_lc[list[i] >> 11], 1);
         __syncthreads();
         if (threadIdx.x < NCLS) {
-            int k = s_lc[threadIdx.x];
-            s_lb[threadIdx.x] = k ? atomicAdd(&cnt_out[threadIdx.x], k) : 0;
+            const int k = s_lc[threadIdx.x];
+            s_lb[threadIdx.x] = k ? seg_off[threadIdx.x] + atomicAdd(&cnt_out[threadIdx.x], k) : 0;
             s_lc[threadIdx.x] = 0;
         }
         __syncthreads();
-        word = take;
-        while (word) {
-            int b = __ffs(word) - 1;
-            word &= word - 1;
-            long long slot = wi * 32 + b;
-            int c = cls[slot];
-            int p = atomicAdd(&s_lc[c], 1);
-            if (seg_ok(ctrl, (long long)seg_off[c] + s_lb[c] + p, seg_off[c], seg_off[c + 1]))
-                st_coherent(q_out + seg_off[c] + s_lb[c] + p, (int)slot);
+        for (int i = lane; i < n; i += 64) {
+            const int e = list[i], c = e >> 11;
+            const int at = s_lb[c] + atomicAdd(&s_lc[c], 1);
+            if (seg_ok(ctrl, at, seg_off[c], seg_off[c + 1])) st_coherent(q_out + at, (int)(w0 * 32) + (e & 2047));
         }
-        if (take | drop) st_coherent_u(bm + wi, word0 & ~(take | drop));
         __syncthreads();
     }
     if (T != NO_WINDOW) flush_deferred(my_dc, my_dm, &s_dc, &s_dm, defer_cnt, defer_min);
@@ -492,6 +596,33 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
 // schedule decision (all threads of a workgroup; the MLP is evaluated redundantly per
 // workgroup so every workgroup reaches the same decision without another barrier)
 // ------------------------------------------------------------------------------------
+// features() by one wavefront: lane c holds class c's count, the sums are butterflies and lane i
+// finishes feature i (one thread walking the classes took 0.9 us of every iteration).  Counts below
+// 2^24 add without rounding, so the features are the host's but for the last bit of larger sums.
+__device__ __forceinline__ void wave_features(const int *count, int it, int n, float *x) {
+    const int c = lane_id();
+    const float k = c >= 1 && c < NCLS ? (float)count[c] : 0.f;
+    const int g = c <= 2 ? 0 : c <= 4 ? 1 : c <= 6 ? 2 : c <= 8 ? 3 : c <= 12 ? 4 : 5;
+    float sum[8] = {k, c >= 1 && c < NCLS ? k * 0.75f * (float)(1u << c) : 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) sum[2 + i] = g == i ? k : 0.f;
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[i] += __shfl_xor(sum[i], o);
+    }
+    const float tot = sum[0];
+    float v = c == 8 ? (float)(it < 256 ? it : 256) / 64.f : 0.f;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+        if (c == 2 + i) v = tot > 0.f ? sum[2 + i] / tot : 0.f;
+    if (c == 0 || c == 1 || c == 9) {
+        const float y = c == 0 ? 1.f + tot : c == 1 ? 1.f + sum[1] : (float)(n > 1 ? n : 1);
+        v = log2f(y) / (c == 0 ? 24.f : 32.f);
+    }
+    if (c < NP_MLP_NIN) x[c] = v;
+}
+
 // The MLP's decision, or the fixed schedule (level, klo, khi) when its output is unusable.
 // Called with scalars, not the SchedDev: a struct passed by reference to a function that is not
 // inlined is first stored to scratch memory by every caller.
@@ -512,7 +643,7 @@ __device__ __noinline__ Cfg decide_mlp(const float *mlp, int n_feat, int flevel,
     const float4 w2 = *(const float4 *)(W2 + 4 * t);
     const float4 w3 = t < 40 ? *(const float4 *)(W3 + 4 * t) : make_float4(0.f, 0.f, 0.f, 0.f);
     const float b1j = b1[j], b2j = b2[j], b3j = t < 40 ? b3[j] : 0.f;
-    if (t == 0) features(cnt, it, n_feat, s_x);
+    if (t < 64) wave_features(cnt, it, n_feat, s_x);
     __syncthreads();
     float a = w1a * s_x[p] + (p + 8 < NP_MLP_NIN ? w1b * s_x[p + 8] : 0.f);
     a += __shfl_xor(a, 1);
@@ -606,10 +737,9 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
                 tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
             }
             __syncthreads();
-            if (threadIdx.x == 0) {
-                long long tot = 0;
-                for (int c = 1; c < NCLS; ++c) tot += tb.cnt[c];
-                s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
+            if (threadIdx.x < 64) {
+                const long long tot = frontier_size(tb.cnt);
+                if (threadIdx.x == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
             }
             __syncthreads();
             if (s_total > 0 || T == NO_WINDOW) break;
@@ -628,7 +758,7 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
             return;
         }
         Cfg cfg = decide(sp, tb.cnt, it);
-        if (threadIdx.x == 0) build_tables(tb, cfg);
+        if (threadIdx.x < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
@@ -669,8 +799,7 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
     const int it = ld_coherent(&ctrl->it_base) + it_off;
     if (threadIdx.x < NCLS) s_cnt[threadIdx.x] = ld_coherent(st.cnt + (it % 3) * NCLS + threadIdx.x);
     __syncthreads();
-    long long tot = 0;
-    for (int c = 1; c < NCLS; ++c) tot += s_cnt[c];
+    const long long tot = frontier_size(s_cnt);  // every wavefront for itself
     const int pass = ld_coherent(&ctrl->pass);  // the compaction of this slot
     if (tot == 0 && !sp.push) {
         const int T = ld_coherent(&ctrl->thresh);
@@ -738,10 +867,10 @@ __global__ __launch_bounds__(WG) void k_expand(DevState st, int it_off) {
     }
     if (PUSH && blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         Cfg cfg = make_cfg(ld_coherent(&ctrl->cfg_level), ld_coherent(&ctrl->cfg_klo),
                            ld_coherent(&ctrl->cfg_khi));
-        build_tables(tb, cfg);
+        build_tables(tb, cfg, TABLES_SINGLE, (long long)gridDim.x * WAVES);
     }
     __syncthreads();
     PushCtx pc;
@@ -1720,10 +1849,9 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
                 tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
             }
             __syncthreads();
-            if (threadIdx.x == 0) {
-                long long tot = 0;
-                for (int c = 1; c < NCLS; ++c) tot += tb.cnt[c];
-                s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
+            if (threadIdx.x < 64) {
+                const long long tot = frontier_size(tb.cnt);
+                if (threadIdx.x == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
             }
             __syncthreads();
             if (s_total > 0) break;
@@ -1746,7 +1874,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             return;
         }
         Cfg cfg = decide(sp, tb.cnt, it);
-        if (threadIdx.x == 0) build_tables(tb, pk_cfg(cfg, false));
+        if (threadIdx.x < 64) build_tables(tb, pk_cfg(cfg, false), TABLES_PACKED, (long long)nb * WAVES);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
@@ -1859,10 +1987,10 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         Cfg cfg = make_cfg(ld_coherent(&ctrl->cfg_level), ld_coherent(&ctrl->cfg_klo),
                            ld_coherent(&ctrl->cfg_khi));
-        build_tables(tb, pk_cfg(cfg, filt), filt);
+        build_tables(tb, pk_cfg(cfg, filt), filt ? TABLES_FILTERED : TABLES_PACKED, (long long)gridDim.x * WAVES);
     }
     if (filt && threadIdx.x < PACK_MAX) s_off[threadIdx.x] = ld_coherent(ctrl->foff + threadIdx.x);
     __syncthreads();
