@@ -339,10 +339,12 @@ static SchedDev make_schedd(np_ctx *c, const np_sched &s, int n_feat) {
 // / 1 M: 0.59 ms with 1, 0.64 with 4; grid 512^2: 1.20 and 1.32), a middling one two (grid 2048^2,
 // 17 M edges: 3.77 with 2, 3.94 with 4; learned on R-MAT s20, 17 M: 1.20 and 1.22), and only large
 // ones all that fit (R-MAT s22, 67 M: 5.6, 4.5, 4.2, 4.1 ms with 1 to 4).
-static int persistent_wgs(np_ctx *c, const np_sched &s, bool batch, bool unit, bool packed, long long edges) {
-    int occ = persistent_max_wgs_per_cu(batch, unit, s.frontier == NP_FRONTIER_PUSH, packed);
+static constexpr long long SMALL_EDGES = 4ll << 20, LARGE_EDGES = 32ll << 20;
+static int persistent_wgs(np_ctx *c, const np_sched &s, const SchedDev &sd, bool batch, bool unit, bool packed,
+                          long long edges) {
+    int occ = persistent_max_wgs_per_cu(batch, unit, sd.push != 0, packed, sd.solo != 0);
     if (occ < 1) occ = 1;
-    const int fit = packed ? occ : edges <= (4ll << 20) ? 1 : edges <= (32ll << 20) ? std::min(2, occ) : occ;
+    const int fit = packed || edges > LARGE_EDGES ? occ : edges > SMALL_EDGES ? std::min(2, occ) : 1;
     int per = s.wgs_per_cu > 0 ? std::min(s.wgs_per_cu, occ) : fit;
     return per * c->num_cus;
 }
@@ -431,9 +433,11 @@ static int run_drive(np_ctx *c, Space &s, const DevState &st, const np_sched &sc
     // the reference's other schedules are per-iteration launches
     if (sd.scheme != NP_SCHEME_CONSOLIDATE && drive == NP_DRIVE_PERSISTENT) drive = NP_DRIVE_HOSTLOOP;
     if (drive == NP_DRIVE_PERSISTENT) {
-        int wgs = persistent_wgs(c, sch, batch, unit, st.kshift >= 0, s.edges);
+        SchedDev psd = sd;
+        psd.solo = st.kshift < 0 && !sd.push && s.edges <= LARGE_EDGES;
+        int wgs = persistent_wgs(c, sch, psd, batch, unit, st.kshift >= 0, s.edges);
         HIPCHK(hipEventRecord(c->ev0, c->stream));
-        hipError_t e = launch_persistent(st, sd, batch, unit, wgs, c->stream);
+        hipError_t e = launch_persistent(st, psd, batch, unit, wgs, c->stream);
         if (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge) {
             // No cooperative queue for this process (another process on the device holds
             // the cooperative dispatch resource) or the grid no longer fits: nothing was
@@ -828,7 +832,7 @@ int np_destroy(np_ctx *c) {
 int np_device_info(np_ctx *c, int32_t *num_cus, int32_t *max_wgs_per_cu) {
     if (!c) { set_error("null context"); return NP_ERR_ARG; }
     if (num_cus) *num_cus = c->num_cus;
-    if (max_wgs_per_cu) *max_wgs_per_cu = persistent_max_wgs_per_cu(false, false, false, false);
+    if (max_wgs_per_cu) *max_wgs_per_cu = persistent_max_wgs_per_cu(false, false, false, false, false);
     return NP_OK;
 }
 
@@ -2240,7 +2244,7 @@ int np_autotune(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, const
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;  // the search is over the consolidation bins
-    int occ = persistent_max_wgs_per_cu(false, false, b0.frontier == NP_FRONTIER_PUSH, false);
+    int occ = persistent_max_wgs_per_cu(false, false, b0.frontier == NP_FRONTIER_PUSH, false, g->m <= LARGE_EDGES);
     std::vector<int> wgs_opts = {0};
     if (occ > 2) wgs_opts.push_back(2);
     if (occ > 4) wgs_opts.push_back(4);
@@ -2302,7 +2306,7 @@ int np_batch_autotune(np_ctx *c, np_batch *b, const np_sched *base, np_sched *be
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;
-    int occ = persistent_max_wgs_per_cu(true, b->unit != 0, false, !b->packs.empty());
+    int occ = persistent_max_wgs_per_cu(true, b->unit != 0, false, !b->packs.empty(), b->sp.edges <= LARGE_EDGES);
     std::vector<int> wgs_opts = {0};
     if (occ > 2) wgs_opts.push_back(2);
     if (occ > 4) wgs_opts.push_back(4);

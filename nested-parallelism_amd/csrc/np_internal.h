@@ -93,6 +93,7 @@ struct SchedDev {
     const float *mlp;       // NP_MLP_NPARAM device floats
     np_trace_rec *trace;
     int scheme;             // NP_SCHEME_* (0: the consolidation bins)
+    int solo;               // persistent drive: small frontiers run on one workgroup
 };
 
 // ---- kernels.hip: solve drivers ----------------------------------------------------
@@ -136,7 +137,7 @@ hipError_t launch_unpermute_parts(const int *dist, const int *lut, const ConcatO
 // with kshift >= 0 runs the source-packed kernels (here and in compact/expand).
 hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch, bool unit,
                              int wgs, hipStream_t s);
-int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed);
+int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo);
 
 // Host-loop / graph drive, one iteration = [compact] + decide + expand.
 hipError_t launch_compact(const DevState &st, int it_off, bool batch, int wgs, hipStream_t s);

@@ -697,9 +697,155 @@ __device__ __forceinline__ void record_trace(const SchedDev &sp, int it, const C
 }
 
 // ------------------------------------------------------------------------------------
+// small frontiers of the persistent drive
+// ------------------------------------------------------------------------------------
+// A frontier of a few hundred vertices costs a whole iteration's two grid barriers, a scan of the
+// bitmap and the work tables (14-18 us) for a few microseconds of work, and road-like graphs start
+// and end with dozens of them.  One workgroup runs such iterations alone, the frontier in LDS, while
+// the others wait at the next grid barrier: about 4 us each (one solve, grid 512^2 1.20 -> 1.03 ms,
+// 2048^2 3.88 -> 3.66; ER 65,536 / 1 M, with few small frontiers, 0.563 -> 0.552).  An improved vertex is appended once
+// (the returned bitmap word decides), so when the frontier outgrows the limits the bitmap holds
+// exactly the vertices pending, and the next compaction takes over.
+constexpr int SOLO_V = 512;        // vertices of a solo frontier
+constexpr int SOLO_E = 4096;       // edges of one
+constexpr int SOLO_ITERS = 256;    // iterations per visit (the other workgroups' wait is bounded)
+
+struct SoloBufs {
+    int list[2][SOLO_V];
+    int pre[SOLO_V + 1];  // exclusive prefix of the degrees
+    int start[SOLO_V];    // first edge - prefix
+    int base[SOLO_V];     // slot base of the vertex's instance
+    int du[SOLO_V];
+    int wsum[WAVES], live, next;
+};
+
+__device__ __forceinline__ bool solo_fits(const ItemTables &tb, int total) {
+    if (total > SOLO_V) return false;
+    const int c = threadIdx.x & 31;  // every half-wave for itself
+    int e = c >= 1 && tb.cnt[c] ? (c >= 13 ? SOLO_E + 1 : tb.cnt[c] << c) : 0;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) e += __shfl_xor(e, o);
+    return e <= SOLO_E;
+}
+
+// Iterations of the queued frontier (classes in tb) until it is empty or outgrows the limits, at
+// most `most`; returns how many.  Called by one whole workgroup.
+template <bool BATCH, bool UNIT>
+__device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTables &tb, const int *q, SoloBufs &sb,
+                                               int total, int most) {
+    const int t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+    unsigned *bm = st.bm[0];
+    // the queue's class segments -> list[0]
+    for (int i = t; i < total; i += WG) {
+        int c = 1, k = i;
+        while (k >= tb.cnt[c]) { k -= tb.cnt[c]; ++c; }
+        sb.list[0][i] = ld_coherent(q + tb.seg[c] + k);
+    }
+    int n = total, iters = 0;
+    long long sum = 0;
+    for (;;) {
+        __syncthreads();
+        if (t == 0) { sb.next = 0; sb.live = 0; }
+        const int *cur = sb.list[iters & 1];
+        int *nxt = sb.list[(iters & 1) ^ 1];
+        // vertices 2t, 2t + 1: flags of an appended vertex are cleared before it is expanded
+        int d[2] = {0, 0}, s[2] = {0, 0};
+        static_assert(SOLO_V == 2 * WG, "two vertices per thread");
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int i = 2 * t + k;
+            if (i >= n) continue;
+            const int slot = cur[i];
+            if (iters > 0) atomicAnd(&bm[slot >> 5], ~(1u << (slot & 31)));
+            int B, VB;
+            decode<BATCH>(st, slot, B, VB);
+            s[k] = st.row[VB + slot - B];
+            d[k] = st.row[VB + slot - B + 1] - s[k];
+            sb.base[i] = B;
+            sb.du[i] = ld_coherent(st.dist + slot);
+        }
+        __syncthreads();  // next and live are zero
+        const unsigned long long m0 = __ballot(d[0] > 0), m1 = __ballot(d[1] > 0);
+        const int incl = wave_incl_scan(d[0] + d[1]);
+        if (lane == 63) {
+            sb.wsum[wave] = incl;
+            atomicAdd(&sb.live, __popcll(m0) + __popcll(m1));
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // the cleared flags are in memory
+        __syncthreads();
+        int before = 0, edges = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            before += w < wave ? sb.wsum[w] : 0;
+            edges += sb.wsum[w];
+        }
+        const int x0 = before + incl - d[0] - d[1], x1 = x0 + d[0];
+        if (2 * t < n) { sb.pre[2 * t] = x0; sb.start[2 * t] = s[0] - x0; }
+        if (2 * t + 1 < n) { sb.pre[2 * t + 1] = x1; sb.start[2 * t + 1] = s[1] - x1; }
+        const int live = sb.live;
+        // empty, or a frontier that the grid should expand: from the second iteration on its flags
+        // were cleared just now, so they are set again for the next compaction
+        if (edges == 0 || iters >= most || (iters > 0 && edges > SOLO_E)) {
+            if (iters > 0 && edges > 0) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    if (2 * t + k < n && d[k] > 0) {
+                        const int slot = cur[2 * t + k];
+                        atomicOr(&bm[slot >> 5], 1u << (slot & 31));
+                    }
+            }
+            break;
+        }
+        __syncthreads();
+        sum += live;
+        ++iters;
+        for (int b0 = 0; b0 < edges; b0 += UNR * WG) {
+            int tv[UNR], alt[UNR], cv[UNR];
+#pragma unroll
+            for (int k = 0; k < UNR; ++k) {
+                const int i = b0 + k * WG + t;
+                int o = 0;  // owner: the last vertex whose prefix is <= i
+#pragma unroll
+                for (int step = SOLO_V / 2; step > 0; step >>= 1)
+                    if (o + step < n && sb.pre[o + step] <= i) o += step;
+                const bool ok = i < edges;
+                const int e = ok ? i + sb.start[o] : 0;
+                tv[k] = ok ? sb.base[o] + st.col[e] : -1;
+                alt[k] = ok ? sb.du[o] + (UNIT ? 1 : st.w[e]) : 0;
+            }
+#pragma unroll
+            for (int k = 0; k < UNR; ++k) cv[k] = tv[k] >= 0 ? ld_coherent(st.dist + tv[k]) : 0;
+            unsigned prev[UNR];
+#pragma unroll
+            for (int k = 0; k < UNR; ++k) {
+                prev[k] = ~0u;
+                if (alt[k] >= cv[k]) continue;
+                atomicMin(&st.dist[tv[k]], alt[k]);
+                prev[k] = atomicOr(&bm[tv[k] >> 5], 1u << (tv[k] & 31));
+            }
+#pragma unroll
+            for (int k = 0; k < UNR; ++k) {
+                if (tv[k] < 0 || (prev[k] >> (tv[k] & 31)) & 1u) continue;
+                const int at = atomicAdd(&sb.next, 1);
+                if (at < SOLO_V) nxt[at] = tv[k];
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // the distances are in memory
+        __syncthreads();
+        n = sb.next;
+        if (n > SOLO_V) break;  // the bitmap has them all
+        if (n == 0) break;
+    }
+    if (t == 0) st.ctrl->frontier_total += sum;
+    return iters;
+}
+
+// ------------------------------------------------------------------------------------
 // persistent drive
 // ------------------------------------------------------------------------------------
-template <bool BATCH, bool UNIT, bool PUSH>
+// SOLO: small frontiers run on one workgroup; a graph of many edges goes without (its solve is a few
+// large iterations, and the registers cost it a workgroup per CU: R-MAT s22 4.26 -> 4.31 ms).
+template <bool BATCH, bool UNIT, bool PUSH, bool SOLO>
 __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
     __shared__ ItemTables tb;
     __shared__ int s_total;
@@ -710,6 +856,7 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
     // priority window: every workgroup computes the same sequence of thresholds
     int T = (!PUSH && sp.delta > 0) ? sp.delta : NO_WINDOW;
     int pass = 0;
+    int extra = 0;  // iterations run by one workgroup alone, beyond one per trip
     for (int it = 0;; ++it) {
         int *cnt_cur = st.cnt + (it % 3) * NCLS;
         int *cnt_zero = st.cnt + ((it + 2) % 3) * NCLS;
@@ -749,15 +896,28 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
             T = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
         }
         const int total = s_total;
-        if (total == 0 || (sp.max_iters > 0 && it >= sp.max_iters)) {
+        const int done_iters = it + extra;
+        if (total == 0 || (sp.max_iters > 0 && done_iters >= sp.max_iters)) {
             if (blockIdx.x == 0 && threadIdx.x == 0) {
-                ctrl->iters = it;
+                ctrl->iters = done_iters;
                 ctrl->done = total == 0 ? 1 : 0;
                 if (total != 0) ctrl->error = NP_ERR_NOT_CONVERGED;
             }
             return;
         }
-        Cfg cfg = decide(sp, tb.cnt, it);
+        if (SOLO && T == NO_WINDOW && !sp.trace && solo_fits(tb, total)) {
+            __shared__ SoloBufs s_solo;
+            int most = SOLO_ITERS;
+            if (sp.max_iters > 0 && sp.max_iters - done_iters < most) most = sp.max_iters - done_iters;
+            if (blockIdx.x == 0) {
+                const int k = solo_iterations<BATCH, UNIT>(st, tb, q_cur, s_solo, total, most);
+                if (threadIdx.x == 0) st_coherent(&ctrl->solo, k);
+            }
+            if (!grid_sync(ctrl, nb, gen)) return;
+            extra += ld_coherent(&ctrl->solo) - 1;
+            continue;
+        }
+        Cfg cfg = decide(sp, tb.cnt, done_iters);
         if (threadIdx.x < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctrl->frontier_total += total;
@@ -2416,25 +2576,24 @@ hipError_t launch_copy_cls(const unsigned char *src, unsigned char *dst, long lo
     return hipGetLastError();
 }
 
-template <bool B, bool U, bool P>
-static const void *persistent_fn() { return (const void *)&k_persistent<B, U, P>; }
+template <bool B, bool U>
+static const void *persistent_fn(bool push, bool solo) {
+    if (push) return (const void *)&k_persistent<B, U, true, false>;
+    return solo ? (const void *)&k_persistent<B, U, false, true> : (const void *)&k_persistent<B, U, false, false>;
+}
 
-static const void *pick_persistent(bool batch, bool unit, bool push) {
-    if (batch) {
-        if (unit) return push ? persistent_fn<true, true, true>() : persistent_fn<true, true, false>();
-        return push ? persistent_fn<true, false, true>() : persistent_fn<true, false, false>();
-    }
-    if (unit) return push ? persistent_fn<false, true, true>() : persistent_fn<false, true, false>();
-    return push ? persistent_fn<false, false, true>() : persistent_fn<false, false, false>();
+static const void *pick_persistent(bool batch, bool unit, bool push, bool solo) {
+    if (batch) return unit ? persistent_fn<true, true>(push, solo) : persistent_fn<true, false>(push, solo);
+    return unit ? persistent_fn<false, true>(push, solo) : persistent_fn<false, false>(push, solo);
 }
 
 static const void *pick_packed(bool unit) {
     return unit ? (const void *)&k_pk_persistent<true> : (const void *)&k_pk_persistent<false>;
 }
 
-int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed) {
+int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo) {
     int nb = 0;
-    const void *fn = packed ? pick_packed(unit) : pick_persistent(batch, unit, push);
+    const void *fn = packed ? pick_packed(unit) : pick_persistent(batch, unit, push, solo);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, WG, 0) != hipSuccess) return 0;
     return nb;
 }
@@ -2444,7 +2603,7 @@ hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch,
     DevState a0 = st;
     SchedDev a1 = sp;
     void *args[] = {&a0, &a1};
-    const void *fn = st.kshift >= 0 ? pick_packed(unit) : pick_persistent(batch, unit, sp.push != 0);
+    const void *fn = st.kshift >= 0 ? pick_packed(unit) : pick_persistent(batch, unit, sp.push != 0, sp.solo != 0);
     return hipLaunchCooperativeKernel(fn, dim3(wgs), dim3(WG), args, 0, s);
 }
 
