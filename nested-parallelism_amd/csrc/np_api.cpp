@@ -56,6 +56,7 @@ static void dfree(T *&p) {
 }
 
 static constexpr int TRACE_CAP = 1 << 15;
+static constexpr int H_SMALL = 1024;  // words of the pinned readback
 
 }  // namespace np
 
@@ -151,7 +152,7 @@ struct np_ctx {
     // repeated calls allocate nothing once it is large enough) and a small pinned readback
     char *ws = nullptr;
     size_t ws_bytes = 0;
-    unsigned long long *h_small = nullptr;  // 4 words
+    unsigned long long *h_small = nullptr;  // H_SMALL words
     int *d_guard = nullptr;                 // 4 ints: CSR validation, distance-range check
     // Live objects made on this context.  np_destroy releases what they hold on the device
     // and detaches them: their handles stay valid for np_graph_free / np_batch_free, which
@@ -752,7 +753,7 @@ int np_create(int device, np_ctx **out) {
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
     if (e == hipSuccess) e = dalloc(&c->ctrl, 1);
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_ctrl, sizeof(Ctrl), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_small, 4 * sizeof(unsigned long long), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_small, H_SMALL * sizeof(unsigned long long), hipHostMallocDefault);
     if (e == hipSuccess) e = dalloc(&c->trace, TRACE_CAP);
     if (e == hipSuccess) e = dalloc(&c->model, NP_MLP_NPARAM);
     if (e == hipSuccess) e = dalloc(&c->d_work2, 4);
@@ -1326,7 +1327,8 @@ int np_color(np_ctx *c, np_graph *g, int32_t method, int32_t *color_out, np_stat
 
 // Row-bin storage (medium rows, huge rows, their chunks) for n rows holding m entries; the
 // three counts are adjacent, cleared by bins_clear.
-static void bins_carve(Carve &cv, RowBins &rb, int n, long long m) {
+// finish: huge rows are finished by their last chunk's wavefront.
+static void bins_carve(Carve &cv, RowBins &rb, int n, long long m, bool finish) {
     const size_t nh = (size_t)(m / PR_HUGE) + 1, nc = (size_t)pr_chunk_cap(m);
     rb.med = cv.take<int>((size_t)n);
     rb.huge = cv.take<int>(nh);
@@ -1334,6 +1336,8 @@ static void bins_carve(Carve &cv, RowBins &rb, int n, long long m) {
     rb.crow = cv.take<int>(nc);
     rb.ck = cv.take<int>(nc);
     rb.part = cv.take<double>(nc);
+    rb.hleft = finish ? cv.take<int>(nh) : nullptr;
+    rb.chuge = finish ? cv.take<int>(nc) : nullptr;
     rb.nmed = cv.take<int>(3);
     rb.nhuge = rb.nmed ? rb.nmed + 1 : nullptr;
     rb.nchunk = rb.nmed ? rb.nmed + 2 : nullptr;
@@ -1343,28 +1347,24 @@ static hipError_t bins_clear(const RowBins &rb, hipStream_t s) { return hipMemse
 // PAGERANK_GPU (apps/pagerank/src/gpu/pagerank_wrapper.cu:199-244, 565-661): damping 0.5, total
 // rank 1000, until no vertex changes by more than 1e-13 (pagerank_wrapper.cu:5-6, pagerank.h:15).
 struct PrBufs {
-    long long *irow;
-    int *src, *pcol;
+    int *irow, *src, *pcol;
     unsigned *tkey;
     RowBins rb;
-    double *rank, *nrank, *contrib, *dsum;
-    unsigned long long *dmax;
-    int *ctl;
+    double *rank, *contrib[2];
+    PrSums *ps;
     float *out;
     void *temp;
 };
 static void pr_carve(Carve &cv, PrBufs &pb, int n, long long m, size_t temp_bytes) {
-    pb.irow = cv.take<long long>((size_t)n + 1);
+    pb.irow = cv.take<int>((size_t)n + 1);
     pb.src = cv.take<int>((size_t)m);
     pb.pcol = cv.take<int>((size_t)m);
     pb.tkey = cv.take<unsigned>((size_t)m);
-    bins_carve(cv, pb.rb, n, m);
+    bins_carve(cv, pb.rb, n, m, true);
     pb.rank = cv.take<double>((size_t)n);
-    pb.nrank = cv.take<double>((size_t)n);
-    pb.contrib = cv.take<double>((size_t)n);
-    pb.dsum = cv.take<double>(2);
-    pb.dmax = cv.take<unsigned long long>(2);
-    pb.ctl = cv.take<int>(2);
+    pb.contrib[0] = cv.take<double>((size_t)n);
+    pb.contrib[1] = cv.take<double>((size_t)n);
+    pb.ps = cv.take<PrSums>(1);
     pb.out = cv.take<float>((size_t)n);
     pb.temp = cv.take<char>(temp_bytes);
 }
@@ -1382,10 +1382,10 @@ int np_pagerank(np_ctx *c, np_graph *g, int32_t max_iters, float *rank_out, np_s
     const long long m = g->m;
     int end_bit = 1;  // key bits covering vertex ids 0..n-1
     while (end_bit < 31 && (1ll << end_bit) < n) ++end_bit;
-    const unsigned *tkey_in = reinterpret_cast<const unsigned *>(g->col);
+    const unsigned *tkey_in = reinterpret_cast<const unsigned *>(g->scol);
     size_t temp_bytes = 0, scan_bytes = 0;
     HIPCHK(pr_sort(nullptr, &temp_bytes, tkey_in, nullptr, nullptr, nullptr, m, end_bit, c->stream));
-    HIPCHK(pr_sources(nullptr, &scan_bytes, g->row, n, m, nullptr, nullptr, c->stream));
+    HIPCHK(pr_sources(nullptr, &scan_bytes, g->srow, n, m, nullptr, nullptr, c->stream));
     temp_bytes = std::max(temp_bytes, scan_bytes);
     PrBufs pb{};
     Carve cv;
@@ -1395,45 +1395,44 @@ int np_pagerank(np_ctx *c, np_graph *g, int32_t max_iters, float *rank_out, np_s
     pr_carve(cv, pb, n, m, temp_bytes);
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     HIPCHK(bins_clear(pb.rb, c->stream));
+    HIPCHK(hipMemsetAsync(pb.ps, 0, sizeof(PrSums), c->stream));
     if (m > 0) {
         size_t sb = scan_bytes;
-        HIPCHK(pr_sources(pb.temp, &sb, g->row, n, m, pb.pcol, pb.src, c->stream));  // pcol: scratch until the sort
+        HIPCHK(pr_sources(pb.temp, &sb, g->srow, n, m, pb.pcol, pb.src, c->stream));  // pcol: scratch until the sort
         size_t tb = temp_bytes;
         HIPCHK(pr_sort(pb.temp, &tb, tkey_in, pb.tkey, pb.src, pb.pcol, m, end_bit, c->stream));
     }
     HIPCHK(launch_pr_offsets(pb.tkey, m, n, pb.irow, c->stream));
-    HIPCHK(launch_pr_bins(pb.irow, n, m, pb.rb, c->stream));
-    HIPCHK(launch_pr_init(pb.rank, n, total / n, c->stream));
-    HIPCHK(hipMemsetAsync(pb.ctl, 0, 2 * sizeof(int), c->stream));
+    HIPCHK(launch_row_bins(pb.irow, n, m, pb.rb, c->stream));
+    HIPCHK(launch_pr_init(g->srow, n, total / n, pb.rank, pb.contrib[0], pb.ps, c->stream));
     const double rw = (1.0 - damping) * total / n;
     const int cap = max_iters > 0 ? max_iters : 100000;
     // Iterations go out PR_BATCH at a time; the device ends the run (see launch_pr_iteration) and
     // the host reads the iteration count once per batch instead of the change once per iteration.
     constexpr int PR_BATCH = 8;
-    double *r[2] = {pb.rank, pb.nrank};
+    static_assert(sizeof(PrSums) <= H_SMALL * sizeof(unsigned long long), "the readback buffer holds the sums");
     int launched = 0, it = 0;
     for (;;) {
         if (launched >= cap) { set_error("PageRank did not converge in %d iterations", cap); return NP_ERR_NOT_CONVERGED; }
         const int k = std::min(PR_BATCH, cap - launched);
         for (int j = 0; j < k; ++j, ++launched)
-            HIPCHK(launch_pr_iteration(launched, pb.ctl, g->row, pb.irow, pb.pcol, pb.rb, r[launched & 1],
-                                       r[(launched + 1) & 1], pb.contrib, n, damping, rw, eps, pb.dsum, pb.dmax,
+            HIPCHK(launch_pr_iteration(launched, pb.ps, g->srow, pb.irow, pb.pcol, pb.rb, pb.rank,
+                                       pb.contrib[launched & 1], pb.contrib[(launched + 1) & 1], n, m, damping, rw, eps,
                                        c->num_cus, c->stream));
-        unsigned long long *h = c->h_small;
-        HIPCHK(hipMemcpyAsync(h, pb.ctl, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipMemcpyAsync(h + 1, pb.dmax, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(c->h_small, pb.ps, sizeof(PrSums), hipMemcpyDeviceToHost, c->stream));
         int rc = ctx_sync(c);
         if (rc) return rc;
-        int hc[2];
-        std::memcpy(hc, h, sizeof hc);
-        if (hc[0]) { it = hc[1]; break; }  // iteration hc[1] changed no vertex by more than EPSILON
-        if (launched >= cap) {             // the last allowed iteration ran: its own change decides
-            double dlast;
-            std::memcpy(&dlast, h + 1 + ((launched - 1) & 1), sizeof dlast);
-            if (!(dlast > eps)) { it = launched; break; }
+        const PrSums &h = *reinterpret_cast<const PrSums *>(c->h_small);
+        double dlast = 0.0;  // the largest change of the last iteration that was launched, if it ran
+        for (const PrSlot &sl : h.slot) {
+            double d;
+            std::memcpy(&d, &sl.dmax[(launched - 1) % 3], sizeof d);
+            dlast = std::max(dlast, d);
         }
+        it = h.iters;
+        if (it < launched || !(dlast > eps)) break;
     }
-    HIPCHK(launch_pr_to_float(r[it & 1], n, pb.out, c->stream));
+    HIPCHK(launch_pr_to_float(pb.rank, g->rl.active ? g->rl.old2new : nullptr, n, pb.out, c->stream));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     HIPCHK(hipMemcpyAsync(rank_out, pb.out, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
     int rc = ctx_sync(c);
@@ -1467,13 +1466,13 @@ int np_spmv(np_ctx *c, np_graph *g, const double *data, const double *x, double 
         d_data = cv.take<double>((size_t)m);
         d_x = cv.take<double>((size_t)n);
         d_y = cv.take<double>((size_t)n);
-        bins_carve(cv, rb, n, m);
+        bins_carve(cv, rb, n, m, false);
     }
     if (m > 0) HIPCHK(hipMemcpyAsync(d_data, data, sizeof(double) * (size_t)m, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(d_x, x, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(bins_clear(rb, c->stream));
     HIPCHK(hipEventRecord(c->ev0, c->stream));
-    HIPCHK(launch_spmv_bins(g->row, n, m, rb, c->stream));
+    HIPCHK(launch_row_bins(g->row, n, m, rb, c->stream));
     HIPCHK(launch_spmv(g->row, g->col, d_data, d_x, d_y, n, rb, c->num_cus, c->stream));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     HIPCHK(hipMemcpyAsync(y, d_y, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));

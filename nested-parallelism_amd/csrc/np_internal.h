@@ -225,8 +225,19 @@ constexpr int PR_HUGE = 2 * PR_CHUNK;
 struct RowBins {
     int *med, *nmed;              // medium rows [n]; count
     int *huge, *hc0, *nhuge;      // huge rows and their first chunk [m / PR_HUGE + 1]; count
+    int *hleft;                   // chunks of each huge row still to finish (null: not kept)
     int *crow, *ck, *nchunk;      // chunk -> row, chunk index [pr_chunk_cap(m)]; count
+    int *chuge;                   // chunk -> index into huge (null: not kept)
     double *part;                 // per-chunk partial sums [pr_chunk_cap(m)]
+};
+// Rotating sums of the iterations (see k_pr_pull), a cache line per slot: workgroup b adds to slot
+// b % PR_SLOTS, because atomics on one line take turns (about 30 ns each: 2,048 workgroups on one
+// pair of sums took longer than their rows).  Zero before launch_pr_init.
+constexpr int PR_SLOTS = 64;
+struct alignas(64) PrSlot { double dsum[3]; unsigned long long dmax[3]; };
+struct PrSums {
+    PrSlot slot[PR_SLOTS];
+    int iters;
 };
 long long pr_chunk_cap(long long m);
 // In-edge CSR: src[e] = source of edge e; sort (col, src) pairs; offsets from the sorted targets.
@@ -236,20 +247,19 @@ hipError_t pr_sources(void *temp, size_t *temp_bytes, const int *row, int n, lon
                       hipStream_t s);
 hipError_t pr_sort(void *temp, size_t *temp_bytes, const unsigned *key_in, unsigned *key_out, const int *val_in,
                    int *val_out, long long m, int end_bit, hipStream_t s);
-hipError_t launch_pr_offsets(const unsigned *key, long long m, int n, long long *irow, hipStream_t s);
-hipError_t launch_pr_init(double *rank, int n, double r0, hipStream_t s);
-// Bins over irow (counts *nmed, *nhuge, *nchunk zero on entry).
-hipError_t launch_pr_bins(const long long *irow, int n, long long m, const RowBins &rb, hipStream_t s);
-// Iteration i, rank -> nrank, decided on the device: ctl[0] (done) is set when iteration i - 1
-// changed no vertex by more than eps, and then nothing runs; else ctl[1] = i + 1.  Sums of
-// iteration i in dsum2[i & 1], dmax2[i & 1] (cleared by the iteration itself); contrib: scratch.
-hipError_t launch_pr_iteration(int i, int *ctl, const int *row, const long long *irow, const int *pcol,
-                               const RowBins &rb, const double *rank, double *nrank, double *contrib, int n,
-                               double damping, double rw, double eps, double *dsum2, unsigned long long *dmax2,
-                               int num_cus, hipStream_t s);
-hipError_t launch_pr_to_float(const double *rank, int n, float *out, hipStream_t s);
-// SpMV y = A x over the graph's CSR, with row bins built by launch_spmv_bins.
-hipError_t launch_spmv_bins(const int *row, int n, long long m, const RowBins &rb, hipStream_t s);
+hipError_t launch_pr_offsets(const unsigned *key, long long m, int n, int *irow, hipStream_t s);
+// Bins over n rows with offsets off (counts *nmed, *nhuge, *nchunk zero on entry).
+hipError_t launch_row_bins(const int *off, int n, long long m, const RowBins &rb, hipStream_t s);
+// rank = r0, contributions and dangling sum of iteration 0.
+hipError_t launch_pr_init(const int *row, int n, double r0, double *rank, double *contrib, PrSums *ps, hipStream_t s);
+// Iteration i, rank in place, contrib -> ncontrib.  Nothing runs once an iteration changed no vertex
+// by more than eps; ps->iters = iterations that ran, the greatest dmax[i % 3] of the slots = the largest change of
+// the i-th.
+hipError_t launch_pr_iteration(int i, PrSums *ps, const int *row, const int *irow, const int *pcol, const RowBins &rb,
+                               double *rank, const double *contrib, double *ncontrib, int n, long long m, double damping,
+                               double rw, double eps, int num_cus, hipStream_t s);
+hipError_t launch_pr_to_float(const double *rank, const int *old2new, int n, float *out, hipStream_t s);
+// SpMV y = A x over the graph's CSR, with row bins built by launch_row_bins.
 hipError_t launch_spmv(const int *row, const int *col, const double *data, const double *x, double *y, int n,
                        const RowBins &rb, int num_cus, hipStream_t s);
 

@@ -76,3 +76,33 @@ def test_gpu_pagerank_cli_matches_oracle(tmp_path, orc):
     got = np.array([float(l.split(":")[1]) for l in lines])
     ref, _ = orc.pagerank(g["row"], g["col"])
     assert np.allclose(got, ref, rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("relabel", [0, 1])
+@pytest.mark.parametrize("n, sizes", [(1, []), (7, [31, 32, 33]), (64, [0, 1, 8, 31]), (3000, [31, 32, 33, 2047, 2048, 2049]),
+                                      (5000, [4095, 4096, 4097, 6143, 6144, 6145, 140000])])
+def test_pagerank_row_forms_in_both_numberings(npa, ctx, orc, relabel, n, sizes):
+    """In-degrees at the edges of the pull's row forms (up to more chunks than a wavefront has
+    lanes), in the original numbering and renumbered by in-degree, dangling vertices and vertices
+    without in-edges among them; repeated calls on one workspace agree with the oracle alike."""
+    rng = np.random.default_rng(500 + n)
+    if sizes:
+        row, col = hub_csr(rng, n, 2 * n, sizes, inward=True)
+    else:
+        row, col = np.array([0, 1], np.int32), np.zeros(1, np.int32)
+    ctx.set_option(npa.CTX_RELABEL, relabel)
+    try:
+        G = npa.Graph.from_csr(ctx, row, col, np.ones(len(col), np.int32))
+    finally:
+        ctx.set_option(npa.CTX_RELABEL, 2)
+    ref, it = orc.pagerank(row, col)
+    first = None
+    for _ in range(3):
+        got, st = ctx.pagerank(G)
+        assert np.allclose(got, ref, rtol=1e-5, atol=1e-9)
+        assert abs(float(got.astype(np.float64).sum()) - 1000.0) < 1e-2
+        assert first is None or abs(st.iterations - first) <= 3
+        first = st.iterations
+    early, st = ctx.pagerank(G, max_iters=first + 3)
+    assert np.allclose(early, ref, rtol=1e-5, atol=1e-9)
+    G.free()
