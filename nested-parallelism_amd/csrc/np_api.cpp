@@ -350,6 +350,13 @@ static int persistent_wgs(np_ctx *c, const np_sched &s, const SchedDev &sd, bool
     return per * c->num_cus;
 }
 
+// Queued (vertex, source) pairs of a packed solve.
+static long long pairs_total(const Ctrl &h) {
+    long long t = 0;
+    for (const BarLeaf &l : h.leaf) t += l.pairs;
+    return t;
+}
+
 static int read_ctrl(np_ctx *c) {
     HIPCHK(hipMemcpyAsync(c->h_ctrl, c->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, c->stream));
     return ctx_sync(c);
@@ -490,7 +497,7 @@ static int run_drive(np_ctx *c, Space &s, const DevState &st, const np_sched &sc
         stats->status = rc;
         stats->kernel_ms = ms;
         stats->drive = drive;
-        stats->pairs_total = st.kshift >= 0 ? h.pairs_total : h.frontier_total;
+        stats->pairs_total = st.kshift >= 0 ? pairs_total(h) : h.frontier_total;
         stats->frontier_total = h.frontier_total;
         stats->edges_total = h.edges_total;
         stats->items_total = h.items_total;
@@ -1750,7 +1757,7 @@ static int run_parts_concurrent(np_ctx *c, std::vector<PartJob> &jobs, const np_
         const Ctrl &h = *j.s->h_pctrl;
         acc->iterations += h.iters;
         acc->frontier_total += h.frontier_total;
-        acc->pairs_total += j.st.kshift >= 0 ? h.pairs_total : h.frontier_total;
+        acc->pairs_total += j.st.kshift >= 0 ? pairs_total(h) : h.frontier_total;
         acc->edges_total += h.edges_total;
         acc->items_total += h.items_total;
         if (h.error && rc == NP_OK) rc = h.error;

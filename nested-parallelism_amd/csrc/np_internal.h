@@ -8,15 +8,22 @@
 
 namespace np {
 
+// Atomics on one cache line take turns (about 30 ns each, from whichever workgroup), so what every
+// workgroup of a launch adds to is split over BAR_LEAVES lines, workgroup b on line b % BAR_LEAVES.
 constexpr int BAR_LEAVES = 32;
-struct alignas(128) BarLeaf { unsigned long long n; unsigned long long pad[15]; };
+struct alignas(128) BarLeaf {
+    unsigned long long n;     // grid barrier: cumulative arrivals
+    long long pairs;          // source-packed: queued (vertex, source) pairs, summed over iterations
+    int dcnt[3];              // per compaction pass (rotating): flagged vertices kept back
+    int dmin[3];              // ... and the least distance among them
+};
 
 // Largest number of sources packed into one distance row.
 constexpr int PACK_MAX = 32;
 
 // Device-side control block of one solve.
 struct Ctrl {
-    BarLeaf leaf[BAR_LEAVES]; // grid barrier: cumulative arrivals per leaf (own cache lines)
+    BarLeaf leaf[BAR_LEAVES]; // per-line sums of the workgroups
     unsigned long long bar;   // grid barrier: cumulative leaf completions
     int error;                // NP_ERR_* raised by a kernel (0 = none)
     int done;                 // frontier emptied
@@ -27,9 +34,6 @@ struct Ctrl {
     int thresh;               // priority window: vertices with dist < thresh are expanded
     int pass;                 // compaction passes so far (host-loop / graph drives)
     int skip;                 // host-loop / graph drives: this slot only raised the window
-    int defer_cnt[3];         // per compaction pass (rotating): flagged vertices kept back
-    int defer_min[3];         // ... and the least distance among them
-    long long pairs_total;    // source-packed: sum over iterations of queued (vertex, source) pairs
     long long edges_total;    // source-packed: sum over iterations of the queued vertices' out-degrees
     long long items_total;    // source-packed: ... of out-degree x queued sources ((edge, source) items)
     int solo;                 // persistent drive: iterations of the last solo visit

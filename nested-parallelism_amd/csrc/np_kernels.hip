@@ -472,16 +472,15 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
 // ------------------------------------------------------------------------------------
 // With a priority window (T < INT_MAX) only flagged vertices with dist < T are queued and
 // unflagged; the others keep their flag, and the pass adds how many were kept and the
-// least distance among them to defer_cnt / defer_min.  T = INT_MAX queues every flag.
+// least distance among them to the pass's deferral sums (BarLeaf).  T = INT_MAX queues every flag.
 constexpr int NO_WINDOW = 0x7FFFFFFF;
 
-// Source-packed frontiers without a window are sparse: a thread scans one bitmap word and visits
-// its set bits, so empty words cost one load (single-source ones: see compaction_impl).  With a priority window
-// a source-packed frontier is dense (deferred vertices stay flagged and are re-read every pass):
-// there each thread owns CPT vertices of a tile of WG * CPT consecutive ones, so the lanes of a
-// wave read the class bytes, masks and distance rows of consecutive vertices and the 32 lanes of
-// one bitmap word rewrite it with one store.  Both count queue slots per class in LDS and
-// reserve them once per class per tile.
+// Without a window frontiers are sparse and whole bitmap words are skipped (compaction_impl, and its
+// form in pk_compaction).  With a priority window a source-packed frontier is dense (deferred
+// vertices stay flagged and are re-read every pass): there each thread owns CPT vertices of a tile
+// of WG * CPT consecutive ones, so the lanes of a wave read the class bytes, masks and distance rows
+// of consecutive vertices and the 32 lanes of one bitmap word rewrite it with one store.  Both count
+// queue slots per class in LDS and reserve them once per class per tile.
 constexpr int CPT = 4;
 
 // One bitmap word per 32 lanes: the first lane of each half-wave stores the kept bits when the
@@ -502,9 +501,9 @@ __device__ __forceinline__ void reserve_classes(int *s_lc, int *s_lb, int *cnt_o
     __syncthreads();
 }
 
-// Deferred-pair statistics of the workgroup -> defer_cnt / defer_min.
-__device__ __forceinline__ void flush_deferred(int my_dc, int my_dm, int *s_dc, int *s_dm, int *defer_cnt,
-                                               int *defer_min) {
+// Deferred-pair statistics of the workgroup -> its line's sums of the pass.  One line for all took
+// turns for longer than the pass: 2,048 workgroups, 0.12 ms (32 sources of a 2048^2 grid).
+__device__ __forceinline__ void flush_deferred(Ctrl *ctrl, int slot, int my_dc, int my_dm, int *s_dc, int *s_dm) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         my_dc += __shfl_xor(my_dc, o);
@@ -513,7 +512,32 @@ __device__ __forceinline__ void flush_deferred(int my_dc, int my_dm, int *s_dc, 
     }
     if (lane_id() == 0 && my_dc) { atomicAdd(s_dc, my_dc); atomicMin(s_dm, my_dm); }
     __syncthreads();
-    if (threadIdx.x == 0 && *s_dc) { atomicAdd(defer_cnt, *s_dc); atomicMin(defer_min, *s_dm); }
+    if (threadIdx.x == 0 && *s_dc) {
+        BarLeaf &l = ctrl->leaf[blockIdx.x % BAR_LEAVES];
+        atomicAdd(&l.dcnt[slot], *s_dc);
+        atomicMin(&l.dmin[slot], *s_dm);
+    }
+}
+// The sums of a pass over all lines (a whole wavefront; the result in every lane).
+__device__ __forceinline__ void deferred_sums(const Ctrl *ctrl, int slot, int *cnt, int *least) {
+    const BarLeaf &l = ctrl->leaf[lane_id() % BAR_LEAVES];
+    int c = lane_id() < BAR_LEAVES ? ld_coherent(&l.dcnt[slot]) : 0;
+    int m = ld_coherent(&l.dmin[slot]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        c += __shfl_xor(c, o);
+        const int x = __shfl_xor(m, o);
+        m = x < m ? x : m;
+    }
+    *cnt = c;
+    *least = m;
+}
+// Clears a pass's sums (threads 0 .. BAR_LEAVES of one workgroup).
+__device__ __forceinline__ void deferred_clear(Ctrl *ctrl, int slot) {
+    if (threadIdx.x < BAR_LEAVES) {
+        st_coherent(&ctrl->leaf[threadIdx.x].dcnt[slot], 0);
+        st_coherent(&ctrl->leaf[threadIdx.x].dmin[slot], NO_WINDOW);
+    }
 }
 
 // A wave loads up to 64 words at once and takes the nonzero ones two at a time, a lane per vertex,
@@ -521,9 +545,17 @@ __device__ __forceinline__ void flush_deferred(int my_dc, int my_dm, int *s_dc, 
 // per word, walking its bits, left all but n / 8192 workgroups idle and waited for every class: one
 // solve on the persistent drive, ER 65,536 / 1 M 0.94 -> 0.82 ms, grid 2048^2 5.12 -> 4.13.
 constexpr int COMPACT_UNR = 4;
+// Words a wavefront takes at once, 8 to 64: about 512 workgroups get a tile, because every tile
+// reserves its classes' queue slots on the same cache lines, where atomics take turns (a tile for
+// each of 2,048 workgroups made the heaviest compactions of 4.2 M vertices 75 -> 95 us).
+__device__ __forceinline__ int compact_words(long long nwords) {
+    const long long wgs = gridDim.x < 512 ? gridDim.x : 512;
+    const long long share = (nwords + wgs * WAVES - 1) / (wgs * WAVES);
+    return share < 8 ? 8 : share < 64 ? (int)share : 64;
+}
 __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const unsigned char *cls, const int *seg_off,
                                                 long long nwords, int *cnt_out, int *q_out, const int *dist,
-                                                int T, int *defer_cnt, int *defer_min) {
+                                                int T, int slot) {
     __shared__ unsigned short s_list[WAVES][64 * 32];
     __shared__ int s_lc[NCLS], s_lb[NCLS];
     __shared__ int s_dc, s_dm;
@@ -532,9 +564,7 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
     int my_dc = 0, my_dm = NO_WINDOW;
     const int lane = lane_id(), half = lane & 31;
     unsigned short *list = s_list[threadIdx.x >> 6];
-    // words per wave: all workgroups take part, but a tile is worth its counter reservations
-    const long long share = (nwords + (long long)gridDim.x * WAVES - 1) / ((long long)gridDim.x * WAVES);
-    const int wt = share < 8 ? 8 : share < 64 ? (int)share : 64;
+    const int wt = compact_words(nwords);
     const long long tile = (long long)WAVES * wt;
     for (long long wb = (long long)blockIdx.x * tile; wb < nwords; wb += (long long)gridDim.x * tile) {
         if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;
@@ -589,7 +619,7 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
         }
         __syncthreads();
     }
-    if (T != NO_WINDOW) flush_deferred(my_dc, my_dm, &s_dc, &s_dm, defer_cnt, defer_min);
+    if (T != NO_WINDOW) flush_deferred(ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
 }
 
 // ------------------------------------------------------------------------------------
@@ -679,7 +709,9 @@ __device__ __forceinline__ Cfg decide(const SchedDev &sp, const int *cnt, int it
 
 __device__ __noinline__ void record_trace_rec(np_trace_rec *r, int it, int level, int klo, int khi, const int *cnt,
                                               long long t0, Ctrl *ctrl) {
-    r->pairs = __hip_atomic_load(&ctrl->pairs_total, __ATOMIC_RELAXED, NP_AGENT);
+    long long pairs = 0;
+    for (int l = 0; l < BAR_LEAVES; ++l) pairs += __hip_atomic_load(&ctrl->leaf[l].pairs, __ATOMIC_RELAXED, NP_AGENT);
+    r->pairs = pairs;
     r->edges = __hip_atomic_load(&ctrl->edges_total, __ATOMIC_RELAXED, NP_AGENT);
     r->iteration = it;
     r->level = level;
@@ -868,14 +900,11 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
         }
         if (blockIdx.x == 0 && threadIdx.x < NCLS) st_coherent(cnt_zero + threadIdx.x, 0);
         for (;;) {
-            int *dc = ctrl->defer_cnt + pass % 3, *dm = ctrl->defer_min + pass % 3;
+            const int slot = pass % 3;
             if (!PUSH) {
                 // the statistics slot of the next pass was last read before the previous barrier
-                if (blockIdx.x == 0 && threadIdx.x == 0) {
-                    st_coherent(ctrl->defer_cnt + (pass + 1) % 3, 0);
-                    st_coherent(ctrl->defer_min + (pass + 1) % 3, NO_WINDOW);
-                }
-                compaction_impl(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, cnt_cur, q_cur, st.dist, T, dc, dm);
+                if (blockIdx.x == 0 && T != NO_WINDOW) deferred_clear(ctrl, (pass + 1) % 3);
+                compaction_impl(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, cnt_cur, q_cur, st.dist, T, slot);
                 if (!grid_sync(ctrl, nb, gen)) return;
                 pass++;
             }
@@ -891,8 +920,9 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
             __syncthreads();
             if (s_total > 0 || T == NO_WINDOW) break;
             // nothing below the window: raise it to the least pending distance + delta
-            if (ld_coherent(dc) == 0) break;
-            const int mn = ld_coherent(dm);
+            int kept, mn;
+            deferred_sums(ctrl, slot, &kept, &mn);
+            if (kept == 0) break;
             T = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
         }
         const int total = s_total;
@@ -944,12 +974,9 @@ __global__ __launch_bounds__(WG) void k_compact(DevState st, int it_off) {
     const int pass = ld_coherent(&ctrl->pass);
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctrl->defer_cnt[(pass + 1) % 3] = 0;
-        ctrl->defer_min[(pass + 1) % 3] = NO_WINDOW;
-    }
+    if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
     compaction_impl(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, st.cnt + (it % 3) * NCLS, st.queue[it & 1],
-                    st.dist, T, ctrl->defer_cnt + pass % 3, ctrl->defer_min + pass % 3);
+                    st.dist, T, pass % 3);
 }
 
 __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_off) {
@@ -963,12 +990,13 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
     const int pass = ld_coherent(&ctrl->pass);  // the compaction of this slot
     if (tot == 0 && !sp.push) {
         const int T = ld_coherent(&ctrl->thresh);
-        if ((T != NO_WINDOW || st.hold_cls) && ld_coherent(ctrl->defer_cnt + pass % 3) > 0) {
+        int kept, mn;
+        deferred_sums(ctrl, pass % 3, &kept, &mn);
+        if ((T != NO_WINDOW || st.hold_cls) && kept > 0) {
             // nothing queued but pairs kept back: raise the window (held vertices need only the
             // next pass); this slot's expansion is skipped
             if (threadIdx.x == 0) {
                 if (T != NO_WINDOW) {
-                    const int mn = ld_coherent(ctrl->defer_min + pass % 3);
                     ctrl->thresh = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
                 }
                 ctrl->skip = 1;
@@ -1849,61 +1877,118 @@ __device__ __forceinline__ unsigned pk_take(const DevState &st, long long v, uns
 // Vertices with pending sources -> class-segmented queue with their source masks.  With a
 // priority window (T < NO_WINDOW) only the (vertex, source) pairs with dist < T are queued;
 // the others stay pending in mflag[v] (and v in the bitmap), and the pass adds their count and
-// least distance to defer_cnt / defer_min.
+// least distance to the pass's deferral sums.
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
-                                              int T, int *defer_cnt, int *defer_min) {
+                                              int T, int slot) {
     __shared__ int s_lc[NCLS], s_lb[NCLS];
-    __shared__ int s_dc, s_dm;
+    __shared__ int s_dc, s_dm, s_pairs;
     unsigned *bm = st.bm[0];
-    if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; }
+    if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; s_pairs = 0; }
     if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;
     __syncthreads();
     int pairs = 0, my_dc = 0, my_dm = NO_WINDOW;
     const long long nv = st.nwords * 32;
     // Without a window every pending vertex is taken whole and nothing stays flagged but the hubs
-    // held for one pass (hold_cls): the frontier is as sparse as a single source's, so a thread
-    // scans one bitmap word as compaction_impl does.
-    for (long long wb = (long long)blockIdx.x * WG; T == NO_WINDOW && wb < st.nwords;
-         wb += (long long)gridDim.x * WG) {
-        const long long wi = wb + threadIdx.x;
-        const unsigned word = wi < st.nwords ? ld_coherent_u(bm + wi) : 0u;
-        unsigned queued = 0, held = 0, hw = 0;
-        bool hw_read = false;
-        for (unsigned w = word; w; w &= w - 1) {
-            const int b = __ffs(w) - 1;
-            const int c = st.cls[wi * 32 + b];
-            if (!c) continue;  // no out-edges: dropped (its mflag stays set, so it is not flagged again)
-            if (st.hold_cls && c >= st.hold_cls) {
-                if (!hw_read) { hw = ld_coherent_u(st.bm[1] + wi); hw_read = true; }
-                if (!((hw >> b) & 1u) && pk_reached(st, wi * 32 + b) < st.hold_min) {
-                    held |= 1u << b;  // more sources are on their way: wait one pass, keep the flag
-                    my_dc++;
-                    continue;
+    // held for one pass (hold_cls): the words are scanned as compaction_impl does (a thread per word
+    // took 0.24 ms where this takes 0.1, R-MAT s24, 16 sources, 8 M vertices queued).
+    if (T == NO_WINDOW) {
+        __shared__ unsigned short s_list[WAVES][64 * 32];
+        __shared__ unsigned s_held[WG];  // per word of the wave: held vertices, and whether it has hubs
+        __shared__ int s_heavy[WG];
+        const int lane = lane_id(), half = lane & 31;
+        unsigned short *list = s_list[threadIdx.x >> 6];
+        const int wt = compact_words(st.nwords);
+        const long long tile = (long long)WAVES * wt;
+        for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
+            const long long w0 = wb + (threadIdx.x >> 6) * wt;
+            const unsigned word = lane < wt && w0 + lane < st.nwords ? ld_coherent_u(bm + w0 + lane) : 0u;
+            unsigned long long nz = __ballot(word != 0);
+            int n = 0;
+            while (nz) {
+                int idx[COMPACT_UNR], c[COMPACT_UNR];
+                unsigned x[COMPACT_UNR];
+#pragma unroll
+                for (int k = 0; k < COMPACT_UNR; ++k) {
+                    const int ia = __ffsll((long long)nz) - 1;
+                    nz &= nz - 1;
+                    const int ib = __ffsll((long long)nz) - 1;
+                    nz &= nz - 1;
+                    idx[k] = lane < 32 ? ia : ib;  // -1: none left
+                    x[k] = __shfl(word, idx[k] < 0 ? 0 : idx[k]);
+                    if (idx[k] < 0) x[k] = 0u;
+                    // no out-edges (class 0): dropped (mflag stays set, so it is not flagged again)
+                    c[k] = (x[k] >> half) & 1u ? (int)st.cls[(w0 + idx[k]) * 32 + half] : 0;
+                }
+#pragma unroll
+                for (int k = 0; k < COMPACT_UNR; ++k) {
+                    const unsigned long long m = __ballot(c[k] != 0);
+                    if (c[k]) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
+                    n += __popcll(m);
                 }
             }
-            queued |= 1u << b;
-            atomicAdd(&s_lc[c], 1);
-        }
-        reserve_classes(s_lc, s_lb, cnt_out);
-        for (unsigned w = queued; w; w &= w - 1) {
-            const long long v = wi * 32 + (__ffs(w) - 1);
-            const int c = st.cls[v];
-            const long long qi = st.seg_off[c] + s_lb[c] + atomicAdd(&s_lc[c], 1);
-            const unsigned t = ld_coherent_u(st.mflag + v);
-            st_coherent_u(st.mflag + v, 0u);
-            if (seg_ok(st.ctrl, qi, st.seg_off[c], st.seg_off[c + 1])) {
-                st_coherent(q_out + qi, (int)v);
-                st_coherent_u(qm_out + qi, t);
+            unsigned stay = 0;  // flags of this lane's word that stay
+            if (st.hold_cls) {
+                // hubs that more sources are on their way to wait one pass and keep their flag; a held
+                // vertex stays flagged, so the held bits are always a subset of the flags: they become
+                // exactly this pass's held vertices (the ones held before are queued).  Renumbered hubs
+                // share a wavefront's words, so their rows are read COMPACT_UNR x 64 at a time.
+                s_held[threadIdx.x] = 0u;
+                s_heavy[threadIdx.x] = 0;
+                unsigned *held_w = s_held + (threadIdx.x & ~63);
+                int *heavy_w = s_heavy + (threadIdx.x & ~63);
+                __builtin_amdgcn_wave_barrier();
+                int left = 0;
+                for (int base = 0; base < n; base += 64 * COMPACT_UNR) {
+                    int e[COMPACT_UNR], reached[COMPACT_UNR];
+                    unsigned hw[COMPACT_UNR];
+#pragma unroll
+                    for (int k = 0; k < COMPACT_UNR; ++k) {
+                        const int i = base + 64 * k + lane;
+                        e[k] = i < n ? (int)list[i] : 0;
+                        const bool heavy = (e[k] >> 11) >= st.hold_cls;
+                        hw[k] = heavy ? ld_coherent_u(st.bm[1] + w0 + ((e[k] & 2047) >> 5)) : 0u;
+                        reached[k] = heavy ? pk_reached(st, w0 * 32 + (e[k] & 2047)) : st.hold_min;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int k = 0; k < COMPACT_UNR; ++k) {
+                        const int wi = (e[k] & 2047) >> 5, bit = e[k] & 31;
+                        const bool heavy = (e[k] >> 11) >= st.hold_cls;
+                        const bool held = heavy && !((hw[k] >> bit) & 1u) && reached[k] < st.hold_min;
+                        if (heavy) heavy_w[wi] = 1;
+                        if (held) atomicOr(&held_w[wi], 1u << bit);
+                        my_dc += held;
+                        const bool take = e[k] != 0 && !held;
+                        const unsigned long long m = __ballot(take);
+                        if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
+                        left += __popcll(m);
+                    }
+                }
+                n = left;
+                __builtin_amdgcn_wave_barrier();
+                stay = s_held[threadIdx.x];
+                if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
             }
-            pairs += __popc(t);
+            if (word != stay) st_coherent_u(bm + w0 + lane, stay);
+            if (!__syncthreads_or(n)) continue;  // s_lc is clear, nothing was counted
+            for (int i = lane; i < n; i += 64) atomicAdd(&s_lc[list[i] >> 11], 1);
+            reserve_classes(s_lc, s_lb, cnt_out);
+            for (int i = lane; i < n; i += 64) {
+                const int e = list[i], c = e >> 11;
+                const long long v = w0 * 32 + (e & 2047);
+                const unsigned t = ld_coherent_u(st.mflag + v);
+                st_coherent_u(st.mflag + v, 0u);
+                const long long qi = st.seg_off[c] + s_lb[c] + atomicAdd(&s_lc[c], 1);
+                if (seg_ok(st.ctrl, qi, st.seg_off[c], st.seg_off[c + 1])) {
+                    st_coherent(q_out + qi, (int)v);
+                    st_coherent_u(qm_out + qi, t);
+                }
+                pairs += __popc(t);
+            }
+            __syncthreads();
+            if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;  // the last loop counted in s_lc
+            __syncthreads();
         }
-        if (word) st_coherent_u(bm + wi, held);
-        // a held vertex stays flagged, so the held bits are always a subset of the flags: they
-        // become exactly this pass's held vertices (the ones held before are queued now)
-        if (hw_read && hw != held) st_coherent_u(st.bm[1] + wi, held);
-        __syncthreads();
-        if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;  // the second loop counted in s_lc
-        __syncthreads();
     }
     for (long long vb = (long long)blockIdx.x * (WG * CPT); T != NO_WINDOW && vb < nv;
          vb += (long long)gridDim.x * (WG * CPT)) {
@@ -1953,9 +2038,11 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o);
-    if (lane_id() == 0 && pairs) atomicAdd((unsigned long long *)&st.ctrl->pairs_total, (unsigned long long)pairs);
-
-    if (T != NO_WINDOW || st.hold_cls) flush_deferred(my_dc, my_dm, &s_dc, &s_dm, defer_cnt, defer_min);
+    if (lane_id() == 0 && pairs) atomicAdd(&s_pairs, pairs);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_pairs)
+        atomicAdd((unsigned long long *)&st.ctrl->leaf[blockIdx.x % BAR_LEAVES].pairs, (unsigned long long)s_pairs);
+    if (T != NO_WINDOW || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
 }
 
 // Lane-bin bound of a packed expansion (see PACK_LANE_CLS); the other bins keep theirs.  A filtered
@@ -1995,13 +2082,10 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
         }
         if (blockIdx.x == 0 && threadIdx.x < NCLS) st_coherent(cnt_zero + threadIdx.x, 0);
         for (;;) {
-            int *dc = ctrl->defer_cnt + pass % 3, *dm = ctrl->defer_min + pass % 3;
+            const int slot = pass % 3;
             // the statistics slot of the next pass was last read before the previous barrier
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                st_coherent(ctrl->defer_cnt + (pass + 1) % 3, 0);
-                st_coherent(ctrl->defer_min + (pass + 1) % 3, NO_WINDOW);
-            }
-            pk_compaction(st, cnt_cur, q_cur, qm_cur, T, dc, dm);
+            if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
+            pk_compaction(st, cnt_cur, q_cur, qm_cur, T, slot);
             if (!grid_sync(ctrl, nb, gen)) return;
             pass++;
             if (threadIdx.x < NCLS) {
@@ -2018,9 +2102,10 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             // nothing queued: done unless pairs were kept back (below the window, or held
             // vertices, which the next pass takes); a window rises to the least pending
             // distance + delta
-            if (ld_coherent(dc) == 0) break;
+            int kept, mn;
+            deferred_sums(ctrl, slot, &kept, &mn);
+            if (kept == 0) break;
             if (T != NO_WINDOW) {
-                const int mn = ld_coherent(dm);
                 T = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
             }
         }
@@ -2052,12 +2137,8 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     const int pass = ld_coherent(&ctrl->pass);
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctrl->defer_cnt[(pass + 1) % 3] = 0;
-        ctrl->defer_min[(pass + 1) % 3] = NO_WINDOW;
-    }
-    pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T,
-                  ctrl->defer_cnt + pass % 3, ctrl->defer_min + pass % 3);
+    if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
+    pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, pass % 3);
 }
 
 // Every vertex's bound, once: between the compaction and the decision that records the offsets (no
@@ -2165,8 +2246,8 @@ __global__ void k_pk_init_sources(DevState st, const int *srcs, int nsrc, int T0
     if (blockIdx.x != 0) return;
     if (threadIdx.x == 0) {
         st.ctrl->thresh = T0;
-        for (int k = 0; k < 3; ++k) st.ctrl->defer_min[k] = NO_WINDOW;
     }
+    for (int k = 0; k < 3; ++k) deferred_clear(st.ctrl, k);
     __syncthreads();
     for (int i = threadIdx.x; i < nsrc; i += blockDim.x) {
         const int v = srcs[i];
@@ -2315,8 +2396,8 @@ __global__ void k_init_sources(DevState st, const int *srcs, int nsrc, int T0) {
     if (blockIdx.x != 0) return;
     if (threadIdx.x == 0) {
         st.ctrl->thresh = T0;
-        for (int k = 0; k < 3; ++k) st.ctrl->defer_min[k] = NO_WINDOW;
     }
+    for (int k = 0; k < 3; ++k) deferred_clear(st.ctrl, k);
     for (int i = threadIdx.x; i < nsrc; i += blockDim.x) {
         int slot = srcs[i];
         st.dist[slot] = 0;

@@ -85,3 +85,29 @@ def test_bound_filter_is_exact(npa, ctx, orc, k, kind):
     b.free()
     G.free()
     g0.free()
+
+
+@pytest.mark.parametrize("unit", [False, True])
+@pytest.mark.parametrize("n, hold", [(40, 6), (2100, 6), (9000, 7)])
+def test_hold_with_hubs_side_by_side(npa, ctx, orc, n, hold, unit):
+    """Every vertex is heavy enough to be held, in every word of a wavefront's share (more than one
+    look at the rows per wavefront), with duplicate sources and vertices reached by few."""
+    rng = np.random.default_rng(n + hold)
+    deg = rng.integers(33, 140, n)
+    row = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = rng.integers(0, n, row[-1]).astype(np.int32)
+    w = rng.integers(1, 60, row[-1]).astype(np.int32)
+    srcs = [int(s) for s in rng.integers(0, n, 19)] + [3, 3, 3]
+    ctx.set_option(npa.CTX_RELABEL, 1)
+    try:
+        G = npa.Graph.from_csr(ctx, row, col, w)
+    finally:
+        ctx.set_option(npa.CTX_RELABEL, 2)
+    b = npa.Batch(ctx, [G] * len(srcs), srcs, unit=unit)
+    for drive in (0, 1, 2):
+        b.solve(npa.Sched(level=2, log2_t_lo=4, log2_t_hi=6, drive=drive, pack_hold=hold))
+        for i, s in enumerate(srcs):
+            ref = orc.bfs_levels(row, col, s) if unit else orc.dijkstra(row, col, w, s)[0]
+            assert np.array_equal(b.get(i), ref), (drive, i)
+    b.free()
+    G.free()
