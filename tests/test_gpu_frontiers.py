@@ -120,3 +120,15 @@ def test_concatenated_small_frontiers(npa, ctx, orc):
         b.free()
     for g in graphs:
         g.free()
+
+
+@pytest.mark.parametrize("deg", [32767, 32768, 32769, 65537, 100000])
+def test_rows_longer_than_a_workgroup_chunk(npa, ctx, orc, deg):
+    """Block level: rows just below, at and above the chunk, and of several chunks, reached first,
+    later and again; both frontier kinds and every drive."""
+    rng = np.random.default_rng(deg)
+    n = 4000
+    src = np.concatenate([np.zeros(deg, np.int64), np.full(deg - 1, 7), rng.integers(0, n, 3 * n)])
+    dst = rng.integers(0, n, len(src))
+    row, col, w = _csr(src, dst, rng.integers(1, 200, len(src)), n)
+    _check(npa, ctx, orc, row, col, w, 5, [npa.Sched(level=1, drive=dr, frontier=fr) for dr in (0, 1, 2) for fr in (0, 1)])
