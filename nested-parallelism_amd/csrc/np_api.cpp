@@ -1084,7 +1084,7 @@ int np_reached_work(np_ctx *c, np_graph *g, const int32_t *d_dist, int32_t inf, 
 // entries, then the backward sweep replays them from the deepest level up.
 struct BcBufs {
     int *lvl = nullptr, *ent_v = nullptr, *owner = nullptr, *srcs = nullptr, *err = nullptr;
-    int *ectl = nullptr, *lv = nullptr, *h_lv = nullptr;
+    int2 *lv = nullptr, *h_lv = nullptr;
     unsigned *ent_m = nullptr, *nmask = nullptr;
     double *sig = nullptr, *del = nullptr, *acc = nullptr;
     long long *cst = nullptr, *h_total = nullptr;
@@ -1092,7 +1092,7 @@ struct BcBufs {
     float *out = nullptr;
     ~BcBufs() {
         dfree(lvl); dfree(ent_v); dfree(owner); dfree(srcs); dfree(err); dfree(ent_m); dfree(nmask);
-        dfree(sig); dfree(del); dfree(acc); dfree(cst); dfree(ctot); dfree(out); dfree(ectl); dfree(lv);
+        dfree(sig); dfree(del); dfree(acc); dfree(cst); dfree(ctot); dfree(out); dfree(lv);
         if (h_total) (void)hipHostFree(h_total);
         if (h_lv) (void)hipHostFree(h_lv);
     }
@@ -1121,7 +1121,7 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     while ((1 << ks) < P) ++ks;
     const long long cap_e = (long long)n * P;  // entries of one batch: at most one per (vertex, source)
     if (cap_e > 0x7FFFFFFFll) { set_error("n x batch sources exceeds 2^31 entries"); return NP_ERR_CAPACITY; }
-    const long long cap_owner = g->m / 2 + (long long)n + 1;  // chunks of one level
+    const long long cap_owner = g->m / 8 + (long long)n + 1;  // chunks of one level
     if (cap_owner > 0x7FFFFFFFll) { set_error("too many chunks for one level"); return NP_ERR_CAPACITY; }
     BcBufs bb;
     const size_t slots = (size_t)n << ks;
@@ -1145,14 +1145,13 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     // have 2, 4, 8, ... levels (deep graphs), at most BC_RUN; levels past the last are empty and
     // cost a few small launches.
     constexpr int BC_RUN = 64;
-    HIPCHK(dalloc(&bb.ectl, 2));  // first entry of the current level, its entry count
-    HIPCHK(dalloc(&bb.lv, 2 * ((size_t)n + BC_RUN + 1)));
-    HIPCHK(hipHostMalloc((void **)&bb.h_lv, 2 * BC_RUN * sizeof(int)));
+    HIPCHK(hipHostMalloc((void **)&bb.h_lv, BC_RUN * sizeof(int2)));
     int run = 8;
     // chunk counters, one per forward level (ctot[d]) and per backward level (ctot[NB + li]),
     // zeroed once per source batch
-    const size_t NB = (size_t)n + BC_RUN + 1;
+    const size_t NB = (size_t)n + BC_RUN + 2;
     HIPCHK(dalloc(&bb.ctot, 2 * NB));
+    HIPCHK(dalloc(&bb.lv, NB));  // first entry and entry count of every forward level
     HIPCHK(hipMemsetAsync(bb.acc, 0, sizeof(double) * (size_t)n, c->stream));
     BcDev b{g->row, g->col, n, ks, bb.lvl, bb.sig, bb.del, bb.nmask};
     HIPCHK(hipEventRecord(c->ev0, c->stream));
@@ -1164,49 +1163,41 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
         HIPCHK(launch_bc_sources(b, bb.srcs, np_, c->stream));
         levels.clear();
         long long E = 0;
-        HIPCHK(hipMemsetAsync(bb.ectl, 0, 2 * sizeof(int), c->stream));
+        HIPCHK(hipMemsetAsync(bb.lv, 0, NB * sizeof(int2), c->stream));
         HIPCHK(hipMemsetAsync(bb.ctot, 0, 2 * NB * sizeof(unsigned long long), c->stream));
         for (int d0 = 0, last = -1, k = run, grow = 2; last < 0;
              d0 += k, k = grow, grow = std::min(BC_RUN, 2 * grow)) {
             if (d0 > n) { set_error("more than n BFS levels"); return NP_ERR_NOT_CONVERGED; }
             for (int d = d0; d < d0 + k; ++d) {
                 // entry count and chunk total stay on the device: compaction (reserving each
-                // entry's chunks), owners, expansion, then the level's record
-                HIPCHK(launch_bc_compact(b, bb.ent_v, bb.ent_m, bb.ectl, bb.cst, bb.ectl + 1, bb.ctot + d, c->stream));
-                HIPCHK(launch_bc_owner(b, bb.ent_v, bb.ent_m, bb.ectl, bb.cst, n, bb.ectl + 1, bb.owner, cap_owner,
-                                       bb.err, c->stream));
-                HIPCHK(launch_bc_expand(b, true, bb.ent_v, bb.ent_m, bb.ectl, bb.cst, bb.owner, bb.ctot + d, cap_owner,
-                                        d, c->num_cus, c->stream));
-                HIPCHK(launch_bc_advance(bb.ectl, bb.ectl + 1, bb.lv, d, c->stream));
+                // entry's chunks and naming their owner), then the expansion
+                HIPCHK(launch_bc_compact(b, bb.ent_v, bb.ent_m, bb.lv, d, bb.cst, bb.ctot + d, bb.owner, cap_owner, bb.err,
+                                         c->stream));
+                HIPCHK(launch_bc_expand(b, true, bb.ent_v, bb.ent_m, bb.lv, bb.cst, bb.owner, bb.ctot + d, cap_owner, d,
+                                        c->num_cus, c->stream));
             }
-            HIPCHK(hipMemcpyAsync(bb.h_lv, bb.lv + 2 * (size_t)d0, 2 * (size_t)k * sizeof(int), hipMemcpyDeviceToHost,
-                                  c->stream));
+            HIPCHK(hipMemcpyAsync(bb.h_lv, bb.lv + d0, (size_t)k * sizeof(int2), hipMemcpyDeviceToHost, c->stream));
             int rc = ctx_sync(c);
             if (rc) return rc;
             for (int j = 0; j < k; ++j) {
-                const int ne = bb.h_lv[2 * j + 1];
+                const int ne = bb.h_lv[j].y;
                 if (ne <= 0) { last = d0 + j; break; }
-                levels.push_back({(long long)bb.h_lv[2 * j], ne});
+                levels.push_back({(long long)bb.h_lv[j].x, ne});
                 E += ne;
             }
         }
         run = std::min<int>(BC_RUN, (int)levels.size() + 1);
         // the deepest level has no successors (dependency 0): its slots only take their factor
-        // 1 / sigma (k_bc_accum adds zeros to bc); level 0 holds the sources
-        if (levels.size() >= 2) {
-            const long long E0 = levels.back().first;
-            HIPCHK(launch_bc_accum(b, bb.ent_v + E0, bb.ent_m + E0, levels.back().second, bb.acc, c->stream));
-        }
-        for (int li = (int)levels.size() - 2; li >= 1; --li) {
-            const long long E0 = levels[(size_t)li].first;
-            const int ne = levels[(size_t)li].second;
-            unsigned long long *ct = bb.ctot + NB + li;
-            HIPCHK(launch_bc_chunks(b, bb.ent_v + E0, bb.ent_m + E0, ne, bb.cst, ct, c->stream));
-            HIPCHK(launch_bc_owner(b, bb.ent_v + E0, bb.ent_m + E0, nullptr, bb.cst, ne, nullptr, bb.owner, cap_owner,
-                                   bb.err, c->stream));
-            HIPCHK(launch_bc_expand(b, false, bb.ent_v + E0, bb.ent_m + E0, nullptr, bb.cst, bb.owner, ct, cap_owner,
-                                    li, c->num_cus, c->stream));
-            HIPCHK(launch_bc_accum(b, bb.ent_v + E0, bb.ent_m + E0, ne, bb.acc, c->stream));
+        // 1 / sigma (k_bc_finish adds zeros to bc); level 0 holds the sources
+        for (int li = (int)levels.size() - 1; li >= 1; --li) {
+            const long long E0 = levels[(size_t)li].first, E1 = levels[(size_t)li - 1].first;
+            const int ne = levels[(size_t)li].second, nn = li > 1 ? levels[(size_t)li - 1].second : 0;
+            unsigned long long *ct = bb.ctot + NB + li - 1;
+            HIPCHK(launch_bc_finish(b, bb.ent_v + E0, bb.ent_m + E0, ne, bb.acc, bb.ent_v + E1, bb.ent_m + E1, nn, bb.cst, ct,
+                                    bb.owner, cap_owner, bb.err, c->stream));
+            if (li > 1)
+                HIPCHK(launch_bc_expand(b, false, bb.ent_v + E1, bb.ent_m + E1, nullptr, bb.cst, bb.owner, ct, cap_owner,
+                                        li - 1, c->num_cus, c->stream));
         }
         st.iterations += (int)levels.size();
         st.frontier_total += E;

@@ -72,3 +72,25 @@ def test_bc_rejects_bad_sources(npa, ctx):
     with pytest.raises(npa.NpError):
         ctx.bc(G, [-1])
     G.free()
+
+
+@pytest.mark.parametrize("nsrc", [1, 2, 17, 32, 33])
+def test_bc_rows_at_chunk_edges(npa, ctx, orc, nsrc):
+    """Rows of out-degree 0, 1 and one below, at and one above each power of two up to 256 (a
+    chunk holds 256 items or 64 edges, whichever split is in use), plus rows of several hundred
+    edges; the targets lie two levels deep and share successors, so sums cross chunks."""
+    degs = sorted({d for k in range(9) for d in (2 ** k - 1, 2 ** k, 2 ** k + 1)} | {512, 700})
+    n = 1200
+    rng = np.random.default_rng(57 + nsrc)
+    deg = np.ones(n, np.int64)
+    hubs = rng.permutation(n)[:2 * len(degs)]
+    deg[hubs] = degs + degs
+    row = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = rng.integers(0, n, row[-1]).astype(np.int32)
+    G = _graph(npa, ctx, row, col)
+    srcs = [int(s) for s in rng.permutation(n)[:nsrc]]
+    srcs[0] = int(hubs[-1])
+    bc, _ = ctx.bc(G, srcs)
+    ref = orc.bc(row, col, srcs)
+    assert np.allclose(bc, ref, rtol=RTOL, atol=ATOL), float(np.max(np.abs(bc - ref)))
+    G.free()
