@@ -1083,17 +1083,17 @@ int np_reached_work(np_ctx *c, np_graph *g, const int32_t *d_dist, int32_t inf, 
 // up to 32; per batch a level-synchronous forward BFS with path counts records every level's
 // entries, then the backward sweep replays them from the deepest level up.
 struct BcBufs {
-    int *lvl = nullptr, *ent_v = nullptr, *owner = nullptr, *srcs = nullptr, *err = nullptr;
-    int2 *lv = nullptr, *h_lv = nullptr;
-    unsigned *ent_m = nullptr, *nmask = nullptr;
+    int *ent_v = nullptr, *srcs = nullptr, *err = nullptr, *h_err = nullptr;
+    uint2 *st = nullptr;
+    int4 *rec = nullptr;
+    BcLevel *lv = nullptr, *h_lv = nullptr;
+    unsigned *ent_m = nullptr;
     double *sig = nullptr, *del = nullptr, *acc = nullptr;
-    long long *cst = nullptr, *h_total = nullptr;
-    unsigned long long *ctot = nullptr;
     float *out = nullptr;
     ~BcBufs() {
-        dfree(lvl); dfree(ent_v); dfree(owner); dfree(srcs); dfree(err); dfree(ent_m); dfree(nmask);
-        dfree(sig); dfree(del); dfree(acc); dfree(cst); dfree(ctot); dfree(out); dfree(lv);
-        if (h_total) (void)hipHostFree(h_total);
+        dfree(ent_v); dfree(srcs); dfree(err); dfree(st); dfree(rec); dfree(lv); dfree(ent_m);
+        dfree(sig); dfree(del); dfree(acc); dfree(out);
+        if (h_err) (void)hipHostFree(h_err);
         if (h_lv) (void)hipHostFree(h_lv);
     }
 };
@@ -1121,39 +1121,35 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     while ((1 << ks) < P) ++ks;
     const long long cap_e = (long long)n * P;  // entries of one batch: at most one per (vertex, source)
     if (cap_e > 0x7FFFFFFFll) { set_error("n x batch sources exceeds 2^31 entries"); return NP_ERR_CAPACITY; }
-    const long long cap_owner = g->m / 8 + (long long)n + 1;  // chunks of one level
-    if (cap_owner > 0x7FFFFFFFll) { set_error("too many chunks for one level"); return NP_ERR_CAPACITY; }
+    const long long cap = g->m / 64 + (long long)n + 1;  // chunks of one level
     BcBufs bb;
     const size_t slots = (size_t)n << ks;
-    HIPCHK(dalloc(&bb.lvl, slots));
+    HIPCHK(dalloc(&bb.st, (size_t)n));
     HIPCHK(dalloc(&bb.sig, slots));
     HIPCHK(dalloc(&bb.del, slots));
-    HIPCHK(dalloc(&bb.nmask, (size_t)n));
     HIPCHK(dalloc(&bb.ent_v, (size_t)cap_e));
     HIPCHK(dalloc(&bb.ent_m, (size_t)cap_e));
-    HIPCHK(dalloc(&bb.cst, (size_t)n + 1));
-    HIPCHK(dalloc(&bb.owner, (size_t)cap_owner));
+    HIPCHK(dalloc(&bb.rec, (size_t)cap));
     HIPCHK(dalloc(&bb.err, 1));
     HIPCHK(hipMemsetAsync(bb.err, 0, sizeof(int), c->stream));
     HIPCHK(dalloc(&bb.srcs, 32));
     HIPCHK(dalloc(&bb.acc, (size_t)n));
     HIPCHK(dalloc(&bb.out, (size_t)n));
-    HIPCHK(hipHostMalloc((void **)&bb.h_total, 2 * sizeof(long long)));
+    HIPCHK(hipHostMalloc((void **)&bb.h_err, sizeof(int)));
     // Forward levels go out several at a time with the entry counts kept on the device; the host
     // reads each run's (first entry, count) pairs once.  The first run is as long as the previous
     // source batch's depth + 1 (depths barely vary on one graph), at most BC_RUN; runs after it
     // have 2, 4, 8, ... levels (deep graphs), at most BC_RUN; levels past the last are empty and
     // cost a few small launches.
     constexpr int BC_RUN = 64;
-    HIPCHK(hipHostMalloc((void **)&bb.h_lv, BC_RUN * sizeof(int2)));
+    HIPCHK(hipHostMalloc((void **)&bb.h_lv, BC_RUN * sizeof(BcLevel)));
     int run = 8;
-    // chunk counters, one per forward level (ctot[d]) and per backward level (ctot[NB + li]),
-    // zeroed once per source batch
+    // one record per forward level (lv[d]) and per backward level (lv[NB + d]), zeroed once per
+    // source batch
     const size_t NB = (size_t)n + BC_RUN + 2;
-    HIPCHK(dalloc(&bb.ctot, 2 * NB));
-    HIPCHK(dalloc(&bb.lv, NB));  // first entry and entry count of every forward level
+    HIPCHK(dalloc(&bb.lv, 2 * NB));
     HIPCHK(hipMemsetAsync(bb.acc, 0, sizeof(double) * (size_t)n, c->stream));
-    BcDev b{g->row, g->col, n, ks, bb.lvl, bb.sig, bb.del, bb.nmask};
+    BcDev b{g->row, g->col, n, ks, bb.st, bb.sig, bb.del};
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     std::vector<std::pair<long long, int>> levels;
     for (size_t b0 = 0; b0 < S.size(); b0 += (size_t)P) {
@@ -1163,41 +1159,35 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
         HIPCHK(launch_bc_sources(b, bb.srcs, np_, c->stream));
         levels.clear();
         long long E = 0;
-        HIPCHK(hipMemsetAsync(bb.lv, 0, NB * sizeof(int2), c->stream));
-        HIPCHK(hipMemsetAsync(bb.ctot, 0, 2 * NB * sizeof(unsigned long long), c->stream));
+        HIPCHK(hipMemsetAsync(bb.lv, 0, 2 * NB * sizeof(BcLevel), c->stream));
         for (int d0 = 0, last = -1, k = run, grow = 2; last < 0;
              d0 += k, k = grow, grow = std::min(BC_RUN, 2 * grow)) {
             if (d0 > n) { set_error("more than n BFS levels"); return NP_ERR_NOT_CONVERGED; }
             for (int d = d0; d < d0 + k; ++d) {
-                // entry count and chunk total stay on the device: compaction (reserving each
-                // entry's chunks and naming their owner), then the expansion
-                HIPCHK(launch_bc_compact(b, bb.ent_v, bb.ent_m, bb.lv, d, bb.cst, bb.ctot + d, bb.owner, cap_owner, bb.err,
-                                         c->stream));
-                HIPCHK(launch_bc_expand(b, true, bb.ent_v, bb.ent_m, bb.lv, bb.cst, bb.owner, bb.ctot + d, cap_owner, d,
-                                        c->num_cus, c->stream));
+                // entry and chunk counts stay on the device
+                HIPCHK(launch_bc_compact(b, bb.ent_v, bb.ent_m, bb.lv + d, bb.rec, cap, bb.err, c->stream));
+                HIPCHK(launch_bc_expand(b, true, bb.lv + d, bb.rec, cap, nullptr, c->num_cus, c->stream));
             }
-            HIPCHK(hipMemcpyAsync(bb.h_lv, bb.lv + d0, (size_t)k * sizeof(int2), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipMemcpyAsync(bb.h_lv, bb.lv + d0, (size_t)k * sizeof(BcLevel), hipMemcpyDeviceToHost, c->stream));
             int rc = ctx_sync(c);
             if (rc) return rc;
             for (int j = 0; j < k; ++j) {
-                const int ne = bb.h_lv[j].y;
-                if (ne <= 0) { last = d0 + j; break; }
-                levels.push_back({(long long)bb.h_lv[j].x, ne});
+                const int ne = (int)(unsigned)bb.h_lv[j].ctl;
+                if (ne == 0) { last = d0 + j; break; }
+                levels.push_back({bb.h_lv[j].first, ne});
                 E += ne;
             }
         }
         run = std::min<int>(BC_RUN, (int)levels.size() + 1);
         // the deepest level has no successors (dependency 0): its slots only take their factor
-        // 1 / sigma (k_bc_finish adds zeros to bc); level 0 holds the sources
+        // 1 / sigma; level 0 holds the sources
         for (int li = (int)levels.size() - 1; li >= 1; --li) {
             const long long E0 = levels[(size_t)li].first, E1 = levels[(size_t)li - 1].first;
             const int ne = levels[(size_t)li].second, nn = li > 1 ? levels[(size_t)li - 1].second : 0;
-            unsigned long long *ct = bb.ctot + NB + li - 1;
-            HIPCHK(launch_bc_finish(b, bb.ent_v + E0, bb.ent_m + E0, ne, bb.acc, bb.ent_v + E1, bb.ent_m + E1, nn, bb.cst, ct,
-                                    bb.owner, cap_owner, bb.err, c->stream));
-            if (li > 1)
-                HIPCHK(launch_bc_expand(b, false, bb.ent_v + E1, bb.ent_m + E1, nullptr, bb.cst, bb.owner, ct, cap_owner,
-                                        li - 1, c->num_cus, c->stream));
+            BcLevel *lv = bb.lv + NB + li - 1;
+            HIPCHK(launch_bc_finish(b, bb.ent_v + E0, bb.ent_m + E0, ne, li + 1 == (int)levels.size(), bb.acc,
+                                    bb.ent_v + E1, bb.ent_m + E1, nn, lv, bb.rec, cap, bb.err, c->stream));
+            if (li > 1) HIPCHK(launch_bc_expand(b, false, lv, bb.rec, cap, bb.acc, c->num_cus, c->stream));
         }
         st.iterations += (int)levels.size();
         st.frontier_total += E;
@@ -1205,12 +1195,10 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     HIPCHK(launch_bc_to_float(bb.acc, n, bb.out, c->stream));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     HIPCHK(hipMemcpyAsync(bc_out, bb.out, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(bb.h_total, bb.err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(bb.h_err, bb.err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     int rc = ctx_sync(c);
     if (rc) return rc;
-    int err = 0;
-    std::memcpy(&err, bb.h_total, sizeof(int));
-    if (err) { set_error("a level exceeded its chunk capacity"); return NP_ERR_CAPACITY; }
+    if (*bb.h_err) { set_error("a level exceeded its chunk capacity"); return NP_ERR_CAPACITY; }
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     st.kernel_ms = ms;

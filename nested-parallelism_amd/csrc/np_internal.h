@@ -168,32 +168,33 @@ hipError_t launch_adam(float *p, const float *grad, float *m, float *v, int n, f
                        float b1, float b2, float eps, int step, hipStream_t s);
 
 // ---- bc.hip: betweenness centrality, up to 32 sources per batch -----------------------
-constexpr int BC_UNSEEN = 0x7FFFFFFF;
 struct BcDev {
     const int *row, *col;  // CSR (original ids)
     int n, ks;             // slots (v << ks) + j for batch source j < 2^ks
-    int *lvl;              // BFS level per slot, BC_UNSEEN when not reached
+    uint2 *st;             // [n] bits per source: .x reached on a level up to the one in hand, .y reached
+                           //     by the expansion in flight
     double *sig, *del;     // shortest-path counts and dependencies per slot
-    unsigned *nmask;       // [n] sources that first reached v in the last expansion
+};
+struct BcLevel {
+    unsigned long long ctl;  // entries (low half) and chunks (high half); zero before the level
+    long long first;         // first entry in ent_v/ent_m; zero for level 0
 };
 hipError_t launch_bc_reset(const BcDev &b, hipStream_t s);
 hipError_t launch_bc_sources(const BcDev &b, const int *srcs, int nsrc, hipStream_t s);
-// lv[d] = {first entry, entry count} of forward level d: .x of level 0 and every .y zero before.
-// Flagged vertices -> the entries of level d, at ent_v/ent_m + lv[d].x, counted in lv[d].y; the
-// first chunk of each at cst[0 .. count) (chunks reserved on *ctot, zero before the level) and the
-// owner of every chunk; a chunk past cap sets *err (nothing is written past cap).
-hipError_t launch_bc_compact(const BcDev &b, int *ent_v, unsigned *ent_m, int2 *lv, int d, long long *cst,
-                             unsigned long long *ctot, int *owner, long long cap, int *err, hipStream_t s);
-// Expansion of the chunks of level d's entries, at ent_v + lv[d].x (lv null: ent_v); chunk total
-// *ctot, read on the device, at most cap.  Forward, it sets lv[d + 1].x.
-hipError_t launch_bc_expand(const BcDev &b, bool fwd, const int *ent_v, const unsigned *ent_m, int2 *lv,
-                            const long long *cst, const int *owner, const unsigned long long *ctot, long long cap,
-                            int d, int num_cus, hipStream_t s);
-// Backward: the finished level's ne entries into bc and their slots' factors; chunk ranges and
-// owners of the next level's nn entries (*ctot zero before).
-hipError_t launch_bc_finish(const BcDev &b, const int *ent_v, const unsigned *ent_m, int ne, double *bc,
-                            const int *nxt_v, const unsigned *nxt_m, int nn, long long *cst, unsigned long long *ctot,
-                            int *owner, long long cap, int *err, hipStream_t s);
+// Vertices reached by the last expansion -> the entries of lv's level at ent_v/ent_m + lv->first and
+// their chunks' records {v, mask, first edge, edges left in the row}; a chunk past cap sets *err
+// (nothing is written past cap).
+hipError_t launch_bc_compact(const BcDev &b, int *ent_v, unsigned *ent_m, BcLevel *lv, int4 *rec, long long cap,
+                             int *err, hipStream_t s);
+// Expansion of lv's chunks (their count is read on the device).  Forward, it sets lv[1].first.
+hipError_t launch_bc_expand(const BcDev &b, bool fwd, BcLevel *lv, const int4 *rec, long long cap, double *bc,
+                            int num_cus, hipStream_t s);
+// Backward: the finished level's ne entries out of seen, and into bc and their slots' factors where
+// the sweep has not done that (`all`: the deepest level, which no sweep has passed); the chunks of
+// the next level's nn entries, counted in lv->ctl.
+hipError_t launch_bc_finish(const BcDev &b, const int *ent_v, const unsigned *ent_m, int ne, bool all, double *bc,
+                            const int *nxt_v, const unsigned *nxt_m, int nn, BcLevel *lv, int4 *rec, long long cap,
+                            int *err, hipStream_t s);
 hipError_t launch_bc_to_float(const double *bc, int n, float *out, hipStream_t s);
 
 // ---- color.hip: graph coloring (longest decreasing-id path labels) -----------------------
