@@ -683,6 +683,53 @@ static void batch_release(np_batch *b) {
     b->nconcat = 0;
 }
 
+// Buffers carved from the context's workspace: a first pass with base == nullptr sizes the
+// layout, the second hands out pointers (each 256-byte aligned).
+struct Carve {
+    char *base = nullptr;
+    size_t off = 0;
+    template <class T>
+    T *take(size_t count) {
+        off = (off + 255) & ~(size_t)255;
+        T *p = base ? reinterpret_cast<T *>(base + off) : nullptr;
+        off += sizeof(T) * (count ? count : 1);
+        return p;
+    }
+};
+
+// The context's workspace, grown to at least `bytes` (its old contents are dropped).
+static hipError_t ctx_workspace(np_ctx *c, size_t bytes, char **p) {
+    if (bytes > c->ws_bytes) {
+        if (c->ws) (void)hipFree(c->ws);
+        c->ws = nullptr;
+        c->ws_bytes = 0;
+        hipError_t e = hipMalloc((void **)&c->ws, bytes);
+        if (e != hipSuccess) return e;
+        c->ws_bytes = bytes;
+    }
+    *p = c->ws;
+    return hipSuccess;
+}
+
+// Buffers of np_bc.
+struct BcBufs {
+    int *ent_v, *srcs, *err;
+    uint2 *st;
+    int4 *rec;
+    BcLevel *lv;
+    unsigned *ent_m;
+    double *sig, *del, *acc;
+    float *out;
+    char *own = nullptr;  // the call's own allocation, when it is not the context's workspace
+    ~BcBufs() { dfree(own); }
+};
+
+// Twelve allocations and as many frees were 0.25 ms of a call on R-MAT s16 and 2 ms on s20 (32
+// sources: 10 % and 40 % of it); the buffers are carved from the context's workspace up to this
+// size.  Above it, the call allocates once and frees: the workspace is not shrunk while the context
+// lives, and a batch of a large graph takes 800 bytes per vertex.
+constexpr size_t BC_WORKSPACE = 1ull << 30;
+
 // ------------------------------------------------------------------------------------
 // C ABI
 // ------------------------------------------------------------------------------------
@@ -1082,22 +1129,6 @@ int np_reached_work(np_ctx *c, np_graph *g, const int32_t *d_dist, int32_t inf, 
 // bc_np_consolidate_gpu + BC_GPU (apps/bc/src/gpu/bc_wrapper.cu:678-809): sources in batches of
 // up to 32; per batch a level-synchronous forward BFS with path counts records every level's
 // entries, then the backward sweep replays them from the deepest level up.
-struct BcBufs {
-    int *ent_v = nullptr, *srcs = nullptr, *err = nullptr, *h_err = nullptr;
-    uint2 *st = nullptr;
-    int4 *rec = nullptr;
-    BcLevel *lv = nullptr, *h_lv = nullptr;
-    unsigned *ent_m = nullptr;
-    double *sig = nullptr, *del = nullptr, *acc = nullptr;
-    float *out = nullptr;
-    ~BcBufs() {
-        dfree(ent_v); dfree(srcs); dfree(err); dfree(st); dfree(rec); dfree(lv); dfree(ent_m);
-        dfree(sig); dfree(del); dfree(acc); dfree(out);
-        if (h_err) (void)hipHostFree(h_err);
-        if (h_lv) (void)hipHostFree(h_lv);
-    }
-};
-
 int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_out, np_stats *stats) {
     if (!c || !g || g->ctx != c || !bc_out || nsrc < 0 || (nsrc > 0 && !srcs)) {
         set_error("bad arguments"); return NP_ERR_ARG;
@@ -1122,41 +1153,52 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     const long long cap_e = (long long)n * P;  // entries of one batch: at most one per (vertex, source)
     if (cap_e > 0x7FFFFFFFll) { set_error("n x batch sources exceeds 2^31 entries"); return NP_ERR_CAPACITY; }
     const long long cap = g->m / 64 + (long long)n + 1;  // chunks of one level
-    BcBufs bb;
+    constexpr int BC_RUN = 64;  // forward levels per run at most
+    static_assert(BC_RUN * sizeof(BcLevel) <= H_SMALL * sizeof(unsigned long long), "the readback buffer holds a run");
+    // one record per forward level (lv[d]) and per backward level (lv[NB + d])
+    const size_t NB = (size_t)n + BC_RUN + 2;
     const size_t slots = (size_t)n << ks;
-    HIPCHK(dalloc(&bb.st, (size_t)n));
-    HIPCHK(dalloc(&bb.sig, slots));
-    HIPCHK(dalloc(&bb.del, slots));
-    HIPCHK(dalloc(&bb.ent_v, (size_t)cap_e));
-    HIPCHK(dalloc(&bb.ent_m, (size_t)cap_e));
-    HIPCHK(dalloc(&bb.rec, (size_t)cap));
-    HIPCHK(dalloc(&bb.err, 1));
+    BcBufs bb;
+    Carve cv;
+    for (int pass = 0; pass < 2; ++pass) {  // size, then carve
+        if (pass) {
+            if (cv.off <= BC_WORKSPACE) {
+                HIPCHK(ctx_workspace(c, cv.off, &cv.base));
+            } else {
+                HIPCHK(dalloc(&bb.own, cv.off));
+                cv.base = bb.own;
+            }
+            cv.off = 0;
+        }
+        bb.st = cv.take<uint2>((size_t)n);
+        bb.sig = cv.take<double>(slots);
+        bb.del = cv.take<double>(slots);
+        bb.ent_v = cv.take<int>((size_t)cap_e);
+        bb.ent_m = cv.take<unsigned>((size_t)cap_e);
+        bb.rec = cv.take<int4>((size_t)cap);
+        bb.lv = cv.take<BcLevel>(2 * NB);
+        bb.err = cv.take<int>(1);
+        bb.srcs = cv.take<int>(S.size());
+        bb.acc = cv.take<double>((size_t)n);
+        bb.out = cv.take<float>((size_t)n);
+    }
     HIPCHK(hipMemsetAsync(bb.err, 0, sizeof(int), c->stream));
-    HIPCHK(dalloc(&bb.srcs, 32));
-    HIPCHK(dalloc(&bb.acc, (size_t)n));
-    HIPCHK(dalloc(&bb.out, (size_t)n));
-    HIPCHK(hipHostMalloc((void **)&bb.h_err, sizeof(int)));
+    HIPCHK(hipMemcpyAsync(bb.srcs, S.data(), sizeof(int) * S.size(), hipMemcpyHostToDevice, c->stream));
+    BcLevel *h_lv = reinterpret_cast<BcLevel *>(c->h_small);
     // Forward levels go out several at a time with the entry counts kept on the device; the host
     // reads each run's (first entry, count) pairs once.  The first run is as long as the previous
     // source batch's depth + 1 (depths barely vary on one graph), at most BC_RUN; runs after it
     // have 2, 4, 8, ... levels (deep graphs), at most BC_RUN; levels past the last are empty and
     // cost a few small launches.
-    constexpr int BC_RUN = 64;
-    HIPCHK(hipHostMalloc((void **)&bb.h_lv, BC_RUN * sizeof(BcLevel)));
     int run = 8;
-    // one record per forward level (lv[d]) and per backward level (lv[NB + d]), zeroed once per
-    // source batch
-    const size_t NB = (size_t)n + BC_RUN + 2;
-    HIPCHK(dalloc(&bb.lv, 2 * NB));
     HIPCHK(hipMemsetAsync(bb.acc, 0, sizeof(double) * (size_t)n, c->stream));
     BcDev b{g->row, g->col, n, ks, bb.st, bb.sig, bb.del};
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     std::vector<std::pair<long long, int>> levels;
     for (size_t b0 = 0; b0 < S.size(); b0 += (size_t)P) {
         const int np_ = (int)std::min<size_t>((size_t)P, S.size() - b0);
-        HIPCHK(hipMemcpyAsync(bb.srcs, S.data() + b0, sizeof(int) * (size_t)np_, hipMemcpyHostToDevice, c->stream));
         HIPCHK(launch_bc_reset(b, c->stream));
-        HIPCHK(launch_bc_sources(b, bb.srcs, np_, c->stream));
+        HIPCHK(launch_bc_sources(b, bb.srcs + b0, np_, c->stream));
         levels.clear();
         long long E = 0;
         HIPCHK(hipMemsetAsync(bb.lv, 0, 2 * NB * sizeof(BcLevel), c->stream));
@@ -1168,13 +1210,13 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
                 HIPCHK(launch_bc_compact(b, bb.ent_v, bb.ent_m, bb.lv + d, bb.rec, cap, bb.err, c->stream));
                 HIPCHK(launch_bc_expand(b, true, bb.lv + d, bb.rec, cap, nullptr, c->num_cus, c->stream));
             }
-            HIPCHK(hipMemcpyAsync(bb.h_lv, bb.lv + d0, (size_t)k * sizeof(BcLevel), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipMemcpyAsync(h_lv, bb.lv + d0, (size_t)k * sizeof(BcLevel), hipMemcpyDeviceToHost, c->stream));
             int rc = ctx_sync(c);
             if (rc) return rc;
             for (int j = 0; j < k; ++j) {
-                const int ne = (int)(unsigned)bb.h_lv[j].ctl;
+                const int ne = (int)(unsigned)h_lv[j].ctl;
                 if (ne == 0) { last = d0 + j; break; }
-                levels.push_back({bb.h_lv[j].first, ne});
+                levels.push_back({h_lv[j].first, ne});
                 E += ne;
             }
         }
@@ -1195,10 +1237,10 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     HIPCHK(launch_bc_to_float(bb.acc, n, bb.out, c->stream));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     HIPCHK(hipMemcpyAsync(bc_out, bb.out, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(bb.h_err, bb.err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipMemcpyAsync(h_lv, bb.err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     int rc = ctx_sync(c);
     if (rc) return rc;
-    if (*bb.h_err) { set_error("a level exceeded its chunk capacity"); return NP_ERR_CAPACITY; }
+    if (*reinterpret_cast<const int *>(h_lv)) { set_error("a level exceeded its chunk capacity"); return NP_ERR_CAPACITY; }
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     st.kernel_ms = ms;
@@ -1207,34 +1249,6 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
 }
 
 }  // extern "C"
-
-// Buffers carved from the context's workspace: a first pass with base == nullptr sizes the
-// layout, the second hands out pointers (each 256-byte aligned).
-struct Carve {
-    char *base = nullptr;
-    size_t off = 0;
-    template <class T>
-    T *take(size_t count) {
-        off = (off + 255) & ~(size_t)255;
-        T *p = base ? reinterpret_cast<T *>(base + off) : nullptr;
-        off += sizeof(T) * (count ? count : 1);
-        return p;
-    }
-};
-
-// The context's workspace, grown to at least `bytes` (its old contents are dropped).
-static hipError_t ctx_workspace(np_ctx *c, size_t bytes, char **p) {
-    if (bytes > c->ws_bytes) {
-        if (c->ws) (void)hipFree(c->ws);
-        c->ws = nullptr;
-        c->ws_bytes = 0;
-        hipError_t e = hipMalloc((void **)&c->ws, bytes);
-        if (e != hipSuccess) return e;
-        c->ws_bytes = bytes;
-    }
-    *p = c->ws;
-    return hipSuccess;
-}
 
 extern "C" {
 
