@@ -81,6 +81,7 @@ struct Space {
     int *src_slots = nullptr;
     int src_cap = 0;
     unsigned *mflag = nullptr;    // source-packed: pending sources per vertex
+    unsigned *deferred = nullptr; // source-packed, from the first solve with a priority window on
     unsigned *qmask[2] = {nullptr, nullptr};
     unsigned char *bound = nullptr;  // source-packed: bound filter (skewed graphs)
     int *sbuf = nullptr, *sbcnt = nullptr;  // NP_SCHEME_GLOBAL_BUFFER (allocated on first use)
@@ -108,7 +109,7 @@ struct Space {
         if (own_cls) dfree(cls);
         cls = nullptr;
         dfree(lut); dfree(inst); dfree(src_slots);
-        dfree(mflag); dfree(qmask[0]); dfree(qmask[1]); dfree(bound);
+        dfree(mflag); dfree(deferred); dfree(qmask[0]); dfree(qmask[1]); dfree(bound);
         dfree(sbuf); dfree(sbcnt);
         dfree(pctrl);
         if (h_pctrl) (void)hipHostFree(h_pctrl);
@@ -1808,6 +1809,10 @@ int np_batch_solve(np_ctx *c, np_batch *b, const np_sched *sched, np_stats *stat
             // hold a heavy vertex while fewer than 3/4 of the pack's sources have reached it
             st.hold_cls = psch.pack_hold;
             st.hold_min = (3 * (int)pk->inst.size() + 3) / 4;
+        }
+        if (psch.delta > 0) {
+            if (!s.deferred) HIPCHK(dalloc(&s.deferred, (size_t)s.nslots));
+            st.deferred = s.deferred;
         }
         if (s.bound && psch.drive != NP_DRIVE_PERSISTENT && psch.delta <= 0) {
             st.bound = s.bound;

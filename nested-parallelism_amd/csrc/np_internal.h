@@ -34,6 +34,7 @@ struct Ctrl {
     int thresh;               // priority window: vertices with dist < thresh are expanded
     int pass;                 // compaction passes so far (host-loop / graph drives)
     int skip;                 // host-loop / graph drives: this slot only raised the window
+    int full;                 // windowed pack: the next compaction looks at the deferred pairs too
     long long edges_total;    // source-packed: sum over iterations of the queued vertices' out-degrees
     long long items_total;    // source-packed: ... of out-degree x queued sources ((edge, source) items)
     int solo;                 // persistent drive: iterations of the last solo visit
@@ -79,6 +80,9 @@ struct DevState {
     // (once per flagging; bm[1] marks the held vertices); hold_cls 0 = never
     int hold_cls;
     int hold_min;
+    // source-packed with a priority window: sources of v whose distance was not below the window when
+    // it was last looked at (bm[1]: vertices with some); null without a window
+    unsigned *deferred;
     // source-packed bound filter (see pk_bound_code): one byte per vertex, null = off; a code step
     // is 2^fshift, and at least fmin sources have to have reached the hub (solver id 0)
     unsigned char *bound;

@@ -488,28 +488,19 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
 // least distance among them to the pass's deferral sums (BarLeaf).  T = INT_MAX queues every flag.
 constexpr int NO_WINDOW = 0x7FFFFFFF;
 
-// Without a window frontiers are sparse and whole bitmap words are skipped (compaction_impl, and its
-// form in pk_compaction).  With a priority window a source-packed frontier is dense (deferred
-// vertices stay flagged and are re-read every pass): there each thread owns CPT vertices of a tile
-// of WG * CPT consecutive ones, so the lanes of a wave read the class bytes, masks and distance rows
-// of consecutive vertices and the 32 lanes of one bitmap word rewrite it with one store.  Both count
-// queue slots per class in LDS and reserve them once per class per tile.
-constexpr int CPT = 4;
-
-// One bitmap word per 32 lanes: the first lane of each half-wave stores the kept bits when the
-// word changed.  v is this lane's vertex; its half-wave covers one word.
-__device__ __forceinline__ void rewrite_word(unsigned *bm, long long v, long long nv, unsigned word, bool keep) {
-    const unsigned nw = (unsigned)(__ballot(keep) >> (lane_id() & 32));
-    if ((lane_id() & 31) == 0 && v < nv && nw != word) st_coherent_u(bm + (v >> 5), nw);
-}
-
-// LDS class counters of this tile -> global reservation (s_lb) and reset for the next tile.
-__device__ __forceinline__ void reserve_classes(int *s_lc, int *s_lb, int *cnt_out) {
+// The waves' class counters of this tile -> global reservation: s_wc[w][c] becomes wave w's first
+// place of class c, so that a wave's vertices stay together in the queue.
+__device__ __forceinline__ void reserve_classes(int (*s_wc)[NCLS], int *cnt_out) {
     __syncthreads();
     if (threadIdx.x < NCLS) {
-        const int k = s_lc[threadIdx.x];
-        s_lb[threadIdx.x] = k ? atomicAdd(&cnt_out[threadIdx.x], k) : 0;
-        s_lc[threadIdx.x] = 0;
+        int k = 0;
+        for (int w = 0; w < WAVES; ++w) k += s_wc[w][threadIdx.x];
+        int at = k ? atomicAdd(&cnt_out[threadIdx.x], k) : 0;
+        for (int w = 0; w < WAVES; ++w) {
+            const int t = s_wc[w][threadIdx.x];
+            s_wc[w][threadIdx.x] = at;
+            at += t;
+        }
     }
     __syncthreads();
 }
@@ -1003,6 +994,15 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
     const int pass = ld_coherent(&ctrl->pass);  // the compaction of this slot
     if (tot == 0 && !sp.push) {
         const int T = ld_coherent(&ctrl->thresh);
+        if (st.deferred && T != NO_WINDOW && !ld_coherent(&ctrl->full)) {
+            // a windowed pack's passes look at the flagged pairs only: now at the deferred ones
+            if (threadIdx.x == 0) {
+                ctrl->full = 1;
+                ctrl->skip = 1;
+                ctrl->pass = pass + 1;
+            }
+            return;
+        }
         int kept, mn;
         deferred_sums(ctrl, pass % 3, &kept, &mn);
         if ((T != NO_WINDOW || st.hold_cls) && kept > 0) {
@@ -1052,6 +1052,7 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
         record_trace(sp, ctrl->iters, cfg, s_cnt, (long long)wall_clock64(), ctrl);
         ctrl->iters += 1;
         ctrl->skip = 0;
+        ctrl->full = 0;
         if (!sp.push) ctrl->pass = pass + 1;
     }
 }
@@ -1851,203 +1852,213 @@ __device__ __forceinline__ int pk_reached(const DevState &st, long long v) {
     return r;
 }
 
-// The pending sources of v (mask m) whose distance at v is below the window T; *dmin
-// receives the least distance among the others.  The row is read with 16-byte loads
-// through the caches: a value older than the last atomicMin is only larger, so it can
-// only keep a pair pending one pass longer (every pending pair is expanded eventually).
-__device__ __forceinline__ unsigned pk_take(const DevState &st, long long v, unsigned m, int T, int *dmin) {
-    *dmin = NO_WINDOW;
-    if (T == NO_WINDOW) return m;
+// Lane q of a group of 8 has vertex v's distances of sources 4q .. 4q + 3 (rows of 1 or 2: source q).
+// Through the caches: a value older than the last atomicMin is only larger, so it can only keep a
+// pair pending one pass longer (every pending pair is expanded eventually).
+__device__ __forceinline__ int4 pk_row_part(const DevState &st, long long v, int q, bool ok) {
     const int *row = st.dist + (v << st.kshift);
+    if (st.kshift < 2) return int4{ok && q < (1 << st.kshift) ? row[q] : 0, 0, 0, 0};
+    return ok && q < (1 << (st.kshift - 2)) ? ((const int4 *)row)[q] : int4{0, 0, 0, 0};
+}
+// The group's sources of mask m whose distance is below the window T, and the least distance among
+// its others (both in every lane of the group).
+__device__ __forceinline__ unsigned pk_take(const DevState &st, int4 x, int q, unsigned m, int T, int *dmin) {
+    const int d[4] = {x.x, x.y, x.z, x.w};
+    const int per = st.kshift < 2 ? 1 : 4;
     unsigned take = 0;
     int dm = NO_WINDOW;
-    if (st.kshift < 2) {  // rows of 1 or 2 distances
-        for (unsigned b = m; b; b &= b - 1) {
-            const int i = __ffs(b) - 1, d = row[i];
-            if (d < T) take |= 1u << i;
-            else dm = d < dm ? d : dm;
-        }
-    } else {
-        const int4 *row4 = (const int4 *)row;
-        const int nq = 1 << (st.kshift - 2);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            if (q >= nq || !((m >> (4 * q)) & 0xFu)) continue;
-            const int4 x = row4[q];
-            const int d[4] = {x.x, x.y, x.z, x.w};
+    for (int k = 0; k < 4; ++k) {
+        if (k >= per || !((m >> (per * q + k)) & 1u)) continue;
+        if (d[k] < T || T == NO_WINDOW) take |= 1u << (per * q + k);
+        else dm = d[k] < dm ? d[k] : dm;
+    }
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                if (!((m >> (4 * q + k)) & 1u)) continue;
-                if (d[k] < T) take |= 1u << (4 * q + k);
-                else dm = d[k] < dm ? d[k] : dm;
-            }
-        }
+    for (int o = 1; o < 8; o <<= 1) {
+        take |= (unsigned)__shfl_xor((int)take, o);
+        const int y = __shfl_xor(dm, o);
+        dm = y < dm ? y : dm;
     }
     *dmin = dm;
     return take;
 }
 
 // Vertices with pending sources -> class-segmented queue with their source masks.  With a
-// priority window (T < NO_WINDOW) only the (vertex, source) pairs with dist < T are queued;
-// the others stay pending in mflag[v] (and v in the bitmap), and the pass adds their count and
-// least distance to the pass's deferral sums.
+// priority window (T < NO_WINDOW) only the (vertex, source) pairs with dist < T are queued; the
+// others move from mflag[v] to deferred[v] (and v from bm[0] to bm[1]).  A deferred pair is below
+// the window only after a relaxation, which flags it again, or after the window has risen: so the
+// passes of one window look at the flagged pairs alone, and only a `full` pass, once before the
+// window rises (the deferred pairs' count and least distance go to the pass's deferral sums) and
+// once after, looks at every deferred one.  Kept flagged and re-read in every pass by a lane per
+// row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid 16.5 -> 7.4 ms
+// of it per solve (13.4 with a lane per row still), the expansions 16.0 -> 18.4 (a deferred vertex that
+// is flagged again sets its frontier bit again), the solve 33.2 -> 26.5 ms.
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
-                                              int T, int slot) {
-    __shared__ int s_lc[NCLS], s_lb[NCLS];
+                                              int T, bool full, int slot) {
+    __shared__ int s_wc[WAVES][NCLS];
+    static_assert(WAVES * NCLS <= WG, "cleared by one store each");
     __shared__ int s_dc, s_dm, s_pairs;
     unsigned *bm = st.bm[0];
     if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; s_pairs = 0; }
-    if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;
+    if (threadIdx.x < WAVES * NCLS) s_wc[0][threadIdx.x] = 0;
     __syncthreads();
     int pairs = 0, my_dc = 0, my_dm = NO_WINDOW;
-    const long long nv = st.nwords * 32;
-    // Without a window every pending vertex is taken whole and nothing stays flagged but the hubs
-    // held for one pass (hold_cls): the words are scanned as compaction_impl does (a thread per word
-    // took 0.24 ms where this takes 0.1, R-MAT s24, 16 sources, 8 M vertices queued).
-    if (T == NO_WINDOW) {
-        __shared__ unsigned short s_list[WAVES][64 * 32];
-        __shared__ unsigned s_held[WG];  // per word of the wave: held vertices, and whether it has hubs
-        __shared__ int s_heavy[WG];
-        const int lane = lane_id(), half = lane & 31;
-        unsigned short *list = s_list[threadIdx.x >> 6];
-        const int wt = compact_words(st.nwords);
-        const long long tile = (long long)WAVES * wt;
-        for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
-            const long long w0 = wb + (threadIdx.x >> 6) * wt;
-            const unsigned word = lane < wt && w0 + lane < st.nwords ? ld_coherent_u(bm + w0 + lane) : 0u;
-            unsigned long long nz = __ballot(word != 0);
-            int n = 0;
-            while (nz) {
-                int idx[COMPACT_UNR], c[COMPACT_UNR];
-                unsigned x[COMPACT_UNR];
+    const bool windowed = T != NO_WINDOW || full;
+    // The words are scanned as compaction_impl does (a thread per word took 0.24 ms where this takes
+    // 0.1, R-MAT s24, 16 sources, 8 M vertices queued); then the hubs held for one pass (hold_cls) or
+    // the vertices without a pair below the window leave the list.
+    __shared__ unsigned short s_list[WAVES][64 * 32];
+    __shared__ unsigned s_held[WG];  // per word of the wave: held or deferred vertices, and whether it has hubs
+    __shared__ int s_heavy[WG];
+    const int lane = lane_id(), half = lane & 31;
+    unsigned short *list = s_list[threadIdx.x >> 6];
+    int *wc = s_wc[threadIdx.x >> 6];
+    const int wt = compact_words(st.nwords);
+    const long long tile = (long long)WAVES * wt;
+    for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
+        const long long w0 = wb + (threadIdx.x >> 6) * wt;
+        const bool in = lane < wt && w0 + lane < st.nwords;
+        const unsigned flagged = in ? ld_coherent_u(bm + w0 + lane) : 0u;
+        const unsigned later = windowed && in ? ld_coherent_u(st.bm[1] + w0 + lane) : 0u;
+        const unsigned word = full ? flagged | later : flagged;
+        unsigned long long nz = __ballot(word != 0);
+        int n = 0;
+        while (nz) {
+            int idx[COMPACT_UNR], c[COMPACT_UNR];
+            unsigned x[COMPACT_UNR];
 #pragma unroll
-                for (int k = 0; k < COMPACT_UNR; ++k) {
-                    const int ia = __ffsll((long long)nz) - 1;
-                    nz &= nz - 1;
-                    const int ib = __ffsll((long long)nz) - 1;
-                    nz &= nz - 1;
-                    idx[k] = lane < 32 ? ia : ib;  // -1: none left
-                    x[k] = __shfl(word, idx[k] < 0 ? 0 : idx[k]);
-                    if (idx[k] < 0) x[k] = 0u;
-                    // no out-edges (class 0): dropped (mflag stays set, so it is not flagged again)
-                    c[k] = (x[k] >> half) & 1u ? (int)st.cls[(w0 + idx[k]) * 32 + half] : 0;
-                }
-#pragma unroll
-                for (int k = 0; k < COMPACT_UNR; ++k) {
-                    const unsigned long long m = __ballot(c[k] != 0);
-                    if (c[k]) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
-                    n += __popcll(m);
-                }
+            for (int k = 0; k < COMPACT_UNR; ++k) {
+                const int ia = __ffsll((long long)nz) - 1;
+                nz &= nz - 1;
+                const int ib = __ffsll((long long)nz) - 1;
+                nz &= nz - 1;
+                idx[k] = lane < 32 ? ia : ib;  // -1: none left
+                x[k] = __shfl(word, idx[k] < 0 ? 0 : idx[k]);
+                if (idx[k] < 0) x[k] = 0u;
+                // no out-edges (class 0): dropped (mflag stays set, so it is not flagged again)
+                c[k] = (x[k] >> half) & 1u ? (int)st.cls[(w0 + idx[k]) * 32 + half] : 0;
             }
-            unsigned stay = 0;  // flags of this lane's word that stay
-            if (st.hold_cls) {
-                // hubs that more sources are on their way to wait one pass and keep their flag; a held
-                // vertex stays flagged, so the held bits are always a subset of the flags: they become
-                // exactly this pass's held vertices (the ones held before are queued).  Renumbered hubs
-                // share a wavefront's words, so their rows are read COMPACT_UNR x 64 at a time.
-                s_held[threadIdx.x] = 0u;
-                s_heavy[threadIdx.x] = 0;
-                unsigned *held_w = s_held + (threadIdx.x & ~63);
-                int *heavy_w = s_heavy + (threadIdx.x & ~63);
-                __builtin_amdgcn_wave_barrier();
-                int left = 0;
-                for (int base = 0; base < n; base += 64 * COMPACT_UNR) {
-                    int e[COMPACT_UNR], reached[COMPACT_UNR];
-                    unsigned hw[COMPACT_UNR];
 #pragma unroll
-                    for (int k = 0; k < COMPACT_UNR; ++k) {
-                        const int i = base + 64 * k + lane;
-                        e[k] = i < n ? (int)list[i] : 0;
-                        const bool heavy = (e[k] >> 11) >= st.hold_cls;
-                        hw[k] = heavy ? ld_coherent_u(st.bm[1] + w0 + ((e[k] & 2047) >> 5)) : 0u;
-                        reached[k] = heavy ? pk_reached(st, w0 * 32 + (e[k] & 2047)) : st.hold_min;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                    for (int k = 0; k < COMPACT_UNR; ++k) {
-                        const int wi = (e[k] & 2047) >> 5, bit = e[k] & 31;
-                        const bool heavy = (e[k] >> 11) >= st.hold_cls;
-                        const bool held = heavy && !((hw[k] >> bit) & 1u) && reached[k] < st.hold_min;
-                        if (heavy) heavy_w[wi] = 1;
-                        if (held) atomicOr(&held_w[wi], 1u << bit);
-                        my_dc += held;
-                        const bool take = e[k] != 0 && !held;
-                        const unsigned long long m = __ballot(take);
-                        if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
-                        left += __popcll(m);
-                    }
-                }
-                n = left;
-                __builtin_amdgcn_wave_barrier();
-                stay = s_held[threadIdx.x];
-                if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
+            for (int k = 0; k < COMPACT_UNR; ++k) {
+                const unsigned long long m = __ballot(c[k] != 0);
+                if (c[k]) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
+                n += __popcll(m);
             }
-            if (word != stay) st_coherent_u(bm + w0 + lane, stay);
-            if (!__syncthreads_or(n)) continue;  // s_lc is clear, nothing was counted
-            for (int i = lane; i < n; i += 64) atomicAdd(&s_lc[list[i] >> 11], 1);
-            reserve_classes(s_lc, s_lb, cnt_out);
-            for (int i = lane; i < n; i += 64) {
-                const int e = list[i], c = e >> 11;
-                const long long v = w0 * 32 + (e & 2047);
-                const unsigned t = ld_coherent_u(st.mflag + v);
-                st_coherent_u(st.mflag + v, 0u);
-                const long long qi = st.seg_off[c] + s_lb[c] + atomicAdd(&s_lc[c], 1);
-                if (seg_ok(st.ctrl, qi, st.seg_off[c], st.seg_off[c + 1])) {
-                    st_coherent(q_out + qi, (int)v);
-                    st_coherent_u(qm_out + qi, t);
-                }
-                pairs += __popc(t);
-            }
-            __syncthreads();
-            if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;  // the last loop counted in s_lc
-            __syncthreads();
         }
-    }
-    for (long long vb = (long long)blockIdx.x * (WG * CPT); T != NO_WINDOW && vb < nv;
-         vb += (long long)gridDim.x * (WG * CPT)) {
-        int qc[CPT], qp[CPT];
-        unsigned qt[CPT];
+        unsigned stay = 0;  // flags of this lane's word that stay
+        if (windowed) {
+            // 8 lanes per vertex read its row; a vertex with a pair below the window keeps its
+            // mask for the queue in mflag, the others leave the list
+            constexpr int WIN_UNR = 4;
+            unsigned *held_w = s_held + (threadIdx.x & ~63);
+            s_held[threadIdx.x] = 0u;
+            __builtin_amdgcn_wave_barrier();
+            const int g = lane >> 3, q = lane & 7;
+            int left = 0;
+            for (int base = 0; base < n; base += 8 * WIN_UNR) {
+                int e[WIN_UNR];
+                unsigned f[WIN_UNR], old[WIN_UNR];
+                int4 x[WIN_UNR];
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const long long v = vb + k * WG + threadIdx.x;
-            const unsigned word = v < nv ? ld_coherent_u(bm + (v >> 5)) : 0u;
-            bool keep = false;
-            qc[k] = 0;
-            qp[k] = 0;
-            qt[k] = 0;
-            if ((word >> (v & 31)) & 1u) {
-                const int c = st.cls[v];
-                if (c) {  // no out-edges: dropped (its mflag stays set, so it is not flagged again)
-                    const unsigned m = ld_coherent_u(st.mflag + v);
+                for (int k = 0; k < WIN_UNR; ++k) {
+                    const int i = base + 8 * k + g;
+                    e[k] = i < n ? (int)list[i] : 0;  // class 0: none
+                    const long long v = w0 * 32 + (e[k] & 2047);
+                    const unsigned lw = __shfl(later, (e[k] & 2047) >> 5);
+                    f[k] = e[k] ? ld_coherent_u(st.mflag + v) : 0u;
+                    old[k] = e[k] && ((lw >> (e[k] & 31)) & 1u) ? ld_coherent_u(st.deferred + v) : 0u;
+                    x[k] = pk_row_part(st, v, q, e[k] != 0);
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int k = 0; k < WIN_UNR; ++k) {
+                    const long long v = w0 * 32 + (e[k] & 2047);
                     int dmin;
-                    const unsigned t = pk_take(st, v, m, T, &dmin);
-                    if (t) {
-                        qc[k] = c;
-                        qt[k] = t;
-                        qp[k] = atomicAdd(&s_lc[c], 1);
-                        st_coherent_u(st.mflag + v, m & ~t);
+                    const unsigned t = pk_take(st, x[k], q, full ? f[k] | old[k] : f[k], T, &dmin);
+                    const unsigned rest = (old[k] | f[k]) & ~t;
+                    const bool take = q == 0 && t != 0;
+                    if (q == 0 && e[k]) {
+                        if (f[k] != t) st_coherent_u(st.mflag + v, t);
+                        if (rest != old[k]) st_coherent_u(st.deferred + v, rest);
+                        if (rest) {
+                            atomicOr(&held_w[(e[k] & 2047) >> 5], 1u << (e[k] & 31));
+                            if (full) {
+                                my_dc += __popc(rest);
+                                my_dm = dmin < my_dm ? dmin : my_dm;
+                            }
+                        }
                     }
-                    if (t != m) {
-                        keep = true;
-                        my_dc += __popc(m & ~t);
-                        my_dm = dmin < my_dm ? dmin : my_dm;
-                    }
+                    const unsigned long long m = __ballot(take);
+                    if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
+                    left += __popcll(m);
                 }
             }
-            rewrite_word(bm, v, nv, word, keep);
+            n = left;
+            __builtin_amdgcn_wave_barrier();
+            const unsigned now = (later & ~word) | s_held[threadIdx.x];
+            if (now != later) st_coherent_u(st.bm[1] + w0 + lane, now);
         }
-        reserve_classes(s_lc, s_lb, cnt_out);
+        if (st.hold_cls) {
+            // hubs that more sources are on their way to wait one pass and keep their flag; a held
+            // vertex stays flagged, so the held bits are always a subset of the flags: they become
+            // exactly this pass's held vertices (the ones held before are queued).  Renumbered hubs
+            // share a wavefront's words, so their rows are read COMPACT_UNR x 64 at a time.
+            s_held[threadIdx.x] = 0u;
+            s_heavy[threadIdx.x] = 0;
+            unsigned *held_w = s_held + (threadIdx.x & ~63);
+            int *heavy_w = s_heavy + (threadIdx.x & ~63);
+            __builtin_amdgcn_wave_barrier();
+            int left = 0;
+            for (int base = 0; base < n; base += 64 * COMPACT_UNR) {
+                int e[COMPACT_UNR], reached[COMPACT_UNR];
+                unsigned hw[COMPACT_UNR];
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            if (!qc[k]) continue;
-            const long long qi = st.seg_off[qc[k]] + s_lb[qc[k]] + qp[k];
-            const long long v = vb + k * WG + threadIdx.x;
-            if (seg_ok(st.ctrl, qi, st.seg_off[qc[k]], st.seg_off[qc[k] + 1])) {
-                st_coherent(q_out + qi, (int)v);
-                st_coherent_u(qm_out + qi, qt[k]);
+                for (int k = 0; k < COMPACT_UNR; ++k) {
+                    const int i = base + 64 * k + lane;
+                    e[k] = i < n ? (int)list[i] : 0;
+                    const bool heavy = (e[k] >> 11) >= st.hold_cls;
+                    hw[k] = heavy ? ld_coherent_u(st.bm[1] + w0 + ((e[k] & 2047) >> 5)) : 0u;
+                    reached[k] = heavy ? pk_reached(st, w0 * 32 + (e[k] & 2047)) : st.hold_min;
+                }
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int k = 0; k < COMPACT_UNR; ++k) {
+                    const int wi = (e[k] & 2047) >> 5, bit = e[k] & 31;
+                    const bool heavy = (e[k] >> 11) >= st.hold_cls;
+                    const bool held = heavy && !((hw[k] >> bit) & 1u) && reached[k] < st.hold_min;
+                    if (heavy) heavy_w[wi] = 1;
+                    if (held) atomicOr(&held_w[wi], 1u << bit);
+                    my_dc += held;
+                    const bool take = e[k] != 0 && !held;
+                    const unsigned long long m = __ballot(take);
+                    if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
+                    left += __popcll(m);
+                }
             }
-            pairs += __popc(qt[k]);
+            n = left;
+            __builtin_amdgcn_wave_barrier();
+            stay = s_held[threadIdx.x];
+            if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
         }
+        if (flagged != stay) st_coherent_u(bm + w0 + lane, stay);
+        if (!__syncthreads_or(n)) continue;  // s_wc is clear, nothing was counted
+        for (int i = lane; i < n; i += 64) atomicAdd(&wc[list[i] >> 11], 1);
+        reserve_classes(s_wc, cnt_out);
+        for (int i = lane; i < n; i += 64) {
+            const int e = list[i], c = e >> 11;
+            const long long v = w0 * 32 + (e & 2047);
+            const unsigned t = ld_coherent_u(st.mflag + v);
+            st_coherent_u(st.mflag + v, 0u);
+            const long long qi = st.seg_off[c] + atomicAdd(&wc[c], 1);
+            if (seg_ok(st.ctrl, qi, st.seg_off[c], st.seg_off[c + 1])) {
+                st_coherent(q_out + qi, (int)v);
+                st_coherent_u(qm_out + qi, t);
+            }
+            pairs += __popc(t);
+        }
+        __syncthreads();
+        if (threadIdx.x < WAVES * NCLS) s_wc[0][threadIdx.x] = 0;  // the last loop counted in s_wc
+        __syncthreads();
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o);
@@ -2055,7 +2066,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     __syncthreads();
     if (threadIdx.x == 0 && s_pairs)
         atomicAdd((unsigned long long *)&st.ctrl->leaf[blockIdx.x % BAR_LEAVES].pairs, (unsigned long long)s_pairs);
-    if (T != NO_WINDOW || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
+    if (full || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
 }
 
 // Lane-bin bound of a packed expansion (see PACK_LANE_CLS); the other bins keep theirs.  A filtered
@@ -2082,6 +2093,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
     long long t_prev = 0;
     // priority window: every workgroup computes the same sequence of thresholds
     int T = sp.delta > 0 ? sp.delta : NO_WINDOW;
+    bool full = false;
     int pass = 0;
     for (int it = 0;; ++it) {
         int *cnt_cur = st.cnt + (it % 3) * NCLS;
@@ -2098,7 +2110,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             const int slot = pass % 3;
             // the statistics slot of the next pass was last read before the previous barrier
             if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-            pk_compaction(st, cnt_cur, q_cur, qm_cur, T, slot);
+            pk_compaction(st, cnt_cur, q_cur, qm_cur, T, full, slot);
             if (!grid_sync(ctrl, nb, gen)) return;
             pass++;
             if (threadIdx.x < NCLS) {
@@ -2111,10 +2123,17 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
                 if (threadIdx.x == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
             }
             __syncthreads();
-            if (s_total > 0) break;
-            // nothing queued: done unless pairs were kept back (below the window, or held
-            // vertices, which the next pass takes); a window rises to the least pending
-            // distance + delta
+            if (s_total > 0) {
+                full = false;
+                break;
+            }
+            // nothing queued: the deferred pairs are looked at; done unless pairs were kept back
+            // (by the window, or held vertices, which the next pass takes); a window rises to the
+            // least pending distance + delta
+            if (T != NO_WINDOW && !full) {
+                full = true;
+                continue;
+            }
             int kept, mn;
             deferred_sums(ctrl, slot, &kept, &mn);
             if (kept == 0) break;
@@ -2151,7 +2170,8 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
     if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-    pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, pass % 3);
+    pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
+                  pass % 3);
 }
 
 // Every vertex's bound, once: between the compaction and the decision that records the offsets (no
@@ -2719,8 +2739,9 @@ hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, i
     hipError_t e;
     if ((e = launch_fill_i32(st.dist, st.nslots << st.kshift, st.inf, s)) != hipSuccess) return e;
     if ((e = launch_fill_u32(st.bm[0], st.nwords, 0u, s)) != hipSuccess) return e;
-    if (st.hold_cls && (e = launch_fill_u32(st.bm[1], st.nwords, 0u, s)) != hipSuccess) return e;
+    if ((st.hold_cls || st.deferred) && (e = launch_fill_u32(st.bm[1], st.nwords, 0u, s)) != hipSuccess) return e;
     if ((e = launch_fill_u32(st.mflag, st.nslots, 0u, s)) != hipSuccess) return e;
+    if (st.deferred && (e = launch_fill_u32(st.deferred, st.nslots, 0u, s)) != hipSuccess) return e;
     if (st.bound && (e = launch_fill_u32((unsigned *)st.bound, (st.nslots + 3) / 4, ~0u, s)) != hipSuccess) return e;
     if ((e = launch_fill_i32(st.cnt, 3 * NCLS, 0, s)) != hipSuccess) return e;
     if (st.sbcnt && (e = launch_fill_i32(st.sbcnt, 3, 0, s)) != hipSuccess) return e;

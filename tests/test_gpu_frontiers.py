@@ -132,3 +132,31 @@ def test_rows_longer_than_a_workgroup_chunk(npa, ctx, orc, deg):
     dst = rng.integers(0, n, len(src))
     row, col, w = _csr(src, dst, rng.integers(1, 200, len(src)), n)
     _check(npa, ctx, orc, row, col, w, 5, [npa.Sched(level=1, drive=dr, frontier=fr) for dr in (0, 1, 2) for fr in (0, 1)])
+
+
+@pytest.mark.parametrize("nsrc", [2, 3, 8, 17, 32])
+@pytest.mark.parametrize("kind", ["grid", "rmat", "dead_ends"])
+def test_packed_window_moves_deferred_pairs(npa, ctx, orc, kind, nsrc):
+    """Windowed packs: pairs deferred, flagged again below and above the window, taken when it
+    rises; from a window that defers nearly everything to one that ends at its first rise and one
+    whose first rise would pass the largest threshold; repeated solves on one batch, with solves
+    without a window between."""
+    rng = np.random.default_rng(nsrc)
+    if kind == "grid":
+        G = npa.Graph.grid(ctx, 40, 53, None, 1, 255, seed=61)
+    elif kind == "rmat":
+        G = npa.Graph.rmat(ctx, 11, 8, wmin=1, wmax=255, seed=62)
+    else:                                   # vertices without out-edges, zero weights, unreached vertices
+        row, col, w = random_csr(rng, 1500, 4000, 0, 300)
+        G = npa.Graph.from_csr(ctx, row, col, w)
+    row, col, w = G.download()
+    srcs = [int(s) for s in rng.integers(0, G.n, nsrc)]
+    ref = [orc.dijkstra(row, col, w, s)[0] for s in srcs]
+    b = npa.Batch(ctx, [G] * nsrc, srcs)
+    for dr in (0, 1, 2):
+        for delta in (1, 40, 0, 700, 2 ** 30):
+            b.solve(npa.Sched(level=2, log2_t_lo=3, log2_t_hi=7, drive=dr, delta=delta))
+            for i in range(nsrc):
+                assert np.array_equal(b.get(i), ref[i]), (dr, delta, i)
+    b.free()
+    G.free()
