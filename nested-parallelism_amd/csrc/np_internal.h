@@ -63,8 +63,8 @@ struct DevState {
     int inf;                  // unreached value written at init
     Ctrl *ctrl;
     // source-packed batch (kshift >= 0): 2^kshift sources of one graph per vertex row,
-    // dist[(v << kshift) + i]; mflag[v] = sources pending at v; bm[0] = vertices with a
-    // nonzero mflag; qmask[] = source mask of each queue entry
+    // dist[(v << kshift) + i]; mflag[v] = sources pending at v; bm[0] = one byte per 8
+    // vertices, nonzero where an mflag may be; qmask[] = source mask of each queue entry
     int kshift;               // -1: one distance per slot
     unsigned *mflag;
     unsigned *qmask[2];
@@ -81,7 +81,7 @@ struct DevState {
     int hold_cls;
     int hold_min;
     // source-packed with a priority window: sources of v whose distance was not below the window when
-    // it was last looked at (bm[1]: vertices with some); null without a window
+    // it was last looked at; null without a window
     unsigned *deferred;
     // source-packed bound filter (see pk_bound_code): one byte per vertex, null = off; a code step
     // is 2^fshift, and at least fmin sources have to have reached the hub (solver id 0)

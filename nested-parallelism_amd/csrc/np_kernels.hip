@@ -49,6 +49,9 @@ __device__ __forceinline__ unsigned ld_coherent_u(const unsigned *p) {
 __device__ __forceinline__ void st_coherent(int *p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, NP_AGENT);
 }
+__device__ __forceinline__ void st_coherent_b(unsigned char *p, unsigned char v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, NP_AGENT);
+}
 __device__ __forceinline__ void st_coherent_u(unsigned *p, unsigned v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, NP_AGENT);
 }
@@ -1360,8 +1363,8 @@ __global__ __launch_bounds__(WG) void k_bfs_hier(DevState st, int it_off) {
 // so one read of an edge's col/w serves every source pending at its tail, and the check
 // of dist[v][*] is one coalesced line instead of one random sector per source.
 // mflag[v] collects the sources whose distance at v improved since v was last queued;
-// bm[0] has one bit per vertex with a nonzero mflag (set by the relaxation that made it
-// nonzero), so the compaction scans n/8 bytes and reads mflag only where work is pending.
+// the relaxation that made it nonzero also stores 1 to a byte that 8 vertices share (pk_mark, in
+// bm[0]), so the compaction scans n/8 bytes and reads mflag only where work is pending.
 // A queue entry carries the source mask it was queued with (qmask).  The work of a
 // queued vertex is out-degree x pending sources; its items are numbered edge-major,
 // item t = (edge t / P, t % P-th pending source), so the P lanes of one edge are adjacent.
@@ -1384,6 +1387,15 @@ __device__ __forceinline__ int nth_set_bit(unsigned m, int k) {
 // short rows; longer ones go to the wavefront and wider bins whatever the schedule says.
 constexpr int PACK_LANE_CLS = 10;
 
+// The mark of v and its 7 neighbours.  A byte, set by a plain store: as a bit set by an atomicOr it
+// was a third of the atomics of a sparse graph's expansion (27 G lines/s whatever they do), 32
+// sources of a 2048^2 grid 26.5 -> 22.1 ms per solve, of 1024^2 9.3 -> 7.7 (ER 1 M and R-MAT within
+// 3 % either way).  A byte per 32 vertices made ER 65,536 25 to 30 % slower: stores to one line take
+// turns too.
+__device__ __forceinline__ unsigned char *pk_mark(const DevState &st, long long v) {
+    return (unsigned char *)st.bm[0] + (v >> 3);
+}
+
 // UNR packed relaxation steps of a wavefront: in step k every lane holds one (edge, source)
 // item -- target tv[k], pending source s, candidate alt[k] = dist[u][s] + w, loaded dist[v][s]
 // cur[k] -- or none (ok[k] false).  The lanes of one edge form a run of consecutive lanes (rs =
@@ -1391,7 +1403,7 @@ constexpr int PACK_LANE_CLS = 10;
 // The reference's relaxation per item (sssp_kernel.cu:46-52): if (dist[v][s] > alt) atomicMin,
 // issued without a return value; each source that passed the check sets its bit in mflag[v],
 // OR-ed across the run first so that one lane per run updates it, and the first bit of mflag[v]
-// sets v's frontier bit.  Flagging on the check alone flags exactly the (v, s) the atomic's old
+// marks v (pk_mark).  Flagging on the check alone flags exactly the (v, s) the atomic's old
 // value would: when alt < cur but a concurrent atomicMin has already stored less, that writer
 // passed its own check in this same launch and flags (v, s) itself (every earlier store is
 // visible to the check).  So no lane waits for an atomic's return before the next step.
@@ -1422,7 +1434,7 @@ __device__ __forceinline__ void pk_relax_steps(const DevState &st, const bool *o
     }
 #pragma unroll
     for (int k = 0; k < UNR; ++k)
-        if (prev[k] == 0) atomicOr(&st.bm[0][tv[k] >> 5], 1u << (tv[k] & 31));
+        if (prev[k] == 0) st_coherent_b(pk_mark(st, tv[k]), 1);
 }
 
 // Items of one queued vertex u -- edges [e0, e1) x the P pending sources of M -- on `stride`
@@ -1727,7 +1739,7 @@ __device__ __forceinline__ void pk_relax_listed(const DevState &st, int u, unsig
         }
 #pragma unroll
         for (int k = 0; k < UNR; ++k)
-            if (prev[k] == 0) atomicOr(&st.bm[0][tv[k] >> 5], 1u << (tv[k] & 31));
+            if (prev[k] == 0) st_coherent_b(pk_mark(st, tv[k]), 1);
     }
 }
 
@@ -1885,30 +1897,28 @@ __device__ __forceinline__ unsigned pk_take(const DevState &st, int4 x, int q, u
 
 // Vertices with pending sources -> class-segmented queue with their source masks.  With a
 // priority window (T < NO_WINDOW) only the (vertex, source) pairs with dist < T are queued; the
-// others move from mflag[v] to deferred[v] (and v from bm[0] to bm[1]).  A deferred pair is below
+// others move from mflag[v] to deferred[v].  A deferred pair is below
 // the window only after a relaxation, which flags it again, or after the window has risen: so the
 // passes of one window look at the flagged pairs alone, and only a `full` pass, once before the
 // window rises (the deferred pairs' count and least distance go to the pass's deferral sums) and
 // once after, looks at every deferred one.  Kept flagged and re-read in every pass by a lane per
 // row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid 16.5 -> 7.4 ms
-// of it per solve (13.4 with a lane per row still), the expansions 16.0 -> 18.4 (a deferred vertex that
-// is flagged again sets its frontier bit again), the solve 33.2 -> 26.5 ms.
+// of it per solve (13.4 with a lane per row still), the solve 33.2 -> 26.5 ms.
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
                                               int T, bool full, int slot) {
     __shared__ int s_wc[WAVES][NCLS];
     static_assert(WAVES * NCLS <= WG, "cleared by one store each");
     __shared__ int s_dc, s_dm, s_pairs;
-    unsigned *bm = st.bm[0];
     if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; s_pairs = 0; }
     if (threadIdx.x < WAVES * NCLS) s_wc[0][threadIdx.x] = 0;
     __syncthreads();
     int pairs = 0, my_dc = 0, my_dm = NO_WINDOW;
     const bool windowed = T != NO_WINDOW || full;
-    // The words are scanned as compaction_impl does (a thread per word took 0.24 ms where this takes
+    // The marks are scanned as compaction_impl scans its words (a thread per word took 0.24 ms where this takes
     // 0.1, R-MAT s24, 16 sources, 8 M vertices queued); then the hubs held for one pass (hold_cls) or
     // the vertices without a pair below the window leave the list.
     __shared__ unsigned short s_list[WAVES][64 * 32];
-    __shared__ unsigned s_held[WG];  // per word of the wave: held or deferred vertices, and whether it has hubs
+    __shared__ unsigned s_held[WG];  // per word of the wave: held vertices, and whether it has hubs
     __shared__ int s_heavy[WG];
     const int lane = lane_id(), half = lane & 31;
     unsigned short *list = s_list[threadIdx.x >> 6];
@@ -1918,14 +1928,12 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
         const long long w0 = wb + (threadIdx.x >> 6) * wt;
         const bool in = lane < wt && w0 + lane < st.nwords;
-        const unsigned flagged = in ? ld_coherent_u(bm + w0 + lane) : 0u;
-        const unsigned later = windowed && in ? ld_coherent_u(st.bm[1] + w0 + lane) : 0u;
-        const unsigned word = full ? flagged | later : flagged;
-        unsigned long long nz = __ballot(word != 0);
+        const unsigned marks = in ? ld_coherent_u(st.bm[0] + w0 + lane) : 0u;  // of 32 vertices
+        unsigned long long nz = __ballot(in && (full || marks));
         int n = 0;
         while (nz) {
             int idx[COMPACT_UNR], c[COMPACT_UNR];
-            unsigned x[COMPACT_UNR];
+            unsigned f[COMPACT_UNR];
 #pragma unroll
             for (int k = 0; k < COMPACT_UNR; ++k) {
                 const int ia = __ffsll((long long)nz) - 1;
@@ -1933,11 +1941,16 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 const int ib = __ffsll((long long)nz) - 1;
                 nz &= nz - 1;
                 idx[k] = lane < 32 ? ia : ib;  // -1: none left
-                x[k] = __shfl(word, idx[k] < 0 ? 0 : idx[k]);
-                if (idx[k] < 0) x[k] = 0u;
-                // no out-edges (class 0): dropped (mflag stays set, so it is not flagged again)
-                c[k] = (x[k] >> half) & 1u ? (int)st.cls[(w0 + idx[k]) * 32 + half] : 0;
+                const long long v = (w0 + idx[k]) * 32 + half;
+                const unsigned mk = full ? ~0u : __shfl(marks, idx[k] < 0 ? 0 : idx[k]);
+                const bool ok = idx[k] >= 0 && (mk >> (half & 24) & 0xFFu) && v < st.nslots;
+                c[k] = ok ? (int)st.cls[v] : 0;
+                f[k] = ok ? ld_coherent_u(st.mflag + v) : 0u;
+                if (full && ok) f[k] |= ld_coherent_u(st.deferred + v);
             }
+            // no out-edges (class 0): dropped
+#pragma unroll
+            for (int k = 0; k < COMPACT_UNR; ++k) c[k] = f[k] ? c[k] : 0;
 #pragma unroll
             for (int k = 0; k < COMPACT_UNR; ++k) {
                 const unsigned long long m = __ballot(c[k] != 0);
@@ -1945,14 +1958,11 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 n += __popcll(m);
             }
         }
-        unsigned stay = 0;  // flags of this lane's word that stay
+        unsigned stay = 0;  // vertices of this lane's word that stay pending
         if (windowed) {
             // 8 lanes per vertex read its row; a vertex with a pair below the window keeps its
             // mask for the queue in mflag, the others leave the list
             constexpr int WIN_UNR = 4;
-            unsigned *held_w = s_held + (threadIdx.x & ~63);
-            s_held[threadIdx.x] = 0u;
-            __builtin_amdgcn_wave_barrier();
             const int g = lane >> 3, q = lane & 7;
             int left = 0;
             for (int base = 0; base < n; base += 8 * WIN_UNR) {
@@ -1964,9 +1974,8 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     const int i = base + 8 * k + g;
                     e[k] = i < n ? (int)list[i] : 0;  // class 0: none
                     const long long v = w0 * 32 + (e[k] & 2047);
-                    const unsigned lw = __shfl(later, (e[k] & 2047) >> 5);
                     f[k] = e[k] ? ld_coherent_u(st.mflag + v) : 0u;
-                    old[k] = e[k] && ((lw >> (e[k] & 31)) & 1u) ? ld_coherent_u(st.deferred + v) : 0u;
+                    old[k] = e[k] ? ld_coherent_u(st.deferred + v) : 0u;
                     x[k] = pk_row_part(st, v, q, e[k] != 0);
                 }
                 __builtin_amdgcn_wave_barrier();
@@ -1980,12 +1989,9 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     if (q == 0 && e[k]) {
                         if (f[k] != t) st_coherent_u(st.mflag + v, t);
                         if (rest != old[k]) st_coherent_u(st.deferred + v, rest);
-                        if (rest) {
-                            atomicOr(&held_w[(e[k] & 2047) >> 5], 1u << (e[k] & 31));
-                            if (full) {
-                                my_dc += __popc(rest);
-                                my_dm = dmin < my_dm ? dmin : my_dm;
-                            }
+                        if (full && rest) {
+                            my_dc += __popc(rest);
+                            my_dm = dmin < my_dm ? dmin : my_dm;
                         }
                     }
                     const unsigned long long m = __ballot(take);
@@ -1995,8 +2001,6 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
             }
             n = left;
             __builtin_amdgcn_wave_barrier();
-            const unsigned now = (later & ~word) | s_held[threadIdx.x];
-            if (now != later) st_coherent_u(st.bm[1] + w0 + lane, now);
         }
         if (st.hold_cls) {
             // hubs that more sources are on their way to wait one pass and keep their flag; a held
@@ -2040,7 +2044,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
             stay = s_held[threadIdx.x];
             if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
         }
-        if (flagged != stay) st_coherent_u(bm + w0 + lane, stay);
+        if (marks && !stay) st_coherent_u(st.bm[0] + w0 + lane, 0u);
         if (!__syncthreads_or(n)) continue;  // s_wc is clear, nothing was counted
         for (int i = lane; i < n; i += 64) atomicAdd(&wc[list[i] >> 11], 1);
         reserve_classes(s_wc, cnt_out);
@@ -2287,7 +2291,7 @@ __global__ void k_pk_init_sources(DevState st, const int *srcs, int nsrc, int T0
         st.dist[((long long)v << st.kshift) + i] = 0;
         if (st.cls[v] == 0) continue;
         atomicOr(&st.mflag[v], 1u << i);
-        atomicOr(&st.bm[0][v >> 5], 1u << (v & 31));
+        st_coherent_b(pk_mark(st, v), 1);
     }
 }
 
@@ -2723,8 +2727,11 @@ hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch,
 
 hipError_t launch_compact(const DevState &st, int it_off, bool batch, int wgs, hipStream_t s) {
     (void)batch;
-    long long need = (st.nwords + WG - 1) / WG;
-    int g = (int)(need < wgs ? (need < 1 ? 1 : need) : wgs);
+    // a workgroup per tile of 8 words per wavefront, up to the 512 that compact_words has in view (a
+    // workgroup per 8,192 vertices left 8 of them on 65,536, each with 8 tiles in turn: 4 sources of
+    // R-MAT s16 1.04 -> 0.91 ms, of grid 256^2 1.91 -> 1.41, one of ER 65,536 0.79 -> 0.66)
+    const long long need = (st.nwords + WAVES * 8 - 1) / (WAVES * 8);
+    const int g = (int)std::min<long long>(std::max<long long>(need, 1), std::min(wgs, 512));
     if (st.kshift >= 0) {
         hipLaunchKernelGGL(k_pk_compact, dim3(g), dim3(WG), 0, s, st, it_off);
         if (st.bound) hipLaunchKernelGGL(k_pk_bounds, dim3(wgs), dim3(WG), 0, s, st);
@@ -2739,7 +2746,7 @@ hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, i
     hipError_t e;
     if ((e = launch_fill_i32(st.dist, st.nslots << st.kshift, st.inf, s)) != hipSuccess) return e;
     if ((e = launch_fill_u32(st.bm[0], st.nwords, 0u, s)) != hipSuccess) return e;
-    if ((st.hold_cls || st.deferred) && (e = launch_fill_u32(st.bm[1], st.nwords, 0u, s)) != hipSuccess) return e;
+    if (st.hold_cls && (e = launch_fill_u32(st.bm[1], st.nwords, 0u, s)) != hipSuccess) return e;
     if ((e = launch_fill_u32(st.mflag, st.nslots, 0u, s)) != hipSuccess) return e;
     if (st.deferred && (e = launch_fill_u32(st.deferred, st.nslots, 0u, s)) != hipSuccess) return e;
     if (st.bound && (e = launch_fill_u32((unsigned *)st.bound, (st.nslots + 3) / 4, ~0u, s)) != hipSuccess) return e;
