@@ -160,3 +160,27 @@ def test_packed_window_moves_deferred_pairs(npa, ctx, orc, kind, nsrc):
                 assert np.array_equal(b.get(i), ref[i]), (dr, delta, i)
     b.free()
     G.free()
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 6, 7, 8, 1027, 4099, 70001])
+def test_distance_range_is_checked_at_every_index(npa, ctx, n):
+    """src -> a -> b with 2^29 on both edges: b's distance would be 2^30, which is refused wherever a
+    (the only finite distance near the limit) lies in the buffer, also one that is not aligned to 16
+    bytes; one less and it is accepted."""
+    half = 1 << 29
+    buf = npa.DeviceBuffer(ctx, n + 3)
+    for a in sorted({0, 1, 2, 3, n // 2, n - 3, n - 2, n - 1} & set(range(n))):
+        src, b = [v for v in (0, 1, n - 1, n // 2) if v != a][:2]
+        for last, fits in ((half, False), (half - 1, True)):
+            G = npa.Graph.from_csr(ctx, *_csr([src, a], [a, b], [half, last], n))
+            want = np.full(n, npa.INF, np.int32)
+            want[src], want[a], want[b] = 0, half, half + last
+            for off in range(4):
+                if fits:
+                    ctx.sssp_device(G, src, buf.ptr + 4 * off, npa.Sched(level=1))
+                    assert np.array_equal(buf.to_host()[off:off + n], want), (a, off)
+                else:
+                    with pytest.raises(npa.NpError):
+                        ctx.sssp_device(G, src, buf.ptr + 4 * off, npa.Sched(level=1))
+            G.free()
+    buf.free()
