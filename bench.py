@@ -266,7 +266,7 @@ def bc_bench(npa, ctx, args):
                    "levels": int(st.iterations), "device_ms": round(dev_ms, 3)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "k_bc_compact+k_bc_owner+k_bc_expand+k_bc_accum (host loop)",
+                     "kernel": "k_bc_compact+k_bc_expand+k_bc_finish (host loop)",
                      "bytes_per_launch": b_alg},
         "cpu_baseline": cpu, "exact": exact,
     }
@@ -380,8 +380,7 @@ def pr_bench(npa, ctx, args):
                    "iterations": it, "device_ms": round(dev_ms, 3)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": measured_traffic("pagerank"),
-                     "kernel": "k_pr_gate+k_pr_contrib+k_pr_pull_light+k_pr_pull_wave+k_pr_pull_huge "
-                               "(8 iterations per readback)",
+                     "kernel": "k_pr_pull (one launch per iteration, 8 iterations per readback)",
                      "bytes_per_launch": b_alg},
         "cpu_baseline": cpu, "exact": exact,
     }
