@@ -193,14 +193,17 @@ __global__ __launch_bounds__(256) void k_bc_expand(BcDev b, BcLevel *lv, const i
             double x = 0.0;
             for (int i = lane >> lp; i < cnt; i += step * BC_UNR) {
                 double f[BC_UNR];
+                bool on[BC_UNR];
 #pragma unroll
                 for (int k = 0; k < BC_UNR; ++k) {
                     const int ik = i + k * step;
                     const int2 e = edge[ik < cnt ? ik : i];
-                    f[k] = ik < cnt && ((unsigned)e.y & bit) ? b.sig[((long long)e.x << b.ks) + src] : 0.0;
+                    on[k] = ik < cnt && ((unsigned)e.y & bit);
+                    f[k] = on[k] ? b.sig[((long long)e.x << b.ks) + src] : 0.0;
                 }
+                // not sv * 0 for the others: a path count past float64 is infinite
 #pragma unroll
-                for (int k = 0; k < BC_UNR; ++k) x += sv * f[k];
+                for (int k = 0; k < BC_UNR; ++k) x += on[k] ? sv * f[k] : 0.0;
             }
             for (int off = 32; off >= (1 << lp); off >>= 1) x += __shfl_xor(x, off);
             const bool whole = r.w <= BC_CHUNK && r.z == b.row[v];  // the row's only chunk

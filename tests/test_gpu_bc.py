@@ -94,3 +94,26 @@ def test_bc_rows_at_chunk_edges(npa, ctx, orc, nsrc):
     ref = orc.bc(row, col, srcs)
     assert np.allclose(bc, ref, rtol=RTOL, atol=ATOL), float(np.max(np.abs(bc - ref)))
     G.free()
+
+
+def test_bc_overflowed_path_count_stays_with_its_source(npa, ctx, orc):
+    """1,024 diamonds in a row give v 2^1024 shortest paths from A, past float64, and one from B along a
+    path of the same length; v's only successor is one step from A.  So v has no successor for A, its
+    infinite count multiplies nothing, and every dependency is finite."""
+    k = 1024
+    a = 3 * np.arange(k + 1)                       # a[0] = A, a[k] = v; the diamond's sides follow each a
+    v, w, b = int(a[k]), int(a[k]) + 1, int(a[k]) + 2
+    side = [(a[:-1], a[:-1] + 1), (a[:-1], a[:-1] + 2), (a[:-1] + 1, a[1:]), (a[:-1] + 2, a[1:])]
+    chain = np.concatenate([b + np.arange(2 * k), [v]])     # B and 2 k - 1 more, then v
+    src = np.concatenate([s for s, _ in side] + [chain[:-1], [v, a[0]]])
+    dst = np.concatenate([d for _, d in side] + [chain[1:], [w, w]])
+    order = np.argsort(src, kind="stable")
+    row = np.zeros(b + 2 * k + 1, np.int64)
+    np.add.at(row, src + 1, 1)
+    row, col = np.cumsum(row).astype(np.int32), dst[order].astype(np.int32)
+    G = _graph(npa, ctx, row, col)
+    ref = orc.bc(row, col, [0, b])
+    assert np.isfinite(ref).all()
+    bc, _ = ctx.bc(G, [0, b])
+    assert np.allclose(bc, ref, rtol=RTOL, atol=ATOL)
+    G.free()
