@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_bc_expand(BcDev b, BcLevel *lv, const i
         const unsigned long long act = __ballot(pm != 0);
         const int cnt = __popcll(act);
         if (pm) edge[__popcll(act & ((1ull << lane) - 1))] = int2{w, (int)pm};
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         const int step = 64 >> lp;  // groups in the wave
         if (FWD) {
             for (int i = lane >> lp; i < cnt; i += step) {
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void k_bc_expand(BcDev b, BcLevel *lv, const i
                 atomicAdd(&b.del[own], x);
             }
         }
-        __builtin_amdgcn_wave_barrier();  // the next chunk's edges overwrite the list
+        wave_lds_order();  // the next chunk's edges overwrite the list
     }
 }
 

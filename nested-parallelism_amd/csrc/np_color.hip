@@ -104,11 +104,6 @@ __device__ __forceinline__ int col_load(const int *p) {
 __device__ __forceinline__ void col_store(int *p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// LDS of one wavefront: its lanes run in step, so only the compiler has to keep the order.
-__device__ __forceinline__ void col_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
 
 // The solve: wavefronts take tickets until none is left (ntick = the number of tickets, on the
 // device).  What bounds it is the longest chain of dependencies (about as many hops as colors),
@@ -137,7 +132,7 @@ __global__ __launch_bounds__(256) void k_color_solve(const int *row, const int *
             w.color[lane] = 0;
         }
         if (lane == 0) w.row[nv] = row[v0 + nv];
-        col_order();
+        wave_lds_order();
         const int e0 = w.row[0] + chunk * COL_EDGES;
         const int left = w.row[nv] - e0;                      // edges from this ticket's first on
         const int ne = left < COL_EDGES ? left : COL_EDGES;
@@ -167,7 +162,7 @@ __global__ __launch_bounds__(256) void k_color_solve(const int *row, const int *
         bool fresh = false;      // a vertex of the ticket got its color in the last round
         unsigned long long spins = 0;
         for (;;) {
-            col_order();
+            wave_lds_order();
             const bool ready = mine && next == t && w.wait[lane] == 0;
             if (ready) {
                 const int cv = w.best[lane] + 1;
@@ -182,7 +177,7 @@ __global__ __launch_bounds__(256) void k_color_solve(const int *row, const int *
             }
             if (__ballot(mine) == 0) break;
             fresh = __ballot(ready) != 0;
-            col_order();
+            wave_lds_order();
             // a color of the ticket's own vertices settles its successors from LDS; only without
             // one are the other wavefronts' colors read again
 #pragma unroll
@@ -213,7 +208,7 @@ __global__ __launch_bounds__(256) void k_color_solve(const int *row, const int *
                 }
             }
         }
-        col_order();
+        wave_lds_order();
     }
     for (int o = 32; o > 0; o >>= 1) { const int x = __shfl_xor(top, o); top = x > top ? x : top; }
     if (lane == 0 && top) atomicMax(&ctl[1], top);

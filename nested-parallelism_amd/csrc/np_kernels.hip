@@ -105,7 +105,7 @@ __device__ __forceinline__ void decode(const DevState &st, int slot, int &B, int
 // the next barrier, so the grid always drains.
 __device__ bool grid_sync(Ctrl *ctrl, unsigned nblocks, unsigned long long &gen) {
     __shared__ int s_ok;
-    __builtin_amdgcn_s_waitcnt(0);
+    stores_done();
     __syncthreads();
     if (threadIdx.x == 0) {
         gen += 1;
@@ -810,7 +810,7 @@ __device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTab
             sb.wsum[wave] = incl;
             atomicAdd(&sb.live, __popcll(m0) + __popcll(m1));
         }
-        __builtin_amdgcn_s_waitcnt(0);  // the cleared flags are in memory
+        stores_done();  // the cleared flags are in memory
         __syncthreads();
         int before = 0, edges = 0;
 #pragma unroll
@@ -869,7 +869,7 @@ __device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTab
                 if (at < SOLO_V) nxt[at] = tv[k];
             }
         }
-        __builtin_amdgcn_s_waitcnt(0);  // the distances are in memory
+        stores_done();  // the distances are in memory
         __syncthreads();
         n = sb.next;
         if (n > SOLO_V) break;  // the bitmap has them all
@@ -1581,7 +1581,7 @@ __device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, const
     int have = 0;
     for (int tb = e0; tb < e1; tb += tile) {
         int nt = e1 - tb < tile ? e1 - tb : tile;
-        __builtin_amdgcn_wave_barrier();       // the previous tile's reads come first
+        wave_lds_order();       // the previous tile's reads come first
         int c[PK_TILE / 64], wv[PK_TILE / 64];
 #pragma unroll
         for (int r = 0; r < PK_TILE / 64; ++r) {
@@ -1615,7 +1615,7 @@ __device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, const
                 if (!UNIT) tw[lane + 64 * r] = wv[r];
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         for (int e = eo; __ballot(on && e < nt) != 0; e += span) {
             int tv[UNR], alt[UNR], cur[UNR];
             bool ok[UNR];
@@ -1776,7 +1776,7 @@ __device__ __forceinline__ void pk_edge_tile(const DevState &st, const PkFilt &p
         }
 #pragma unroll
         for (int k = 0; k < UNR; ++k) b[k] = c[k] >= 0 ? (int)st.bound[c[k]] : 0;
-        __builtin_amdgcn_wave_barrier();  // the list's previous reads come first
+        wave_lds_order();  // the list's previous reads come first
 #pragma unroll
         for (int k = 0; k < UNR; ++k) {
             const int t = __shfl(thr, o[k]);
@@ -1790,7 +1790,7 @@ __device__ __forceinline__ void pk_edge_tile(const DevState &st, const PkFilt &p
             }
             have += __popcll(m);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_order();
         if (have > PK_SLICE - UNR * 64 || base + UNR * 64 >= total) {
             pk_relax_listed(st, u, M, tcol, tw, town, have);
             have = 0;
@@ -1958,6 +1958,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 n += __popcll(m);
             }
         }
+        wave_lds_order();   // the list, written by all lanes, is read from here on
         unsigned stay = 0;  // vertices of this lane's word that stay pending
         if (windowed) {
             // 8 lanes per vertex read its row; a vertex with a pair below the window keeps its
@@ -1978,7 +1979,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     old[k] = e[k] ? ld_coherent_u(st.deferred + v) : 0u;
                     x[k] = pk_row_part(st, v, q, e[k] != 0);
                 }
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_order();
 #pragma unroll
                 for (int k = 0; k < WIN_UNR; ++k) {
                     const long long v = w0 * 32 + (e[k] & 2047);
@@ -2000,7 +2001,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 }
             }
             n = left;
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
         }
         if (st.hold_cls) {
             // hubs that more sources are on their way to wait one pass and keep their flag; a held
@@ -2011,7 +2012,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
             s_heavy[threadIdx.x] = 0;
             unsigned *held_w = s_held + (threadIdx.x & ~63);
             int *heavy_w = s_heavy + (threadIdx.x & ~63);
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
             int left = 0;
             for (int base = 0; base < n; base += 64 * COMPACT_UNR) {
                 int e[COMPACT_UNR], reached[COMPACT_UNR];
@@ -2024,7 +2025,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     hw[k] = heavy ? ld_coherent_u(st.bm[1] + w0 + ((e[k] & 2047) >> 5)) : 0u;
                     reached[k] = heavy ? pk_reached(st, w0 * 32 + (e[k] & 2047)) : st.hold_min;
                 }
-                __builtin_amdgcn_wave_barrier();
+                wave_lds_order();
 #pragma unroll
                 for (int k = 0; k < COMPACT_UNR; ++k) {
                     const int wi = (e[k] & 2047) >> 5, bit = e[k] & 31;
@@ -2040,7 +2041,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 }
             }
             n = left;
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_order();
             stay = s_held[threadIdx.x];
             if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
         }

@@ -249,10 +249,11 @@ __global__ __launch_bounds__(256) void k_pr_pull(int i, PrSums *ps, RowBins rb, 
             if (lane == 0) {
                 // the partial sum is in memory before the count tells so
                 __hip_atomic_store(rb.part + o, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __builtin_amdgcn_s_waitcnt(0);
+                stores_done();
                 last = atomicSub(&rb.hleft[h], 1) == 1;
             }
             if (__builtin_amdgcn_readfirstlane(last)) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // no read of part[] before the count
                 const int k = (int)(((long long)end - irow[v] + PR_CHUNK - 1) / PR_CHUNK);
                 double t = 0.0;  // lane by lane and then the butterfly: the same order every time
                 for (int j = lane; j < k; j += 64)
