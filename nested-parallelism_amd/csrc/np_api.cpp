@@ -344,7 +344,7 @@ static SchedDev make_schedd(np_ctx *c, const np_sched &s, int n_feat) {
 static constexpr long long SMALL_EDGES = 4ll << 20, LARGE_EDGES = 32ll << 20;
 static int persistent_wgs(np_ctx *c, const np_sched &s, const SchedDev &sd, bool batch, bool unit, bool packed,
                           long long edges) {
-    int occ = persistent_max_wgs_per_cu(batch, unit, sd.push != 0, packed, sd.solo != 0);
+    int occ = persistent_max_wgs_per_cu(batch, unit, sd.push != 0, packed, sd.solo != 0, sd.delta > 0);
     if (occ < 1) occ = 1;
     const int fit = packed || edges > LARGE_EDGES ? occ : edges > SMALL_EDGES ? std::min(2, occ) : 1;
     int per = s.wgs_per_cu > 0 ? std::min(s.wgs_per_cu, occ) : fit;
@@ -888,7 +888,7 @@ int np_destroy(np_ctx *c) {
 int np_device_info(np_ctx *c, int32_t *num_cus, int32_t *max_wgs_per_cu) {
     if (!c) { set_error("null context"); return NP_ERR_ARG; }
     if (num_cus) *num_cus = c->num_cus;
-    if (max_wgs_per_cu) *max_wgs_per_cu = persistent_max_wgs_per_cu(false, false, false, false, false);
+    if (max_wgs_per_cu) *max_wgs_per_cu = persistent_max_wgs_per_cu(false, false, false, false, false, false);
     return NP_OK;
 }
 
@@ -2248,7 +2248,7 @@ int np_autotune(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, const
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;  // the search is over the consolidation bins
-    int occ = persistent_max_wgs_per_cu(false, false, b0.frontier == NP_FRONTIER_PUSH, false, g->m <= LARGE_EDGES);
+    int occ = persistent_max_wgs_per_cu(false, false, b0.frontier == NP_FRONTIER_PUSH, false, g->m <= LARGE_EDGES, false);
     std::vector<int> wgs_opts = {0};
     if (occ > 2) wgs_opts.push_back(2);
     if (occ > 4) wgs_opts.push_back(4);
@@ -2310,7 +2310,7 @@ int np_batch_autotune(np_ctx *c, np_batch *b, const np_sched *base, np_sched *be
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;
-    int occ = persistent_max_wgs_per_cu(true, b->unit != 0, false, !b->packs.empty(), b->sp.edges <= LARGE_EDGES);
+    int occ = persistent_max_wgs_per_cu(true, b->unit != 0, false, !b->packs.empty(), b->sp.edges <= LARGE_EDGES, false);
     std::vector<int> wgs_opts = {0};
     if (occ > 2) wgs_opts.push_back(2);
     if (occ > 4) wgs_opts.push_back(4);

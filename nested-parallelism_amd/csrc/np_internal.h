@@ -162,7 +162,7 @@ hipError_t launch_unpermute_parts(const int *dist, const int *lut, const ConcatO
 // with kshift >= 0 runs the source-packed kernels (here and in compact/expand).
 hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch, bool unit,
                              int wgs, hipStream_t s);
-int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo);
+int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo, bool window);
 
 // Host-loop / graph drive, one iteration = [compact] + decide + expand.
 hipError_t launch_compact(const DevState &st, int it_off, bool batch, int wgs, hipStream_t s);

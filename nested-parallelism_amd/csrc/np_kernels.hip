@@ -33,7 +33,19 @@ static constexpr unsigned long long SPIN_LIMIT = 1ull << 24;
 // ------------------------------------------------------------------------------------
 // small helpers
 // ------------------------------------------------------------------------------------
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+// threadIdx.x for one phase of a persistent kernel.  What a phase derives from it is the same in every
+// iteration, so the compiler would compute it once, before the loop, and hold it in registers through
+// all other phases; behind this it is computed again where it is used.  k_persistent 130 (with the
+// small-frontier path 150) -> 93 (110) VGPRs, 3 -> 5 (4) workgroups per CU; k_pk_persistent 156 -> 120,
+// 3 -> 4; k_pk_expand (64 at most) no longer spills.  A limit on the registers alone (waves_per_eu)
+// gave the same count and lost it again: every wavefront had fewer loads in flight.
+__device__ __forceinline__ int phase_tid() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+__device__ __forceinline__ int lane_id() { return phase_tid() & 63; }
+__device__ __forceinline__ unsigned long long lanes_below(int lane) { return (1ull << lane) - 1; }
 
 // Data that one workgroup writes and another reads inside a persistent launch (queue
 // entries, bitmap words, counters, distances) only moves through device-coherent
@@ -415,6 +427,7 @@ template <bool BATCH, bool UNIT, bool PUSH, bool GUARD>
 __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, ItemTables &tb) {
     const long long G = tb.pre[0][NCLS], K = tb.pre[1][NCLS], W = tb.pre[2][NCLS],
                     T = tb.pre[3][NCLS];
+    const int tid = phase_tid(), lane = tid & 63;
     // workgroup items: the whole workgroup strides one vertex's edges
     for (long long k = blockIdx.x; k < K; k += gridDim.x) {
         int c = find_class(tb.pre[1], k);
@@ -427,15 +440,15 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
         int v = slot - B;
         int s = st.row[VB + v], e = st.row[VB + v + 1];
         int du = ld_coherent(st.dist + slot);
-        if (PUSH && j == 0 && threadIdx.x == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
+        if (PUSH && j == 0 && tid == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
         if (j > (e - s - 1) >> WG_CHUNK_SHIFT) continue;  // a class's rows have half to all of its chunks
         int e0 = s + (j << WG_CHUNK_SHIFT);
         int e1 = e - e0 > (1 << WG_CHUNK_SHIFT) ? e0 + (1 << WG_CHUNK_SHIFT) : e;
-        relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, threadIdx.x, WG);
+        relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, tid, WG);
     }
     // wavefront-granular items: grid chunks, wavefront items, lane tiles, round-robin
     const long long NW = (long long)gridDim.x * WAVES;
-    const long long gw = (long long)blockIdx.x * WAVES + (threadIdx.x >> 6);
+    const long long gw = (long long)blockIdx.x * WAVES + (tid >> 6);
     const long long U = G + W + T;
     for (long long u = gw; u < U; u += NW) {
         if (u < G) {
@@ -452,10 +465,10 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
             int e0 = s + (j << GRID_CHUNK_SHIFT);
             int e1 = e0 + (1 << GRID_CHUNK_SHIFT);
             if (e1 > e) e1 = e;
-            if (PUSH && j == 0 && lane_id() == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
+            if (PUSH && j == 0 && lane == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
             if (e0 < e1) {
                 int du = ld_coherent(st.dist + slot);
-                relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, lane_id(), 64);
+                relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, lane, 64);
             }
         } else if (u < G + W) {
             long long i = u - G;
@@ -467,8 +480,8 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
             int v = slot - B;
             int e0 = st.row[VB + v], e1 = st.row[VB + v + 1];
             int du = ld_coherent(st.dist + slot);
-            if (PUSH && lane_id() == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
-            relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, lane_id(), 64);
+            if (PUSH && lane == 0) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
+            relax_range<UNIT, PUSH, GUARD>(st, pc, B, e0, e1, du, lane, 64);
         } else {
             long long t = u - G - W;
             int c = find_class(tb.pre[3], t);
@@ -547,7 +560,8 @@ __device__ __forceinline__ void deferred_clear(Ctrl *ctrl, int slot) {
 }
 
 // A wave loads up to 64 words at once and takes the nonzero ones two at a time, a lane per vertex,
-// COMPACT_UNR pairs in flight; the vertices to queue gather in LDS as (offset, class).  A thread
+// COMPACT_UNR pairs in flight (one fewer in the persistent kernel without the small-frontier path, which
+// then fits 5 workgroups on a CU; grid 3200^2 on 3: 6.58 ms with 4 or 3, 6.72 with 2); the vertices to queue gather in LDS as (offset, class).  A thread
 // per word, walking its bits, left all but n / 8192 workgroups idle and waited for every class: one
 // solve on the persistent drive, ER 65,536 / 1 M 0.94 -> 0.82 ms, grid 2048^2 5.12 -> 4.13.
 constexpr int COMPACT_UNR = 4;
@@ -559,6 +573,7 @@ __device__ __forceinline__ int compact_words(long long nwords) {
     const long long share = (nwords + wgs * WAVES - 1) / (wgs * WAVES);
     return share < 8 ? 8 : share < 64 ? (int)share : 64;
 }
+template <int UNROLL>
 __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const unsigned char *cls, const int *seg_off,
                                                 long long nwords, int *cnt_out, int *q_out, const int *dist,
                                                 int T, int slot) {
@@ -566,23 +581,24 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
     __shared__ int s_lc[NCLS], s_lb[NCLS];
     __shared__ int s_dc, s_dm;
     static_assert(NCLS <= 32, "an entry holds 11 bits of offset and 5 of class");
-    if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; }
+    const int tid = phase_tid();
+    if (tid == 0) { s_dc = 0; s_dm = NO_WINDOW; }
     int my_dc = 0, my_dm = NO_WINDOW;
-    const int lane = lane_id(), half = lane & 31;
-    unsigned short *list = s_list[threadIdx.x >> 6];
+    const int lane = tid & 63, half = lane & 31;
+    unsigned short *list = s_list[tid >> 6];
     const int wt = compact_words(nwords);
     const long long tile = (long long)WAVES * wt;
     for (long long wb = (long long)blockIdx.x * tile; wb < nwords; wb += (long long)gridDim.x * tile) {
-        if (threadIdx.x < NCLS) s_lc[threadIdx.x] = 0;
-        const long long w0 = wb + (threadIdx.x >> 6) * wt;
+        if (tid < NCLS) s_lc[tid] = 0;
+        const long long w0 = wb + (tid >> 6) * wt;
         const unsigned word = lane < wt && w0 + lane < nwords ? ld_coherent_u(bm + w0 + lane) : 0u;
         unsigned long long nz = __ballot(word != 0);
         int n = 0;
         while (nz) {
-            int idx[COMPACT_UNR], c[COMPACT_UNR], d[COMPACT_UNR];
-            unsigned x[COMPACT_UNR];
+            int idx[UNROLL], c[UNROLL], d[UNROLL];
+            unsigned x[UNROLL];
 #pragma unroll
-            for (int k = 0; k < COMPACT_UNR; ++k) {
+            for (int k = 0; k < UNROLL; ++k) {
                 const int ia = __ffsll((long long)nz) - 1;
                 nz &= nz - 1;
                 const int ib = __ffsll((long long)nz) - 1;
@@ -594,16 +610,16 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
             }
             if (T != NO_WINDOW) {
 #pragma unroll
-                for (int k = 0; k < COMPACT_UNR; ++k)
+                for (int k = 0; k < UNROLL; ++k)
                     d[k] = c[k] ? ld_coherent(dist + (w0 + idx[k]) * 32 + half) : 0;
             }
 #pragma unroll
-            for (int k = 0; k < COMPACT_UNR; ++k) {
+            for (int k = 0; k < UNROLL; ++k) {
                 const bool defer = T != NO_WINDOW && c[k] && d[k] >= T;
                 if (defer) { my_dc++; my_dm = d[k] < my_dm ? d[k] : my_dm; }
                 const bool take = c[k] && !defer;  // no out-edges (class 0): dropped
                 const unsigned long long m = __ballot(take), kept = __ballot(defer);
-                if (take) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
+                if (take) list[n + __popcll(m & lanes_below(lane))] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
                 n += __popcll(m);
                 const unsigned nw = (unsigned)(kept >> (lane & 32));
                 if (half == 0 && nw != x[k]) st_coherent_u(bm + w0 + idx[k], nw);
@@ -612,10 +628,10 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
         if (!__syncthreads_or(n)) continue;  // s_lc is clear, nothing was counted
         for (int i = lane; i < n; i += 64) atomicAdd(&s_lc[list[i] >> 11], 1);
         __syncthreads();
-        if (threadIdx.x < NCLS) {
-            const int k = s_lc[threadIdx.x];
-            s_lb[threadIdx.x] = k ? seg_off[threadIdx.x] + atomicAdd(&cnt_out[threadIdx.x], k) : 0;
-            s_lc[threadIdx.x] = 0;
+        if (tid < NCLS) {
+            const int k = s_lc[tid];
+            s_lb[tid] = k ? seg_off[tid] + atomicAdd(&cnt_out[tid], k) : 0;
+            s_lc[tid] = 0;
         }
         __syncthreads();
         for (int i = lane; i < n; i += 64) {
@@ -713,9 +729,10 @@ __device__ __forceinline__ Cfg decide(const SchedDev &sp, const int *cnt, int it
     return decide_mlp(sp.mlp, sp.n_feat, sp.level, sp.klo, sp.khi, cnt, it);
 }
 
-__device__ __noinline__ void record_trace_rec(np_trace_rec *r, int it, int level, int klo, int khi, const int *cnt,
-                                              long long t0, Ctrl *ctrl) {
+__device__ __forceinline__ void record_trace_rec(np_trace_rec *r, int it, int level, int klo, int khi, const int *cnt,
+                                                 long long t0, Ctrl *ctrl) {
     long long pairs = 0;
+#pragma unroll 1
     for (int l = 0; l < BAR_LEAVES; ++l) pairs += __hip_atomic_load(&ctrl->leaf[l].pairs, __ATOMIC_RELAXED, NP_AGENT);
     r->pairs = pairs;
     r->edges = __hip_atomic_load(&ctrl->edges_total, __ATOMIC_RELAXED, NP_AGENT);
@@ -723,6 +740,7 @@ __device__ __noinline__ void record_trace_rec(np_trace_rec *r, int it, int level
     r->level = level;
     r->log2_t_lo = klo;
     r->log2_t_hi = khi;
+#pragma unroll 1
     for (int c = 0; c < NCLS; ++c) r->count[c] = cnt[c];
     r->t_begin = t0;
     r->t_end = t0;
@@ -771,7 +789,7 @@ __device__ __forceinline__ bool solo_fits(const ItemTables &tb, int total) {
 template <bool BATCH, bool UNIT>
 __device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTables &tb, const int *q, SoloBufs &sb,
                                                int total, int most) {
-    const int t = threadIdx.x, lane = lane_id(), wave = t >> 6;
+    const int t = phase_tid(), lane = t & 63, wave = t >> 6;
     unsigned *bm = st.bm[0];
     // the queue's class segments -> list[0]
     for (int i = t; i < total; i += WG) {
@@ -881,8 +899,8 @@ __device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTab
 // ------------------------------------------------------------------------------------
 // persistent drive
 // ------------------------------------------------------------------------------------
-// SOLO: small frontiers run on one workgroup; a graph of many edges goes without (its solve is a few
-// large iterations, and the registers cost it a workgroup per CU: R-MAT s22 4.26 -> 4.31 ms).
+// SOLO: small frontiers run on one workgroup.  The registers of that (117 against 95) cost a workgroup
+// per CU, 4 instead of 5, so graphs that want more go without (persistent_wgs in np_api.cpp).
 template <bool BATCH, bool UNIT, bool PUSH, bool SOLO>
 __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
     __shared__ ItemTables tb;
@@ -896,32 +914,33 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
     int pass = 0;
     int extra = 0;  // iterations run by one workgroup alone, beyond one per trip
     for (int it = 0;; ++it) {
+        const int tid = phase_tid();
         int *cnt_cur = st.cnt + (it % 3) * NCLS;
         int *cnt_zero = st.cnt + ((it + 2) % 3) * NCLS;
         int *q_cur = st.queue[it & 1];
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (blockIdx.x == 0 && tid == 0) {
             long long now = (long long)wall_clock64();
             if (it > 0 && sp.trace && it - 1 < sp.trace_cap) sp.trace[it - 1].t_end = now;
             t_prev = now;
         }
-        if (blockIdx.x == 0 && threadIdx.x < NCLS) st_coherent(cnt_zero + threadIdx.x, 0);
+        if (blockIdx.x == 0 && tid < NCLS) st_coherent(cnt_zero + tid, 0);
         for (;;) {
             const int slot = pass % 3;
             if (!PUSH) {
                 // the statistics slot of the next pass was last read before the previous barrier
                 if (blockIdx.x == 0 && T != NO_WINDOW) deferred_clear(ctrl, (pass + 1) % 3);
-                compaction_impl(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, cnt_cur, q_cur, st.dist, T, slot);
+                compaction_impl<SOLO ? COMPACT_UNR : COMPACT_UNR - 1>(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, cnt_cur, q_cur, st.dist, T, slot);
                 if (!grid_sync(ctrl, nb, gen)) return;
                 pass++;
             }
-            if (threadIdx.x < NCLS) {
-                tb.cnt[threadIdx.x] = ld_coherent(cnt_cur + threadIdx.x);
-                tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
+            if (tid < NCLS) {
+                tb.cnt[tid] = ld_coherent(cnt_cur + tid);
+                tb.seg[tid] = st.seg_off[tid];
             }
             __syncthreads();
-            if (threadIdx.x < 64) {
+            if (tid < 64) {
                 const long long tot = frontier_size(tb.cnt);
-                if (threadIdx.x == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
+                if (tid == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
             }
             __syncthreads();
             if (s_total > 0 || T == NO_WINDOW) break;
@@ -934,7 +953,7 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
         const int total = s_total;
         const int done_iters = it + extra;
         if (total == 0 || (sp.max_iters > 0 && done_iters >= sp.max_iters)) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
+            if (blockIdx.x == 0 && tid == 0) {
                 ctrl->iters = done_iters;
                 ctrl->done = total == 0 ? 1 : 0;
                 if (total != 0) ctrl->error = NP_ERR_NOT_CONVERGED;
@@ -947,15 +966,15 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
             if (sp.max_iters > 0 && sp.max_iters - done_iters < most) most = sp.max_iters - done_iters;
             if (blockIdx.x == 0) {
                 const int k = solo_iterations<BATCH, UNIT>(st, tb, q_cur, s_solo, total, most);
-                if (threadIdx.x == 0) st_coherent(&ctrl->solo, k);
+                if (tid == 0) st_coherent(&ctrl->solo, k);
             }
             if (!grid_sync(ctrl, nb, gen)) return;
             extra += ld_coherent(&ctrl->solo) - 1;
             continue;
         }
         Cfg cfg = decide(sp, tb.cnt, done_iters);
-        if (threadIdx.x < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (tid < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
+        if (blockIdx.x == 0 && tid == 0) {
             ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
         }
@@ -981,7 +1000,7 @@ __global__ __launch_bounds__(WG) void k_compact(DevState st, int it_off) {
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
     if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-    compaction_impl(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, st.cnt + (it % 3) * NCLS, st.queue[it & 1],
+    compaction_impl<COMPACT_UNR>(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, st.cnt + (it % 3) * NCLS, st.queue[it & 1],
                     st.dist, T, pass % 3);
 }
 
@@ -1408,7 +1427,7 @@ __device__ __forceinline__ unsigned char *pk_mark(const DevState &st, long long 
 // visible to the check).  So no lane waits for an atomic's return before the next step.
 // Vertices without out-edges are flagged too and dropped by the compaction.  Every lane of the
 // wavefront calls it together.
-__device__ __forceinline__ void pk_relax_steps(const DevState &st, const bool *ok, const int *tv, int s,
+__device__ __forceinline__ void pk_relax_steps(const DevState &st, int lane, const bool *ok, const int *tv, int s,
                                                const int *alt, const int *cur, int rs, bool last) {
 #pragma unroll
     for (int k = 0; k < UNR; ++k) {
@@ -1416,7 +1435,6 @@ __device__ __forceinline__ void pk_relax_steps(const DevState &st, const bool *o
             atomicMin(st.dist + (((unsigned)tv[k] << st.kshift) + (unsigned)s), alt[k]);
     }
     // every step's mflag OR is issued before any old value is tested: one wait for all UNR
-    const int lane = lane_id();
     unsigned prev[UNR];
 #pragma unroll
     for (int k = 0; k < UNR; ++k) {
@@ -1470,7 +1488,7 @@ __device__ __forceinline__ void pk_relax_vertex(const DevState &st, int u, unsig
 #pragma unroll
         for (int k = 0; k < UNR; ++k)
             cur[k] = ok[k] ? ld_coherent(st.dist + (((unsigned)tv[k] << ks) + (unsigned)s)) : 0;
-        pk_relax_steps(st, ok, tv, s, alt, cur, rs, last);
+        pk_relax_steps(st, lane, ok, tv, s, alt, cur, rs, last);
     }
 }
 
@@ -1629,7 +1647,7 @@ __device__ __forceinline__ void pk_relax_vertex_staged(const DevState &st, const
 #pragma unroll
             for (int k = 0; k < UNR; ++k)
                 cur[k] = ok[k] ? ld_coherent(st.dist + (((unsigned)tv[k] << ks) + (unsigned)s)) : 0;
-            pk_relax_steps(st, ok, tv, s, alt, cur, rs, last);
+            pk_relax_steps(st, lane, ok, tv, s, alt, cur, rs, last);
         }
     }
 }
@@ -1693,7 +1711,7 @@ __device__ __forceinline__ void pk_lane_tile(const DevState &st, const int *q, c
 #pragma unroll
             for (int kk = 0; kk < UNR; ++kk)
                 cur[kk] = ok[kk] ? ld_coherent(st.dist + (((unsigned)tv[kk] << ks) + (unsigned)s)) : 0;
-            pk_relax_steps(st, ok, tv, s, alt, cur, rs, last);
+            pk_relax_steps(st, lane, ok, tv, s, alt, cur, rs, last);
         }
     }
 }
@@ -1800,6 +1818,7 @@ __device__ __forceinline__ void pk_edge_tile(const DevState &st, const PkFilt &p
 template <bool UNIT, bool FILT>
 __device__ void pk_expansion(const DevState &st, const PkFilt &pf, const int *q, const unsigned *qm, ItemTables &tb,
                              int *tcol, int *tw, unsigned char *town) {
+    const int tid = phase_tid();
     const long long G = tb.pre[0][NCLS], K = tb.pre[1][NCLS], W = tb.pre[2][NCLS],
                     T = tb.pre[3][NCLS];
     for (long long k = blockIdx.x; k < K; k += gridDim.x) {
@@ -1807,10 +1826,10 @@ __device__ void pk_expansion(const DevState &st, const PkFilt &pf, const int *q,
         long long qi = tb.seg[c] + (k - tb.pre[1][c]);
         int u = ld_coherent(q + qi);
         unsigned M = ld_coherent_u(qm + qi);
-        pk_relax_vertex<UNIT>(st, u, M, st.row[u], st.row[u + 1], threadIdx.x, WG);
+        pk_relax_vertex<UNIT>(st, u, M, st.row[u], st.row[u + 1], tid, WG);
     }
     const long long NW = (long long)gridDim.x * WAVES;
-    const long long gw = (long long)blockIdx.x * WAVES + (threadIdx.x >> 6);
+    const long long gw = (long long)blockIdx.x * WAVES + (tid >> 6);
     const long long U = G + W + T;
     for (long long x = gw; x < U; x += NW) {
         if (x < G) {
@@ -1903,13 +1922,15 @@ __device__ __forceinline__ unsigned pk_take(const DevState &st, int4 x, int q, u
 // once after, looks at every deferred one.  Kept flagged and re-read in every pass by a lane per
 // row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid 16.5 -> 7.4 ms
 // of it per solve (13.4 with a lane per row still), the solve 33.2 -> 26.5 ms.
+template <int WIN_UNR>
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
                                               int T, bool full, int slot) {
     __shared__ int s_wc[WAVES][NCLS];
     static_assert(WAVES * NCLS <= WG, "cleared by one store each");
     __shared__ int s_dc, s_dm, s_pairs;
-    if (threadIdx.x == 0) { s_dc = 0; s_dm = NO_WINDOW; s_pairs = 0; }
-    if (threadIdx.x < WAVES * NCLS) s_wc[0][threadIdx.x] = 0;
+    const int tid = phase_tid();
+    if (tid == 0) { s_dc = 0; s_dm = NO_WINDOW; s_pairs = 0; }
+    if (tid < WAVES * NCLS) s_wc[0][tid] = 0;
     __syncthreads();
     int pairs = 0, my_dc = 0, my_dm = NO_WINDOW;
     const bool windowed = T != NO_WINDOW || full;
@@ -1919,13 +1940,13 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     __shared__ unsigned short s_list[WAVES][64 * 32];
     __shared__ unsigned s_held[WG];  // per word of the wave: held vertices, and whether it has hubs
     __shared__ int s_heavy[WG];
-    const int lane = lane_id(), half = lane & 31;
-    unsigned short *list = s_list[threadIdx.x >> 6];
-    int *wc = s_wc[threadIdx.x >> 6];
+    const int lane = tid & 63, half = lane & 31;
+    unsigned short *list = s_list[tid >> 6];
+    int *wc = s_wc[tid >> 6];
     const int wt = compact_words(st.nwords);
     const long long tile = (long long)WAVES * wt;
     for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
-        const long long w0 = wb + (threadIdx.x >> 6) * wt;
+        const long long w0 = wb + (tid >> 6) * wt;
         const bool in = lane < wt && w0 + lane < st.nwords;
         const unsigned marks = in ? ld_coherent_u(st.bm[0] + w0 + lane) : 0u;  // of 32 vertices
         unsigned long long nz = __ballot(in && (full || marks));
@@ -1953,7 +1974,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
 #pragma unroll
             for (int k = 0; k < COMPACT_UNR; ++k) {
                 const unsigned long long m = __ballot(c[k] != 0);
-                if (c[k]) list[n + __popcll(m & __lanemask_lt())] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
+                if (c[k]) list[n + __popcll(m & lanes_below(lane))] = (unsigned short)((c[k] << 11) | (idx[k] * 32 + half));
                 n += __popcll(m);
             }
         }
@@ -1962,7 +1983,6 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
         if (windowed) {
             // 8 lanes per vertex read its row; a vertex with a pair below the window keeps its
             // mask for the queue in mflag, the others leave the list
-            constexpr int WIN_UNR = 4;
             const int g = lane >> 3, q = lane & 7;
             int left = 0;
             for (int base = 0; base < n; base += 8 * WIN_UNR) {
@@ -1995,7 +2015,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                         }
                     }
                     const unsigned long long m = __ballot(take);
-                    if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
+                    if (take) list[left + __popcll(m & lanes_below(lane))] = (unsigned short)e[k];
                     left += __popcll(m);
                 }
             }
@@ -2007,10 +2027,10 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
             // vertex stays flagged, so the held bits are always a subset of the flags: they become
             // exactly this pass's held vertices (the ones held before are queued).  Renumbered hubs
             // share a wavefront's words, so their rows are read COMPACT_UNR x 64 at a time.
-            s_held[threadIdx.x] = 0u;
-            s_heavy[threadIdx.x] = 0;
-            unsigned *held_w = s_held + (threadIdx.x & ~63);
-            int *heavy_w = s_heavy + (threadIdx.x & ~63);
+            s_held[tid] = 0u;
+            s_heavy[tid] = 0;
+            unsigned *held_w = s_held + (tid & ~63);
+            int *heavy_w = s_heavy + (tid & ~63);
             wave_lds_order();
             int left = 0;
             for (int base = 0; base < n; base += 64 * COMPACT_UNR) {
@@ -2035,14 +2055,14 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     my_dc += held;
                     const bool take = e[k] != 0 && !held;
                     const unsigned long long m = __ballot(take);
-                    if (take) list[left + __popcll(m & __lanemask_lt())] = (unsigned short)e[k];
+                    if (take) list[left + __popcll(m & lanes_below(lane))] = (unsigned short)e[k];
                     left += __popcll(m);
                 }
             }
             n = left;
             wave_lds_order();
-            stay = s_held[threadIdx.x];
-            if (s_heavy[threadIdx.x]) st_coherent_u(st.bm[1] + w0 + lane, stay);
+            stay = s_held[tid];
+            if (s_heavy[tid]) st_coherent_u(st.bm[1] + w0 + lane, stay);
         }
         if (marks && !stay) st_coherent_u(st.bm[0] + w0 + lane, 0u);
         if (!__syncthreads_or(n)) continue;  // s_wc is clear, nothing was counted
@@ -2061,14 +2081,14 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
             pairs += __popc(t);
         }
         __syncthreads();
-        if (threadIdx.x < WAVES * NCLS) s_wc[0][threadIdx.x] = 0;  // the last loop counted in s_wc
+        if (tid < WAVES * NCLS) s_wc[0][tid] = 0;  // the last loop counted in s_wc
         __syncthreads();
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o);
-    if (lane_id() == 0 && pairs) atomicAdd(&s_pairs, pairs);
+    if (lane == 0 && pairs) atomicAdd(&s_pairs, pairs);
     __syncthreads();
-    if (threadIdx.x == 0 && s_pairs)
+    if (tid == 0 && s_pairs)
         atomicAdd((unsigned long long *)&st.ctrl->leaf[blockIdx.x % BAR_LEAVES].pairs, (unsigned long long)s_pairs);
     if (full || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
 }
@@ -2086,7 +2106,11 @@ __device__ __forceinline__ Cfg pk_cfg(Cfg c, bool filt) {
     return c;
 }
 
-template <bool UNIT>
+// WINDOW: a priority window is on.  Its compaction keeps 4 rows per lane group in flight, for which 3
+// workgroups fit on a CU; without a window 2 are enough for code that is not reached, and 4 fit (with 2
+// the window itself, 32 sources of a 2048^2 grid: 23.1 -> 24.0 ms; with 3 workgroups on a CU the packs
+// without one, 32 sources of R-MAT s20: 5.0 -> 6.1 ms).
+template <bool UNIT, bool WINDOW>
 __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) {
     __shared__ ItemTables tb;
     __shared__ int s_tcol[WAVES][PK_TILE], s_tw[WAVES][PK_TILE];
@@ -2100,31 +2124,32 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
     bool full = false;
     int pass = 0;
     for (int it = 0;; ++it) {
+        const int tid = phase_tid();
         int *cnt_cur = st.cnt + (it % 3) * NCLS;
         int *cnt_zero = st.cnt + ((it + 2) % 3) * NCLS;
         int *q_cur = st.queue[it & 1];
         unsigned *qm_cur = st.qmask[it & 1];
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (blockIdx.x == 0 && tid == 0) {
             long long now = (long long)wall_clock64();
             if (it > 0 && sp.trace && it - 1 < sp.trace_cap) sp.trace[it - 1].t_end = now;
             t_prev = now;
         }
-        if (blockIdx.x == 0 && threadIdx.x < NCLS) st_coherent(cnt_zero + threadIdx.x, 0);
+        if (blockIdx.x == 0 && tid < NCLS) st_coherent(cnt_zero + tid, 0);
         for (;;) {
             const int slot = pass % 3;
             // the statistics slot of the next pass was last read before the previous barrier
             if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-            pk_compaction(st, cnt_cur, q_cur, qm_cur, T, full, slot);
+            pk_compaction<WINDOW ? 4 : 2>(st, cnt_cur, q_cur, qm_cur, T, full, slot);
             if (!grid_sync(ctrl, nb, gen)) return;
             pass++;
-            if (threadIdx.x < NCLS) {
-                tb.cnt[threadIdx.x] = ld_coherent(cnt_cur + threadIdx.x);
-                tb.seg[threadIdx.x] = st.seg_off[threadIdx.x];
+            if (tid < NCLS) {
+                tb.cnt[tid] = ld_coherent(cnt_cur + tid);
+                tb.seg[tid] = st.seg_off[tid];
             }
             __syncthreads();
-            if (threadIdx.x < 64) {
+            if (tid < 64) {
                 const long long tot = frontier_size(tb.cnt);
-                if (threadIdx.x == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
+                if (tid == 0) s_total = tot > 0x7FFFFFFF ? 0x7FFFFFFF : (int)tot;
             }
             __syncthreads();
             if (s_total > 0) {
@@ -2147,7 +2172,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
         }
         const int total = s_total;
         if (total == 0 || (sp.max_iters > 0 && it >= sp.max_iters)) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
+            if (blockIdx.x == 0 && tid == 0) {
                 ctrl->iters = it;
                 ctrl->done = total == 0 ? 1 : 0;
                 if (total != 0) ctrl->error = NP_ERR_NOT_CONVERGED;
@@ -2155,13 +2180,13 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             return;
         }
         Cfg cfg = decide(sp, tb.cnt, it);
-        if (threadIdx.x < 64) build_tables(tb, pk_cfg(cfg, false), TABLES_PACKED, (long long)nb * WAVES);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (tid < 64) build_tables(tb, pk_cfg(cfg, false), TABLES_PACKED, (long long)nb * WAVES);
+        if (blockIdx.x == 0 && tid == 0) {
             ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
         }
         __syncthreads();
-        pk_expansion<UNIT, false>(st, PkFilt{}, q_cur, qm_cur, tb, s_tcol[threadIdx.x >> 6], s_tw[threadIdx.x >> 6], nullptr);
+        pk_expansion<UNIT, false>(st, PkFilt{}, q_cur, qm_cur, tb, s_tcol[tid >> 6], s_tw[tid >> 6], nullptr);
         if (!grid_sync(ctrl, nb, gen)) return;
     }
 }
@@ -2174,7 +2199,7 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
     if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-    pk_compaction(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
+    pk_compaction<4>(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
                   pass % 3);
 }
 
@@ -2728,13 +2753,14 @@ static const void *pick_persistent(bool batch, bool unit, bool push, bool solo) 
     return unit ? persistent_fn<false, true>(push, solo) : persistent_fn<false, false>(push, solo);
 }
 
-static const void *pick_packed(bool unit) {
-    return unit ? (const void *)&k_pk_persistent<true> : (const void *)&k_pk_persistent<false>;
+static const void *pick_packed(bool unit, bool window) {
+    if (window) return unit ? (const void *)&k_pk_persistent<true, true> : (const void *)&k_pk_persistent<false, true>;
+    return unit ? (const void *)&k_pk_persistent<true, false> : (const void *)&k_pk_persistent<false, false>;
 }
 
-int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo) {
+int persistent_max_wgs_per_cu(bool batch, bool unit, bool push, bool packed, bool solo, bool window) {
     int nb = 0;
-    const void *fn = packed ? pick_packed(unit) : pick_persistent(batch, unit, push, solo);
+    const void *fn = packed ? pick_packed(unit, window) : pick_persistent(batch, unit, push, solo);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, WG, 0) != hipSuccess) return 0;
     return nb;
 }
@@ -2744,7 +2770,7 @@ hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch,
     DevState a0 = st;
     SchedDev a1 = sp;
     void *args[] = {&a0, &a1};
-    const void *fn = st.kshift >= 0 ? pick_packed(unit) : pick_persistent(batch, unit, sp.push != 0, sp.solo != 0);
+    const void *fn = st.kshift >= 0 ? pick_packed(unit, sp.delta > 0) : pick_persistent(batch, unit, sp.push != 0, sp.solo != 0);
     return hipLaunchCooperativeKernel(fn, dim3(wgs), dim3(WG), args, 0, s);
 }
 
