@@ -84,7 +84,8 @@ typedef struct np_sched {
     int32_t log2_t_hi;   /* 0..30 */
     int32_t drive;       /* NP_DRIVE_* */
     int32_t frontier;    /* NP_FRONTIER_* */
-    int32_t wgs_per_cu;  /* persistent grid: workgroups per CU (0 = occupancy maximum) */
+    int32_t wgs_per_cu;  /* persistent grid: workgroups per CU, at most as many as fit
+                            (0 = chosen by the graph's edges and its rows' lengths) */
     int32_t graph_chunk; /* NP_DRIVE_GRAPH: iterations per captured chunk (0 = 16) */
     int32_t max_iters;   /* 0 = no cap beyond n+1 */
     int32_t trace;       /* nonzero: record per-iteration trace (np_trace_*) */

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <climits>
 #include <cmath>
 #include <vector>
 #include <algorithm>
@@ -336,19 +337,45 @@ static SchedDev make_schedd(np_ctx *c, const np_sched &s, int n_feat) {
     return d;
 }
 
-// Workgroups of a persistent solve over `edges` edges.  Every workgroup more makes the two grid
-// barriers of an iteration dearer, so a graph whose iterations are short gets one per CU (ER 65,536
-// / 1 M: 0.59 ms with 1, 0.64 with 4; grid 512^2: 1.20 and 1.32), a middling one two (grid 2048^2,
-// 17 M edges: 3.77 with 2, 3.94 with 4; learned on R-MAT s20, 17 M: 1.20 and 1.22), and only large
-// ones all that fit (R-MAT s22, 67 M: 5.6, 4.5, 4.2, 4.1 ms with 1 to 4).
+// Workgroups per CU of a persistent solve that does not ask for a number.  Every workgroup more makes
+// the two grid barriers of an iteration dearer, so a graph whose iterations are short gets one (ER
+// 65,536 / 1 M: 0.56 ms with 1, 0.59 with 4), a middling one two (grid 2048^2, 17 M edges: 3.48 with
+// 2, 3.54 with 4) and a large one three (ER 2 M / 41 M: 4.25 with 2, 4.27 with 3, 4.38 with 5; R-MAT
+// s22: 4.7, 3.6, 3.5, 3.35, 3.3 with 1 to 5).  But a row at or above the schedule's lower bin takes a
+// wavefront for itself, four dependent accesses long, and where a frontier can hold many of them the
+// wavefronts in flight decide: one workgroup more per 256 such rows on a CU (lower bin 2^4: ER 1 M /
+// 31 M, 1.0 M such rows: 8.3, 5.1, 4.0, 3.4 ms with 1 to 4; ER 2 M / 41 M: 15, 9.1, 7.1, 6.0, 5.4 with 1 to 5;
+// ER 65,536 / 1 M, 35 K: 0.64, 0.59, 0.58; R-MAT s20, 190 K: 1.60, 1.35, 1.38, 1.43).
 static constexpr long long SMALL_EDGES = 4ll << 20, LARGE_EDGES = 32ll << 20;
-static int persistent_wgs(np_ctx *c, const np_sched &s, const SchedDev &sd, bool batch, bool unit, bool packed,
-                          long long edges) {
-    int occ = persistent_max_wgs_per_cu(batch, unit, sd.push != 0, packed, sd.solo != 0, sd.delta > 0);
-    if (occ < 1) occ = 1;
-    const int fit = packed || edges > LARGE_EDGES ? occ : edges > SMALL_EDGES ? std::min(2, occ) : 1;
-    int per = s.wgs_per_cu > 0 ? std::min(s.wgs_per_cu, occ) : fit;
-    return per * c->num_cus;
+static int wanted_wgs(const np_ctx *c, const np_sched &s, const Space &sp, bool packed) {
+    if (s.wgs_per_cu > 0) return s.wgs_per_cu;
+    // vertices of out-degree at or above a bound
+    auto rows = [&](int first_class) {
+        long long r = 0;
+        for (int k = first_class; k < NCLS; ++k) r += sp.hist[k];
+        return r;
+    };
+    const long long per_wg = 256ll * c->num_cus;
+    // a pack: as many as give each tile of 64 vertices a wavefront (16 sources, 3 or 4 workgroups: ER
+    // 262,144 vertices 2.78, 2.34 ms; R-MAT s16 1.42, 1.51; s18, 150 K with out-edges 1.75, 1.82; s19 2.36, 2.10)
+    if (packed) return (int)std::max(3ll, std::min(8ll, (rows(1) + per_wg - 1) / per_wg));
+    const long long by_edges = sp.edges > LARGE_EDGES ? 3 : sp.edges > SMALL_EDGES ? 2 : 1;
+    return (int)std::max(by_edges, std::min(8ll, 1 + rows(s.log2_t_lo + 1) / per_wg));
+}
+// The grid of a persistent solve, and whether small frontiers run on one workgroup (sd->solo): not on
+// a graph of many edges, whose solve is a few large iterations, nor where more workgroups are wanted
+// than that kernel's registers allow.
+static int persistent_wgs(np_ctx *c, const np_sched &s, SchedDev *sd, const Space &sp, bool batch, bool unit,
+                          bool packed) {
+    const bool push = sd->push != 0, window = sd->delta > 0;
+    const int want = wanted_wgs(c, s, sp, packed);
+    sd->solo = !packed && !push && sp.edges <= LARGE_EDGES;
+    int occ = persistent_max_wgs_per_cu(batch, unit, push, packed, sd->solo != 0, window);
+    if (sd->solo && want > occ) {
+        sd->solo = 0;
+        occ = persistent_max_wgs_per_cu(batch, unit, push, packed, false, window);
+    }
+    return std::min(want, std::max(occ, 1)) * c->num_cus;
 }
 
 // Queued (vertex, source) pairs of a packed solve.
@@ -443,8 +470,7 @@ static int run_drive(np_ctx *c, Space &s, const DevState &st, const np_sched &sc
     if (sd.scheme != NP_SCHEME_CONSOLIDATE && drive == NP_DRIVE_PERSISTENT) drive = NP_DRIVE_HOSTLOOP;
     if (drive == NP_DRIVE_PERSISTENT) {
         SchedDev psd = sd;
-        psd.solo = st.kshift < 0 && !sd.push && s.edges <= LARGE_EDGES;
-        int wgs = persistent_wgs(c, sch, psd, batch, unit, st.kshift >= 0, s.edges);
+        int wgs = persistent_wgs(c, sch, &psd, s, batch, unit, st.kshift >= 0);
         HIPCHK(hipEventRecord(c->ev0, c->stream));
         hipError_t e = launch_persistent(st, psd, batch, unit, wgs, c->stream);
         if (e == hipErrorIllegalState || e == hipErrorCooperativeLaunchTooLarge) {
