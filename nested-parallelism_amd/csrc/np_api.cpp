@@ -362,6 +362,16 @@ static int wanted_wgs(const np_ctx *c, const np_sched &s, const Space &sp, bool 
     const long long by_edges = sp.edges > LARGE_EDGES ? 3 : sp.edges > SMALL_EDGES ? 2 : 1;
     return (int)std::max(by_edges, std::min(8ll, 1 + rows(s.log2_t_lo + 1) / per_wg));
 }
+// The grid sizes np_autotune and np_batch_autotune time for schedule s (grid_candidates): sp is the
+// space that runs it, null when parts of different kinds do.
+static std::vector<int> grid_options(const np_ctx *c, np_sched s, const Space *sp, bool batch, bool unit, bool packed) {
+    s.wgs_per_cu = 0;
+    const bool push = s.frontier == NP_FRONTIER_PUSH;
+    const int occ = std::max(1, persistent_max_wgs_per_cu(batch, unit, push, packed, false, s.delta > 0));
+    int w[4];
+    const int k = grid_candidates(sp ? std::min(occ, wanted_wgs(c, s, *sp, packed)) : 0, occ, w);
+    return std::vector<int>(w, w + k);
+}
 // The grid of a persistent solve, and whether small frontiers run on one workgroup (sd->solo): not on
 // a graph of many edges, whose solve is a few large iterations, nor where more workgroups are wanted
 // than that kernel's registers allow.
@@ -2274,10 +2284,7 @@ int np_autotune(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, const
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;  // the search is over the consolidation bins
-    int occ = persistent_max_wgs_per_cu(false, false, b0.frontier == NP_FRONTIER_PUSH, false, g->m <= LARGE_EDGES, false);
-    std::vector<int> wgs_opts = {0};
-    if (occ > 2) wgs_opts.push_back(2);
-    if (occ > 4) wgs_opts.push_back(4);
+    if ((rc = graph_space(c, g))) return rc;
     const int klos[] = {3, 4, 5, 6, 7};
     const int khis[] = {6, 8, 10, 12, 14, 30};
     double bestt = 1e30;
@@ -2291,12 +2298,13 @@ int np_autotune(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, const
             for (int khi : khis) {
                 if (lv == 0 && khi != khis[0]) continue;  // level 0 has no upper bin
                 if (khi < klo) continue;
-                for (int wg : wgs_opts) {
+                np_sched s = b0;
+                s.drive = drive;
+                s.level = lv; s.log2_t_lo = klo; s.log2_t_hi = khi;
+                s.trace = 0;
+                for (int wg : grid_options(c, s, &g->sp, false, false, false)) {
                     if (drive != NP_DRIVE_PERSISTENT && wg != 0) continue;  // one grid size per kernel
-                    np_sched s = b0;
-                    s.drive = drive;
-                    s.level = lv; s.log2_t_lo = klo; s.log2_t_hi = khi; s.wgs_per_cu = wg;
-                    s.trace = 0;
+                    s.wgs_per_cu = wg;
                     double tot = 0;
                     for (int i = 0; i < nsrc && rc == NP_OK; ++i) {
                         np_stats st;
@@ -2336,10 +2344,8 @@ int np_batch_autotune(np_ctx *c, np_batch *b, const np_sched *base, np_sched *be
     int rc = validate_sched(base, &b0);
     if (rc) return rc;
     b0.scheme = NP_SCHEME_CONSOLIDATE;
-    int occ = persistent_max_wgs_per_cu(true, b->unit != 0, false, !b->packs.empty(), b->sp.edges <= LARGE_EDGES, false);
-    std::vector<int> wgs_opts = {0};
-    if (occ > 2) wgs_opts.push_back(2);
-    if (occ > 4) wgs_opts.push_back(4);
+    const bool packed = !b->packs.empty();
+    const Space *one = !packed ? &b->sp : b->packs.size() == 1 && b->nconcat == 0 ? &b->packs[0]->sp : nullptr;
     const int klos[] = {3, 4, 5, 6, 7};
     const int khis[] = {6, 8, 10, 12, 14, 30};
     // One solve per candidate in the searches; a single timing varies by a few percent, so the
@@ -2379,12 +2385,13 @@ int np_batch_autotune(np_ctx *c, np_batch *b, const np_sched *base, np_sched *be
             for (int khi : khis) {
                 if (lv == 0 && khi != khis[0]) continue;  // level 0 has no upper bin
                 if (khi < klo) continue;
-                for (int wg : wgs_opts) {
+                np_sched s = b0;
+                s.drive = drive;
+                s.level = lv; s.log2_t_lo = klo; s.log2_t_hi = khi;
+                s.trace = 0;
+                for (int wg : grid_options(c, s, one, true, b->unit != 0, packed)) {
                     if (drive != NP_DRIVE_PERSISTENT && wg != 0) continue;  // one grid size per kernel
-                    np_sched s = b0;
-                    s.drive = drive;
-                    s.level = lv; s.log2_t_lo = klo; s.log2_t_hi = khi; s.wgs_per_cu = wg;
-                    s.trace = 0;
+                    s.wgs_per_cu = wg;
                     double t;
                     if ((rc = once(s, &t))) return rc;
                 }

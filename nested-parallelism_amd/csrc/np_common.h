@@ -44,6 +44,19 @@ NP_HD Cfg make_cfg(int level, int klo, int khi) {
     return c;
 }
 
+// Grid sizes (workgroups per CU) an autotuner times for one schedule of the persistent drive: 0, the
+// library's rule (which takes `rule` of them; 0 when several parts have rules of their own), then one, two
+// and all that fit, without the one the rule takes.  Returns their number; out holds 4.
+NP_HD int grid_candidates(int rule, int occ, int *out) {
+    int k = 0;
+    out[k++] = 0;
+    for (int i = 0; i < 3; ++i) {
+        const int w = i < 2 ? i + 1 : occ;
+        if (w != rule && w <= occ && w != out[k - 1]) out[k++] = w;
+    }
+    return k;
+}
+
 // ---------------------------------------------------------------------------------
 // Counter-based random numbers: SplitMix64 (G. Steele, D. Lea, C. Flood, "Fast
 // splittable pseudorandom number generators", OOPSLA 2014) finaliser over a keyed
