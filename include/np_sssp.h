@@ -412,7 +412,8 @@ int np_color(np_ctx *ctx, np_graph *g, int32_t method, int32_t *color_out, np_st
  * float64; rank_out[n] receives float values (graph.rankArray, FLOAT_T = float).  max_iters = 0:
  * no cap beyond 100000 (NP_ERR_NOT_CONVERGED past it).  stats.iterations = iterations run.
  * Its device buffers (in-edge CSR, row bins, ranks) come from a workspace the context keeps
- * and grows to the largest call (shared with np_spmv, freed by np_destroy), so repeated calls
+ * and grows to the largest call (shared with np_spmv, and with np_bc and np_color calls of up to
+ * 1 GiB, which allocate and free more than that themselves; freed by np_destroy), so repeated calls
  * allocate nothing; calls on one context must not overlap (one context per thread). */
 int np_pagerank(np_ctx *ctx, np_graph *g, int32_t max_iters, float *rank_out, np_stats *stats);
 

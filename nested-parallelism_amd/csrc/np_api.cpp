@@ -748,6 +748,23 @@ static hipError_t ctx_workspace(np_ctx *c, size_t bytes, char **p) {
     return hipSuccess;
 }
 
+// Device memory of one np_bc or np_color call: the context's workspace up to CALL_WORKSPACE (or what it
+// holds already), above that an allocation that ends with the call.  Twelve allocations and as many
+// frees were 0.25 ms of an np_bc call on R-MAT s16 and 2 ms on s20 (32 sources: 10 % and 40 % of it); but the
+// workspace is not shrunk while the context lives, and np_bc takes up to 800 bytes per vertex of a
+// large graph, np_color 16.
+constexpr size_t CALL_WORKSPACE = 1ull << 30;
+struct CallMemory {
+    char *own = nullptr;
+    hipError_t take(np_ctx *c, size_t bytes, char **p) {
+        if (bytes <= std::max(CALL_WORKSPACE, c->ws_bytes)) return ctx_workspace(c, bytes, p);
+        hipError_t e = dalloc(&own, bytes);
+        *p = own;
+        return e;
+    }
+    ~CallMemory() { dfree(own); }
+};
+
 // Buffers of np_bc.
 struct BcBufs {
     int *ent_v, *srcs, *err;
@@ -757,15 +774,7 @@ struct BcBufs {
     unsigned *ent_m;
     double *sig, *del, *acc;
     float *out;
-    char *own = nullptr;  // the call's own allocation, when it is not the context's workspace
-    ~BcBufs() { dfree(own); }
 };
-
-// Twelve allocations and as many frees were 0.25 ms of a call on R-MAT s16 and 2 ms on s20 (32
-// sources: 10 % and 40 % of it); the buffers are carved from the context's workspace up to this
-// size.  Above it, the call allocates once and frees: the workspace is not shrunk while the context
-// lives, and a batch of a large graph takes 800 bytes per vertex.
-constexpr size_t BC_WORKSPACE = 1ull << 30;
 
 // ------------------------------------------------------------------------------------
 // C ABI
@@ -1196,15 +1205,11 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     const size_t NB = (size_t)n + BC_RUN + 2;
     const size_t slots = (size_t)n << ks;
     BcBufs bb;
+    CallMemory mem;
     Carve cv;
     for (int pass = 0; pass < 2; ++pass) {  // size, then carve
         if (pass) {
-            if (cv.off <= BC_WORKSPACE) {
-                HIPCHK(ctx_workspace(c, cv.off, &cv.base));
-            } else {
-                HIPCHK(dalloc(&bb.own, cv.off));
-                cv.base = bb.own;
-            }
+            HIPCHK(mem.take(c, cv.off, &cv.base));
             cv.off = 0;
         }
         bb.st = cv.take<uint2>((size_t)n);
@@ -1285,10 +1290,6 @@ int np_bc(np_ctx *c, np_graph *g, const int32_t *srcs, int32_t nsrc, float *bc_o
     return NP_OK;
 }
 
-}  // extern "C"
-
-extern "C" {
-
 // ---- graph coloring --------------------------------------------------------------------
 // GRAPH_COLOR_GPU (apps/graph-color/src/gpu/graph_color_wrapper.cu:598-699): method 0 = one launch
 // in the order of the ids (O(m)), method 1 = the reference's rounds (O(rounds x m)).
@@ -1303,10 +1304,11 @@ int np_color(np_ctx *c, np_graph *g, int32_t method, int32_t *color_out, np_stat
     int *h = (int *)c->h_small;
     HIPCHK(color_scan(nullptr, &cb.temp_bytes, nullptr, nullptr, n, c->stream));
     const long long cap = color_ticket_cap(n, g->m);
+    CallMemory mem;
     Carve cv;
-    for (int pass = 0; pass < 2; ++pass) {  // size, then carve from the context's workspace
+    for (int pass = 0; pass < 2; ++pass) {  // size, then carve
         if (pass) {
-            HIPCHK(ctx_workspace(c, cv.off, &cv.base));
+            HIPCHK(mem.take(c, cv.off, &cv.base));
             cv.off = 0;
         }
         cb.color = cv.take<int>((size_t)n);

@@ -1,6 +1,8 @@
+import ctypes
 import importlib.util
 import os
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -85,3 +87,20 @@ def hub_csr(rng, n, m, hub_sizes, inward=False):
 
 def load_golden(name):
     return dict(np.load(os.path.join(GOLDEN, name), allow_pickle=False))
+
+
+def free_bytes(npa):
+    """Free device memory, as the library's HIP runtime reports it."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert npa.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def memory_is_back(npa, before):
+    """Whether free device memory returns to within 64 MiB of `before` (a large free shows up in the
+    report some milliseconds after the call)."""
+    for _ in range(100):
+        if free_bytes(npa) >= before - (64 << 20):
+            return True
+        time.sleep(0.05)
+    return False

@@ -6,7 +6,7 @@ order varies) and returns float32, as the reference's float *bc; the bar is
 import numpy as np
 import pytest
 
-from conftest import random_csr
+from conftest import free_bytes, memory_is_back, random_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -117,3 +117,23 @@ def test_bc_overflowed_path_count_stays_with_its_source(npa, ctx, orc):
     bc, _ = ctx.bc(G, [0, b])
     assert np.allclose(bc, ref, rtol=RTOL, atol=ATOL)
     G.free()
+
+
+def test_bc_buffers_larger_than_the_kept_workspace(npa, orc):
+    """13.6 million vertices: the call's buffers take more than 1 GiB, so it allocates and frees them
+    itself; same results, and the memory is back afterwards."""
+    ctx = npa.Context(0)                       # nothing kept from other calls
+    n = 13 << 20
+    rng = np.random.default_rng(58)
+    src = np.sort(rng.integers(0, 3000, 20000))
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    col = rng.integers(0, 3000, 20000).astype(np.int32)
+    G = _graph(npa, ctx, row, col)
+    before = free_bytes(npa)
+    bc, _ = ctx.bc(G, [int(src[0])])
+    assert memory_is_back(npa, before)
+    ref = orc.bc(row, col, [int(src[0])])
+    assert np.allclose(bc, ref, rtol=RTOL, atol=ATOL)
+    G.free()
+    ctx.close()

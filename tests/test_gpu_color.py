@@ -5,7 +5,7 @@ import subprocess
 import numpy as np
 import pytest
 
-from conftest import GOLDEN, PKG_DIR, load_golden, random_csr
+from conftest import GOLDEN, PKG_DIR, free_bytes, load_golden, memory_is_back, random_csr
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +99,22 @@ def test_color_ticket_boundaries_match_oracle(npa, ctx, orc, case):
         assert np.array_equal(got, ref), case
         assert st.iterations == int(ref.max())
     G.free()
+
+
+def test_color_gives_back_large_buffers(npa, orc):
+    """84 million vertices: the call's buffers take more than the 1 GiB that a context keeps, so the
+    memory is back afterwards; same colors."""
+    ctx = npa.Context(0)                              # nothing kept from other calls
+    n = 80 << 20
+    rng = np.random.default_rng(76)
+    src = np.sort(rng.integers(0, n, 4000))
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    col = np.where(rng.random(4000) < 0.5, src[rng.integers(0, 4000, 4000)], rng.integers(0, n, 4000)).astype(np.int32)
+    G = npa.Graph.from_csr(ctx, row, col, np.ones(len(col), np.int32))
+    before = free_bytes(npa)
+    got, _ = ctx.color(G)
+    assert memory_is_back(npa, before)
+    assert np.array_equal(got, orc.color(row, col))
+    G.free()
+    ctx.close()
