@@ -284,7 +284,10 @@ int np_batch_solve(np_ctx *ctx, np_batch *b, const np_sched *sched, np_stats *st
 /* Host copy of instance i's distances (int32[n_i]). */
 int np_batch_get(np_ctx *ctx, np_batch *b, int32_t i, int32_t *dist_out);
 /* Device address of instance i's distances, in the caller's vertex ids (valid until the
- * next solve or free of the batch). */
+ * next solve or free of the batch).  Results of instances that share a graph, or whose graph is
+ * renumbered, are written to the caller's ids when they are asked for: the first request after a solve
+ * writes that instance's (every instance's of the part when the solve before had several asked for),
+ * the second all the others of the part. */
 int np_batch_device_dist(np_batch *b, int32_t i, const int32_t **d_dist);
 /* Number of packs and of instances in the concatenated part. */
 int np_batch_layout(const np_batch *b, int32_t *packs, int32_t *concatenated);

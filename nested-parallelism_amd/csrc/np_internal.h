@@ -147,8 +147,8 @@ hipError_t launch_copy_cls(const unsigned char *src, unsigned char *dst, long lo
 // Source-packed state: dist rows set to inf, source i of srcs[] at lane i (nsrc <= 2^kshift);
 // delta > 0 starts a priority window at T = delta.
 hipError_t launch_init_packed(const DevState &st, const int *d_srcs, int nsrc, int delta, hipStream_t s);
-// out[to.off[j] + v] = dist[(map(v) << kshift) + j] for j < to.count, map = old2new or identity
-// (old2new null).
+// out[to.off[j] + v] = dist[(map(v) << kshift) + j] for j < to.count with to.off[j] >= 0, map = old2new
+// or identity (old2new null).
 struct UnpackTo { long long off[PACK_MAX]; int count; };
 hipError_t launch_unpack(const int *dist, int kshift, const UnpackTo &to, const int *old2new, int n, int *out,
                          hipStream_t s);

@@ -2343,7 +2343,7 @@ __global__ __launch_bounds__(WG) void k_unpack(const int *dist, UnpackTo to, con
         }
 #pragma unroll
         for (int j = 0; j < (1 << KS); ++j)
-            if (j < to.count) out[to.off[j] + v] = d[j];
+            if (j < to.count && to.off[j] >= 0) out[to.off[j] + v] = d[j];
     }
 }
 

@@ -111,3 +111,60 @@ def test_hold_with_hubs_side_by_side(npa, ctx, orc, n, hold, unit):
             assert np.array_equal(b.get(i), ref), (drive, i)
     b.free()
     G.free()
+
+
+def _at(npa, ctx, ptr, n):
+    out = np.empty(n, np.int32)
+    assert npa.load().np_dev_copy(ctx.h, out.ctypes.data, ptr, out.nbytes, 1) == 0
+    return out
+
+
+@pytest.mark.parametrize("k", [2, 4, 9, 32])
+@pytest.mark.parametrize("part", ["pack", "concatenated"])
+def test_one_request_writes_one_result(npa, ctx, orc, k, part):
+    """A program that asks for one result after each solve does not pay for the others: what an earlier
+    solve wrote for another instance is still there.  Then every mix of requests over repeated solves
+    of a pack, or of renumbered graphs in one slot space, gives the results of its own solve."""
+    rng = np.random.default_rng(400 + k)
+    ctx.set_option(npa.CTX_RELABEL, 1)
+    try:
+        graphs = [npa.Graph.from_csr(ctx, *random_csr(rng, 700 + 13 * j, 6000, 1, 50)) for j in range(1 if part == "pack" else k)]
+    finally:
+        ctx.set_option(npa.CTX_RELABEL, 2)
+    of = graphs * k if part == "pack" else graphs
+    host = [g.download() for g in graphs]
+    csr = host * k if part == "pack" else host
+    srcs = [int(np.argmax(np.diff(r[0]) == d)) for r, d in zip(csr, [max(np.diff(r[0])) for r in csr])]
+    srcs = [int(rng.integers(g.n)) if part == "pack" and j else s for j, (g, s) in enumerate(zip(of, srcs))]
+    full = [orc.dijkstra(*r, s)[0] for r, s in zip(csr, srcs)]
+    b = npa.Batch(ctx, of, srcs)
+    assert b.layout() == ((1, 0) if part == "pack" else (0, k))
+
+    def solve(stop):
+        """A whole solve, or one stopped after the sources' own expansion."""
+        if not stop:
+            b.solve(npa.Sched(level=1))
+            return full
+        with pytest.raises(npa.NpError):
+            b.solve(npa.Sched(level=1, max_iters=1))
+        one = []
+        for (row, col, w), s, g in zip(csr, srcs, of):
+            d = np.full(g.n, npa.INF, np.int32)
+            np.minimum.at(d, col[row[s]:row[s + 1]], w[row[s]:row[s + 1]])
+            d[s] = 0
+            one.append(d)
+        return one
+
+    solve(False)
+    p = b.device_dist(1)
+    assert np.array_equal(_at(npa, ctx, p, of[1].n), full[1])
+    want = solve(True)
+    assert np.array_equal(_at(npa, ctx, b.device_dist(0), of[0].n), want[0])
+    assert np.array_equal(_at(npa, ctx, p, of[1].n), full[1])
+    for step, asked in enumerate([[0], [1], [0, 1], list(range(k)), [k - 1], [k - 1, 0], [0], list(range(k)), [], [1, 1, 0]]):
+        want = solve(step % 2 == 1)
+        for i in asked:
+            assert np.array_equal(b.get(i), want[i]), (step, asked, i)
+    b.free()
+    for g in graphs:
+        g.free()
