@@ -304,10 +304,10 @@ __device__ __forceinline__ void lane_tile(const DevState &st, const PushCtx &pc,
 }
 
 // Shortest rows: a lane per queued vertex walks its edges, UNR loads in flight.  No owner search;
-// the rows of neighbouring vertices share cache lines.  Not for pushed frontiers: the vertices would be
+// the rows of neighbouring vertices share cache lines.  Not for pushed distances: the vertices would be
 // appended in an order that keeps neighbours apart, and the next frontier's reads with them (grid 3200^2
-// 36.4 -> 38.2 ms, 2048^2 16.1 -> 16.8).
-template <bool BATCH, bool UNIT>
+// 36.4 -> 38.2 ms, 2048^2 16.1 -> 16.8); levels settle at once and gain (grid 1200^2 1.81 -> 1.72).
+template <bool BATCH, bool UNIT, bool PUSH>
 __device__ __forceinline__ void lane_serial(const DevState &st, const PushCtx &pc, const int *q, long long qidx,
                                             int nvalid) {
     const int lane = lane_id();
@@ -319,6 +319,7 @@ __device__ __forceinline__ void lane_serial(const DevState &st, const PushCtx &p
         s = st.row[VB + v];
         d = st.row[VB + v + 1] - s;
         du = ld_coherent(st.dist + slot);
+        if (PUSH) st_coherent_u(pc.bm_cur + (slot >> 5), 0u);
     }
     for (int i = 0; __ballot(i < d) != 0; i += UNR) {
         int tv[UNR], alt[UNR], cur[UNR];
@@ -332,8 +333,10 @@ __device__ __forceinline__ void lane_serial(const DevState &st, const PushCtx &p
         for (int k = 0; k < UNR; ++k) cur[k] = i + k < d ? ld_coherent(st.dist + tv[k]) : 0;
 #pragma unroll
         for (int k = 0; k < UNR; ++k) {
+            bool want = false;
             int c = 0;
-            if (alt[k] < cur[k]) relax_tail<false>(st, pc, tv[k], alt[k], c);
+            if (alt[k] < cur[k]) want = relax_tail<PUSH>(st, pc, tv[k], alt[k], c);
+            if (PUSH) push_wave(st, pc, want, tv[k], c);
         }
     }
 }
@@ -489,7 +492,7 @@ __device__ void expansion(const DevState &st, const PushCtx &pc, const int *q, I
             const int tv = c <= SERIAL_CLS ? 64 : tb.tv;
             long long first = ti * tv;
             int nvalid = (int)((long long)tb.cnt[c] - first < tv ? (long long)tb.cnt[c] - first : tv);
-            if (!PUSH && c <= SERIAL_CLS) lane_serial<BATCH, UNIT>(st, pc, q, tb.seg[c] + first, nvalid);
+            if ((UNIT || !PUSH) && c <= SERIAL_CLS) lane_serial<BATCH, UNIT, PUSH>(st, pc, q, tb.seg[c] + first, nvalid);
             else lane_tile<BATCH, UNIT, PUSH, GUARD>(st, pc, q, tb.seg[c] + first, nvalid);
         }
     }
