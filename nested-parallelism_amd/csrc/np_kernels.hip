@@ -732,27 +732,26 @@ __device__ __forceinline__ Cfg decide(const SchedDev &sp, const int *cnt, int it
     return decide_mlp(sp.mlp, sp.n_feat, sp.level, sp.klo, sp.khi, cnt, it);
 }
 
-__device__ __forceinline__ void record_trace_rec(np_trace_rec *r, int it, int level, int klo, int khi, const int *cnt,
-                                                 long long t0, Ctrl *ctrl) {
-    long long pairs = 0;
-#pragma unroll 1
-    for (int l = 0; l < BAR_LEAVES; ++l) pairs += __hip_atomic_load(&ctrl->leaf[l].pairs, __ATOMIC_RELAXED, NP_AGENT);
-    r->pairs = pairs;
-    r->edges = __hip_atomic_load(&ctrl->edges_total, __ATOMIC_RELAXED, NP_AGENT);
-    r->iteration = it;
-    r->level = level;
-    r->log2_t_lo = klo;
-    r->log2_t_hi = khi;
-#pragma unroll 1
-    for (int c = 0; c < NCLS; ++c) r->count[c] = cnt[c];
-    r->t_begin = t0;
-    r->t_end = t0;
-}
-
+// The first wavefront records an iteration (lane c holds class c; t0 is lane 0's).
 __device__ __forceinline__ void record_trace(const SchedDev &sp, int it, const Cfg &cfg, const int *cnt,
                                              long long t0, Ctrl *ctrl) {
     if (!sp.trace || it >= sp.trace_cap) return;
-    record_trace_rec(sp.trace + it, it, cfg.level, cfg.klo, cfg.khi, cnt, t0, ctrl);
+    np_trace_rec *r = sp.trace + it;
+    const int lane = lane_id();
+    long long pairs = lane < BAR_LEAVES ? __hip_atomic_load(&ctrl->leaf[lane].pairs, __ATOMIC_RELAXED, NP_AGENT) : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) pairs += __shfl_xor(pairs, o);
+    if (lane < NCLS) r->count[lane] = cnt[lane];
+    if (lane == 0) {
+        r->pairs = pairs;
+        r->edges = __hip_atomic_load(&ctrl->edges_total, __ATOMIC_RELAXED, NP_AGENT);
+        r->iteration = it;
+        r->level = cfg.level;
+        r->log2_t_lo = cfg.klo;
+        r->log2_t_hi = cfg.khi;
+        r->t_begin = t0;
+        r->t_end = t0;
+    }
 }
 
 // ------------------------------------------------------------------------------------
@@ -977,8 +976,8 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
         }
         Cfg cfg = decide(sp, tb.cnt, done_iters);
         if (tid < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
-        if (blockIdx.x == 0 && tid == 0) {
-            ctrl->frontier_total += total;
+        if (blockIdx.x == 0 && tid < 64) {
+            if (tid == 0) ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
         }
         __syncthreads();
@@ -1064,16 +1063,15 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
         }
     }
     Cfg cfg = decide(sp, s_cnt, ctrl->iters);
-    if (threadIdx.x == 0) {
-        if (ctrl->cfg_pad == 0) {  // cfg_pad != 0: a forced schedule (stepping) is kept
-            ctrl->cfg_level = cfg.level;
-            ctrl->cfg_klo = cfg.klo;
-            ctrl->cfg_khi = cfg.khi;
-        } else {
-            cfg = make_cfg(ctrl->cfg_level, ctrl->cfg_klo, ctrl->cfg_khi);
-        }
-        ctrl->frontier_total += tot;
+    if (threadIdx.x < 64) {
+        if (ctrl->cfg_pad != 0) cfg = make_cfg(ctrl->cfg_level, ctrl->cfg_klo, ctrl->cfg_khi);  // forced (stepping)
         record_trace(sp, ctrl->iters, cfg, s_cnt, (long long)wall_clock64(), ctrl);
+    }
+    if (threadIdx.x == 0) {
+        ctrl->cfg_level = cfg.level;
+        ctrl->cfg_klo = cfg.klo;
+        ctrl->cfg_khi = cfg.khi;
+        ctrl->frontier_total += tot;
         ctrl->iters += 1;
         ctrl->skip = 0;
         ctrl->full = 0;
@@ -2184,8 +2182,8 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
         }
         Cfg cfg = decide(sp, tb.cnt, it);
         if (tid < 64) build_tables(tb, pk_cfg(cfg, false), TABLES_PACKED, (long long)nb * WAVES);
-        if (blockIdx.x == 0 && tid == 0) {
-            ctrl->frontier_total += total;
+        if (blockIdx.x == 0 && tid < 64) {
+            if (tid == 0) ctrl->frontier_total += total;
             record_trace(sp, it, cfg, tb.cnt, t_prev, ctrl);
         }
         __syncthreads();
