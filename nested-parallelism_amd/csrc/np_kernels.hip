@@ -1884,12 +1884,23 @@ __device__ __forceinline__ int pk_reached(const DevState &st, long long v) {
 }
 
 // Lane q of a group of 8 has vertex v's distances of sources 4q .. 4q + 3 (rows of 1 or 2: source q).
-// Through the caches: a value older than the last atomicMin is only larger, so it can only keep a
-// pair pending one pass longer (every pending pair is expanded eventually).
+// Through the caches in a launch of its own, which starts with none of them.  Inside the persistent
+// kernel a cached row can be many iterations old, and only larger: pairs below the window were
+// deferred, and the window rose above distances that were long passed (3 sources of a 2048^2 grid,
+// window 2000: 339 iterations against 146 of launches), so there the loads are coherent.
+template <bool COHERENT>
 __device__ __forceinline__ int4 pk_row_part(const DevState &st, long long v, int q, bool ok) {
     const int *row = st.dist + (v << st.kshift);
-    if (st.kshift < 2) return int4{ok && q < (1 << st.kshift) ? row[q] : 0, 0, 0, 0};
-    return ok && q < (1 << (st.kshift - 2)) ? ((const int4 *)row)[q] : int4{0, 0, 0, 0};
+    if (st.kshift < 2) {
+        const bool in = ok && q < (1 << st.kshift);
+        return int4{!in ? 0 : COHERENT ? ld_coherent(row + q) : row[q], 0, 0, 0};
+    }
+    if (!ok || q >= (1 << (st.kshift - 2))) return int4{0, 0, 0, 0};
+    if (!COHERENT) return ((const int4 *)row)[q];
+    const unsigned long long *p = (const unsigned long long *)row + 2 * q;
+    const unsigned long long a = __hip_atomic_load(p, __ATOMIC_RELAXED, NP_AGENT);
+    const unsigned long long b = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, NP_AGENT);
+    return int4{(int)a, (int)(a >> 32), (int)b, (int)(b >> 32)};
 }
 // The group's sources of mask m whose distance is below the window T, and the least distance among
 // its others (both in every lane of the group).
@@ -1923,7 +1934,7 @@ __device__ __forceinline__ unsigned pk_take(const DevState &st, int4 x, int q, u
 // once after, looks at every deferred one.  Kept flagged and re-read in every pass by a lane per
 // row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid 16.5 -> 7.4 ms
 // of it per solve (13.4 with a lane per row still), the solve 33.2 -> 26.5 ms.
-template <int WIN_UNR>
+template <int WIN_UNR, bool COHERENT>
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
                                               int T, bool full, int slot) {
     __shared__ int s_wc[WAVES][NCLS];
@@ -1997,7 +2008,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                     const long long v = w0 * 32 + (e[k] & 2047);
                     f[k] = e[k] ? ld_coherent_u(st.mflag + v) : 0u;
                     old[k] = e[k] ? ld_coherent_u(st.deferred + v) : 0u;
-                    x[k] = pk_row_part(st, v, q, e[k] != 0);
+                    x[k] = pk_row_part<COHERENT>(st, v, q, e[k] != 0);
                 }
                 wave_lds_order();
 #pragma unroll
@@ -2140,7 +2151,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             const int slot = pass % 3;
             // the statistics slot of the next pass was last read before the previous barrier
             if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-            pk_compaction<WINDOW ? 4 : 2>(st, cnt_cur, q_cur, qm_cur, T, full, slot);
+            pk_compaction<WINDOW ? 4 : 2, true>(st, cnt_cur, q_cur, qm_cur, T, full, slot);
             if (!grid_sync(ctrl, nb, gen)) return;
             pass++;
             if (tid < NCLS) {
@@ -2200,7 +2211,7 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
     if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-    pk_compaction<4>(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
+    pk_compaction<4, false>(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
                   pass % 3);
 }
 

@@ -184,3 +184,18 @@ def test_distance_range_is_checked_at_every_index(npa, ctx, n):
                         ctx.sssp_device(G, src, buf.ptr + 4 * off, npa.Sched(level=1))
             G.free()
     buf.free()
+
+
+@pytest.mark.parametrize("nsrc", [2, 3, 16])
+def test_packed_window_follows_the_current_distances_on_every_drive(npa, ctx, nsrc):
+    """One launch per solve sees other workgroups' distances as launches per step do: a window that
+    goes by rows of earlier iterations defers pairs below it and rises above them, which showed as more
+    than twice the iterations."""
+    G = npa.Graph.grid(ctx, 700, 701, None, 1, 1000, seed=97)
+    srcs = [int(s) for s in npa.pick_sources(G.download()[0], nsrc, 9)]
+    b = npa.Batch(ctx, [G] * nsrc, srcs)
+    for delta in (1000, 3000, 8000):
+        it = [b.solve(npa.Sched(level=2, log2_t_lo=6, log2_t_hi=8, delta=delta, drive=dr)).iterations for dr in (0, 1, 2)]
+        assert it[0] <= 1.15 * min(it[1:]), (delta, it)
+    b.free()
+    G.free()
