@@ -31,7 +31,7 @@ constexpr int BAR_LEAVES = 32;
 struct alignas(128) BarLeaf {
     unsigned long long n;     // grid barrier: cumulative arrivals
     long long pairs;          // source-packed: queued (vertex, source) pairs, summed over iterations
-    int dcnt[3];              // per compaction pass (rotating): flagged vertices kept back
+    int dcnt[3];              // per compaction pass, a pack's per window (rotating): flagged vertices kept back
     int dmin[3];              // ... and the least distance among them
 };
 
@@ -52,6 +52,7 @@ struct Ctrl {
     int pass;                 // compaction passes so far (host-loop / graph drives)
     int skip;                 // host-loop / graph drives: this slot only raised the window
     int full;                 // windowed pack: the next compaction looks at the deferred pairs too
+    int win;                  // windowed pack: times the window has risen
     long long edges_total;    // source-packed: sum over iterations of the queued vertices' out-degrees
     long long items_total;    // source-packed: ... of out-degree x queued sources ((edge, source) items)
     int solo;                 // persistent drive: iterations of the last solo visit

@@ -1017,23 +1017,17 @@ __global__ __launch_bounds__(WG) void k_decide(DevState st, SchedDev sp, int it_
     const int pass = ld_coherent(&ctrl->pass);  // the compaction of this slot
     if (tot == 0 && !sp.push) {
         const int T = ld_coherent(&ctrl->thresh);
-        if (st.deferred && T != NO_WINDOW && !ld_coherent(&ctrl->full)) {
-            // a windowed pack's passes look at the flagged pairs only: now at the deferred ones
-            if (threadIdx.x == 0) {
-                ctrl->full = 1;
-                ctrl->skip = 1;
-                ctrl->pass = pass + 1;
-            }
-            return;
-        }
+        const int win = ld_coherent(&ctrl->win);
         int kept, mn;
-        deferred_sums(ctrl, pass % 3, &kept, &mn);
-        if ((T != NO_WINDOW || st.hold_cls) && kept > 0) {
+        deferred_sums(ctrl, (st.deferred ? win : pass) % 3, &kept, &mn);
+        if (T != NO_WINDOW ? mn != NO_WINDOW : st.hold_cls && kept != 0) {
             // nothing queued but pairs kept back: raise the window (held vertices need only the
             // next pass); this slot's expansion is skipped
             if (threadIdx.x == 0) {
                 if (T != NO_WINDOW) {
                     ctrl->thresh = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
+                    ctrl->full = 1;  // a pack's next pass looks at its deferred pairs
+                    ctrl->win = win + 1;
                 }
                 ctrl->skip = 1;
                 ctrl->pass = pass + 1;
@@ -1927,13 +1921,16 @@ __device__ __forceinline__ unsigned pk_take(const DevState &st, int4 x, int q, u
 
 // Vertices with pending sources -> class-segmented queue with their source masks.  With a
 // priority window (T < NO_WINDOW) only the (vertex, source) pairs with dist < T are queued; the
-// others move from mflag[v] to deferred[v].  A deferred pair is below
-// the window only after a relaxation, which flags it again, or after the window has risen: so the
-// passes of one window look at the flagged pairs alone, and only a `full` pass, once before the
-// window rises (the deferred pairs' count and least distance go to the pass's deferral sums) and
-// once after, looks at every deferred one.  Kept flagged and re-read in every pass by a lane per
-// row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid 16.5 -> 7.4 ms
-// of it per solve (13.4 with a lane per row still), the solve 33.2 -> 26.5 ms.
+// others move from mflag[v] to deferred[v].  A deferred pair is below the window only after a
+// relaxation, which flags it again, or after the window has risen: so the passes of one window look at
+// the flagged pairs alone, and only a `full` pass, the first one after the window has risen, looks at
+// every deferred one.  Every pass adds the pairs it defers to the window's sums (`slot`), so the least
+// of them bounds all that are pending from below when the window has to rise; the bound may belong to
+// a pair taken since, then the window rises once more.  Kept flagged and re-read in every pass by a
+// lane per row, the rows of the deferred were most of the compaction: 32 sources of a 2048^2 grid
+// 16.5 -> 7.4 ms of it per solve (13.4 with a lane per row still), the solve 33.2 -> 26.5 ms.  A second
+// full pass, to find the least pending distance before the window rises, cost small packs more than
+// that saved (persistent drive, 3 sources of a 300^2 grid 6.2 -> 8.0 ms).
 template <int WIN_UNR, bool COHERENT>
 __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, int *q_out, unsigned *qm_out,
                                               int T, bool full, int slot) {
@@ -2015,20 +2012,21 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
                 for (int k = 0; k < WIN_UNR; ++k) {
                     const long long v = w0 * 32 + (e[k] & 2047);
                     int dmin;
-                    const unsigned t = pk_take(st, x[k], q, full ? f[k] | old[k] : f[k], T, &dmin);
+                    const unsigned m = full ? f[k] | old[k] : f[k];
+                    const unsigned t = pk_take(st, x[k], q, m, T, &dmin);
                     const unsigned rest = (old[k] | f[k]) & ~t;
                     const bool take = q == 0 && t != 0;
                     if (q == 0 && e[k]) {
                         if (f[k] != t) st_coherent_u(st.mflag + v, t);
                         if (rest != old[k]) st_coherent_u(st.deferred + v, rest);
-                        if (full && rest) {
-                            my_dc += __popc(rest);
+                        if (m & ~t) {
+                            my_dc += __popc(m & ~t);
                             my_dm = dmin < my_dm ? dmin : my_dm;
                         }
                     }
-                    const unsigned long long m = __ballot(take);
-                    if (take) list[left + __popcll(m & lanes_below(lane))] = (unsigned short)e[k];
-                    left += __popcll(m);
+                    const unsigned long long queued = __ballot(take);
+                    if (take) list[left + __popcll(queued & lanes_below(lane))] = (unsigned short)e[k];
+                    left += __popcll(queued);
                 }
             }
             n = left;
@@ -2102,7 +2100,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     __syncthreads();
     if (tid == 0 && s_pairs)
         atomicAdd((unsigned long long *)&st.ctrl->leaf[blockIdx.x % BAR_LEAVES].pairs, (unsigned long long)s_pairs);
-    if (full || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
+    if (windowed || st.hold_cls) flush_deferred(st.ctrl, slot, my_dc, my_dm, &s_dc, &s_dm);
 }
 
 // Lane-bin bound of a packed expansion (see PACK_LANE_CLS); the other bins keep theirs.  A filtered
@@ -2134,7 +2132,7 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
     // priority window: every workgroup computes the same sequence of thresholds
     int T = sp.delta > 0 ? sp.delta : NO_WINDOW;
     bool full = false;
-    int pass = 0;
+    int pass = 0, win = 0;
     for (int it = 0;; ++it) {
         const int tid = phase_tid();
         int *cnt_cur = st.cnt + (it % 3) * NCLS;
@@ -2148,10 +2146,11 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
         }
         if (blockIdx.x == 0 && tid < NCLS) st_coherent(cnt_zero + tid, 0);
         for (;;) {
-            const int slot = pass % 3;
-            // the statistics slot of the next pass was last read before the previous barrier
-            if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
-            pk_compaction<WINDOW ? 4 : 2, true>(st, cnt_cur, q_cur, qm_cur, T, full, slot);
+            // the sums of a window, or of a pass (held vertices); the next ones' were last read before
+            // the previous barrier
+            const int sums = st.deferred ? win : pass;
+            if (blockIdx.x == 0) deferred_clear(ctrl, (sums + 1) % 3);
+            pk_compaction<WINDOW ? 4 : 2, true>(st, cnt_cur, q_cur, qm_cur, T, full, sums % 3);
             if (!grid_sync(ctrl, nb, gen)) return;
             pass++;
             if (tid < NCLS) {
@@ -2168,18 +2167,16 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
                 full = false;
                 break;
             }
-            // nothing queued: the deferred pairs are looked at; done unless pairs were kept back
-            // (by the window, or held vertices, which the next pass takes); a window rises to the
-            // least pending distance + delta
-            if (T != NO_WINDOW && !full) {
-                full = true;
-                continue;
-            }
+            // nothing queued: done unless pairs are kept back (by the window, which rises to the least
+            // of them + delta, or held vertices, which the next pass takes)
+            if (st.deferred && T == NO_WINDOW) break;
             int kept, mn;
-            deferred_sums(ctrl, slot, &kept, &mn);
-            if (kept == 0) break;
+            deferred_sums(ctrl, sums % 3, &kept, &mn);
+            if (T == NO_WINDOW ? kept == 0 : mn == NO_WINDOW) break;
             if (T != NO_WINDOW) {
                 T = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
+                full = true;
+                win++;
             }
         }
         const int total = s_total;
@@ -2210,9 +2207,10 @@ __global__ __launch_bounds__(WG) void k_pk_compact(DevState st, int it_off) {
     const int pass = ld_coherent(&ctrl->pass);
     const int T = ld_coherent(&ctrl->thresh);
     if (blockIdx.x == 0 && threadIdx.x < NCLS) st.cnt[((it + 2) % 3) * NCLS + threadIdx.x] = 0;
-    if (blockIdx.x == 0) deferred_clear(ctrl, (pass + 1) % 3);
+    const int sums = st.deferred ? ld_coherent(&ctrl->win) : pass;  // as in k_pk_persistent
+    if (blockIdx.x == 0) deferred_clear(ctrl, (sums + 1) % 3);
     pk_compaction<4, false>(st, st.cnt + (it % 3) * NCLS, st.queue[it & 1], st.qmask[it & 1], T, ld_coherent(&ctrl->full) != 0,
-                  pass % 3);
+                  sums % 3);
 }
 
 // Every vertex's bound, once: between the compaction and the decision that records the offsets (no
