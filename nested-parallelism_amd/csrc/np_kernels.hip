@@ -570,11 +570,19 @@ __device__ __forceinline__ void deferred_clear(Ctrl *ctrl, int slot) {
 constexpr int COMPACT_UNR = 4;
 // Words a wavefront takes at once, 8 to 64: about 512 workgroups get a tile, because every tile
 // reserves its classes' queue slots on the same cache lines, where atomics take turns (a tile for
-// each of 2,048 workgroups made the heaviest compactions of 4.2 M vertices 75 -> 95 us).
-__device__ __forceinline__ int compact_words(long long nwords) {
-    const long long wgs = gridDim.x < 512 ? gridDim.x : 512;
-    const long long share = (nwords + wgs * WAVES - 1) / (wgs * WAVES);
-    return share < 8 ? 8 : share < 64 ? (int)share : 64;
+// each of 2,048 workgroups made the heaviest compactions of 4.2 M vertices 75 -> 95 us).  A windowed
+// pack reads a row of distances per vertex: from 4 words on, and 1,024 workgroups where 512 would
+// take more than 32 (persistent drive, 16 sources of ER 65,536 2.95 ms with 8, 1.97 with 4; 3 sources
+// of a 2048^2 grid, window 8,000: 6.56 ms with 512, 6.21 with 1,024; of 1200^2, 22 words each, launches 5.94 and 6.23).
+__host__ __device__ __forceinline__ int compact_words(long long nwords, int grid, bool windowed) {
+    auto share = [&](long long most) {
+        const long long waves = (grid < most ? grid : most) * WAVES;
+        return (nwords + waves - 1) / waves;
+    };
+    long long w = share(512);
+    if (windowed && w > 32) w = share(1024) > 32 ? share(1024) : 32;
+    const long long least = windowed ? 4 : 8;
+    return (int)(w < least ? least : w < 64 ? w : 64);
 }
 template <int UNROLL>
 __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const unsigned char *cls, const int *seg_off,
@@ -589,7 +597,7 @@ __device__ __forceinline__ void compaction_impl(Ctrl *ctrl, unsigned *bm, const 
     int my_dc = 0, my_dm = NO_WINDOW;
     const int lane = tid & 63, half = lane & 31;
     unsigned short *list = s_list[tid >> 6];
-    const int wt = compact_words(nwords);
+    const int wt = compact_words(nwords, gridDim.x, false);
     const long long tile = (long long)WAVES * wt;
     for (long long wb = (long long)blockIdx.x * tile; wb < nwords; wb += (long long)gridDim.x * tile) {
         if (tid < NCLS) s_lc[tid] = 0;
@@ -1952,7 +1960,7 @@ __device__ __forceinline__ void pk_compaction(const DevState &st, int *cnt_out, 
     const int lane = tid & 63, half = lane & 31;
     unsigned short *list = s_list[tid >> 6];
     int *wc = s_wc[tid >> 6];
-    const int wt = compact_words(st.nwords);
+    const int wt = compact_words(st.nwords, gridDim.x, st.deferred != nullptr);
     const long long tile = (long long)WAVES * wt;
     for (long long wb = (long long)blockIdx.x * tile; wb < st.nwords; wb += (long long)gridDim.x * tile) {
         const long long w0 = wb + (tid >> 6) * wt;
@@ -2786,11 +2794,11 @@ hipError_t launch_persistent(const DevState &st, const SchedDev &sp, bool batch,
 
 hipError_t launch_compact(const DevState &st, int it_off, bool batch, int wgs, hipStream_t s) {
     (void)batch;
-    // a workgroup per tile of 8 words per wavefront, up to the 512 that compact_words has in view (a
+    // a workgroup per tile, up to the ones that compact_words has in view (a
     // workgroup per 8,192 vertices left 8 of them on 65,536, each with 8 tiles in turn: 4 sources of
     // R-MAT s16 1.04 -> 0.91 ms, of grid 256^2 1.91 -> 1.41, one of ER 65,536 0.79 -> 0.66)
-    const long long need = (st.nwords + WAVES * 8 - 1) / (WAVES * 8);
-    const int g = (int)std::min<long long>(std::max<long long>(need, 1), std::min(wgs, 512));
+    const long long tile = (long long)WAVES * compact_words(st.nwords, wgs, st.deferred != nullptr);
+    const int g = (int)std::min<long long>(std::max<long long>((st.nwords + tile - 1) / tile, 1), wgs);
     if (st.kshift >= 0) {
         hipLaunchKernelGGL(k_pk_compact, dim3(g), dim3(WG), 0, s, st, it_off);
         if (st.bound) hipLaunchKernelGGL(k_pk_bounds, dim3(wgs), dim3(WG), 0, s, st);
