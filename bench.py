@@ -939,9 +939,10 @@ def run_config(npa, ctx, args):
     kernel += " (%s drive)" % {0: "persistent", 1: "host-loop", 2: "graph"}[scheds[head].drive]
     achieved = per_launch_bytes / (hr["launch_ms"] * 1e-3) / 1e9
     traffic, traffic_note = roofline_traffic(args, args.config, head, scheds[head], head in batches)
-    # work of one traced solve of the fastest mode (not timed): edge rows read (out-degrees of the queued
-    # vertices), (edge, source) items and queued (vertex, source) pairs; for packs the mean number of
-    # sources pending per edge row read and the re-expansion of pairs over the reached ones
+    # work of one traced solve of the fastest mode (not timed): out-degrees of the queued vertices
+    # (edge_rows: edges looked at; those that the bound filter drops read a byte of their target instead of
+    # its row of distances), (edge, source) items before the filter and queued (vertex, source) pairs; for
+    # packs the mean number of sources pending per such edge and the re-expansion of pairs over the reached ones
     work = None
     if head in batches:
         st = batches[head].solve(scheds[head].copy(trace=1))

@@ -88,7 +88,9 @@ typedef struct np_sched {
                             (0 = chosen by the graph's edges and its rows' lengths) */
     int32_t graph_chunk; /* NP_DRIVE_GRAPH: iterations per captured chunk (0 = 16) */
     int32_t max_iters;   /* 0 = no cap beyond n+1 */
-    int32_t trace;       /* nonzero: record per-iteration trace (np_trace_*) */
+    int32_t trace;       /* nonzero: record per-iteration trace (np_trace_*).  A traced solve keeps
+                            every iteration on the whole grid, where one without a trace runs
+                            small frontiers on one workgroup */
     int32_t scheme;      /* NP_SCHEME_*: 0 = the consolidation bins above; others are the
                             reference's other schedules (config.solution) */
     int32_t delta;       /* scan frontier: priority window.  0 = every flagged vertex is
@@ -153,7 +155,9 @@ typedef struct np_stats {
                                frontier_total except in source-packed batch parts */
     int64_t edges_total;    /* source-packed parts of traced solves (sched.trace) on the
                                host-loop and graph drives: sum over iterations of the
-                               out-degrees of the queued vertices (edge rows read); 0 elsewhere */
+                               out-degrees of the queued vertices (edges looked at; where
+                               the bound filter is on most of them read one byte of their
+                               target and no row of distances); 0 elsewhere */
     int64_t items_total;    /* same solves: sum of out-degree x queued sources ((edge, source)
                                relaxations attempted); 0 elsewhere */
     int64_t reserved[2];

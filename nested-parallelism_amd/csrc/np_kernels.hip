@@ -36,8 +36,8 @@ static constexpr unsigned long long SPIN_LIMIT = 1ull << 24;
 // threadIdx.x for one phase of a persistent kernel.  What a phase derives from it is the same in every
 // iteration, so the compiler would compute it once, before the loop, and hold it in registers through
 // all other phases; behind this it is computed again where it is used.  k_persistent 130 (with the
-// small-frontier path 150) -> 93 (110) VGPRs, 3 -> 5 (4) workgroups per CU; k_pk_persistent 156 -> 120,
-// 3 -> 4; k_pk_expand (64 at most) no longer spills.  A limit on the registers alone (waves_per_eu)
+// small-frontier path 150) -> 95 (117) VGPRs, 3 -> 5 (4) workgroups per CU; k_pk_persistent without a
+// window 156 -> 124, 3 -> 4; k_pk_expand (64 at most) no longer spills.  A limit on the registers alone (waves_per_eu)
 // gave the same count and lost it again: every wavefront had fewer loads in flight.
 __device__ __forceinline__ int phase_tid() {
     int t = threadIdx.x;
@@ -1503,9 +1503,10 @@ __device__ __forceinline__ void pk_relax_vertex(const DevState &st, int u, unsig
 // value.  An edge (u, v) with min over u's pending s of (dist[u][s] - off[s]) + w >= bound[v] can
 // improve no source, so it is dropped after reading one byte.  The bounds are upper bounds whatever
 // off[] is (any constants would do) and stay valid without upkeep, because distances only fall; a
-// vertex's bound is refreshed when it is expanded.  Sources that had not reached the hub when off[]
-// was taken (fmask clear) have no part in the bounds, and edges of a vertex pending for one of them
-// are never dropped.  16 sources of R-MAT s24, one solve: the four heaviest filtered expansions
+// vertex's bound is refreshed when it is expanded, as a tile, by a wavefront or by the whole grid.
+// Rows in the workgroup bin (level 1, from class PK_TILE_CLS on) are neither filtered nor refreshed.
+// Sources that had not reached the hub when off[] was taken (fmask clear) have no part in the bounds,
+// and edges of a vertex pending for one of them are never dropped.  16 sources of R-MAT s24, one solve: the four heaviest filtered expansions
 // 5.2 / 4.8 / 3.7 / 1.6 -> 4.1 / 3.2 / 2.4 / 1.1 ms, for 0.29 ms of bounds; what is left of them is
 // the stream of the rows themselves.
 // A byte holds ceil((bound - FBASE) / 2^fshift) with FBASE = -64 steps, 255 = no bound.

@@ -18,9 +18,9 @@
 // in-degree (bins built once): fewer than 32 in-edges, 8 lanes per vertex (consecutive in-edges,
 // coalesced); up to PR_HUGE, one wavefront per vertex; longer (R-MAT hubs reach 10^5 in-edges, a
 // single wavefront on one would be the whole pass's tail), PR_CHUNK-entry chunks on one wavefront
-// each, whose partial sums the wavefront that finishes last adds in chunk order, so results do not
-// depend on scheduling.  All in
-// float64, so the reference's EPSILON is reachable (float ranks near 1000/n cannot move by
+// each, whose partial sums the wavefront that finishes last adds in chunk order, so a row's sum does
+// not depend on scheduling.  The dangling sum does, in its last bits: it is added up by atomics in
+// order of arrival.  All in float64, so the reference's EPSILON is reachable (float ranks near 1000/n cannot move by
 // less than an ulp ~1e-9); ranks are returned as float32, the reference's FLOAT_T.  The file also
 // holds SpMV (apps/SpMV), the same row-split product without PageRank's terms.
 #include <hip/hip_runtime.h>
