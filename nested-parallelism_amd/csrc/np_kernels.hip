@@ -36,7 +36,7 @@ static constexpr unsigned long long SPIN_LIMIT = 1ull << 24;
 // threadIdx.x for one phase of a persistent kernel.  What a phase derives from it is the same in every
 // iteration, so the compiler would compute it once, before the loop, and hold it in registers through
 // all other phases; behind this it is computed again where it is used.  k_persistent 130 (with the
-// small-frontier path 150) -> 95 (117) VGPRs, 3 -> 5 (4) workgroups per CU; k_pk_persistent without a
+// small-frontier path 150) -> 93 (116) VGPRs, 3 -> 5 (4) workgroups per CU; k_pk_persistent without a
 // window 156 -> 124, 3 -> 4; k_pk_expand (64 at most) no longer spills.  A limit on the registers alone (waves_per_eu)
 // gave the same count and lost it again: every wavefront had fewer loads in flight.
 __device__ __forceinline__ int phase_tid() {
@@ -909,7 +909,7 @@ __device__ __forceinline__ int solo_iterations(const DevState &st, const ItemTab
 // ------------------------------------------------------------------------------------
 // persistent drive
 // ------------------------------------------------------------------------------------
-// SOLO: small frontiers run on one workgroup.  The registers of that (117 against 95) cost a workgroup
+// SOLO: small frontiers run on one workgroup.  The registers of that (116 against 93) cost a workgroup
 // per CU, 4 instead of 5, so graphs that want more go without (persistent_wgs in np_api.cpp).
 template <bool BATCH, bool UNIT, bool PUSH, bool SOLO>
 __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
@@ -921,28 +921,29 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
     long long t_prev = 0;
     // priority window: every workgroup computes the same sequence of thresholds
     int T = (!PUSH && sp.delta > 0) ? sp.delta : NO_WINDOW;
-    int pass = 0;
-    int extra = 0;  // iterations run by one workgroup alone, beyond one per trip
+    int next = 0;  // counters and sums of the next compaction pass
     for (int it = 0;; ++it) {
-        const int tid = phase_tid();
-        int *cnt_cur = st.cnt + (it % 3) * NCLS;
-        int *cnt_zero = st.cnt + ((it + 2) % 3) * NCLS;
         int *q_cur = st.queue[it & 1];
-        if (blockIdx.x == 0 && tid == 0) {
+        if (blockIdx.x == 0 && phase_tid() == 0) {
             long long now = (long long)wall_clock64();
             if (it > 0 && sp.trace && it - 1 < sp.trace_cap) sp.trace[it - 1].t_end = now;
             t_prev = now;
         }
-        if (blockIdx.x == 0 && tid < NCLS) st_coherent(cnt_zero + tid, 0);
+        if (PUSH && blockIdx.x == 0 && threadIdx.x < NCLS) st_coherent(st.cnt + ((it + 2) % 3) * NCLS + threadIdx.x, 0);
         for (;;) {
-            const int slot = pass % 3;
+            const int slot = next;
+            // every pass has counters of its own: one that queues nothing is followed by the next without
+            // a barrier, while slower workgroups are still reading its zeros
+            const int *cnt_cur = st.cnt + (PUSH ? it % 3 : slot) * NCLS;
             if (!PUSH) {
-                // the statistics slot of the next pass was last read before the previous barrier
-                if (blockIdx.x == 0 && T != NO_WINDOW) deferred_clear(ctrl, (pass + 1) % 3);
-                compaction_impl<SOLO ? COMPACT_UNR : COMPACT_UNR - 1>(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, cnt_cur, q_cur, st.dist, T, slot);
+                // the counters and the statistics slot of the next pass were last read before the previous barrier
+                next = slot == 2 ? 0 : slot + 1;
+                if (blockIdx.x == 0 && phase_tid() < NCLS) st_coherent(st.cnt + next * NCLS + phase_tid(), 0);
+                if (blockIdx.x == 0 && T != NO_WINDOW) deferred_clear(ctrl, next);
+                compaction_impl<SOLO ? COMPACT_UNR : COMPACT_UNR - 1>(st.ctrl, st.bm[0], st.cls, st.seg_off, st.nwords, st.cnt + slot * NCLS, q_cur, st.dist, T, slot);
                 if (!grid_sync(ctrl, nb, gen)) return;
-                pass++;
             }
+            const int tid = phase_tid();
             if (tid < NCLS) {
                 tb.cnt[tid] = ld_coherent(cnt_cur + tid);
                 tb.seg[tid] = st.seg_off[tid];
@@ -958,13 +959,13 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
             int kept, mn;
             deferred_sums(ctrl, slot, &kept, &mn);
             if (kept == 0) break;
-            T = mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta;
+            T = __builtin_amdgcn_readfirstlane(mn > NO_WINDOW - sp.delta ? NO_WINDOW : mn + sp.delta);
         }
-        const int total = s_total;
-        const int done_iters = it + extra;
-        if (total == 0 || (sp.max_iters > 0 && done_iters >= sp.max_iters)) {
+        const int tid = phase_tid();
+        const int total = __builtin_amdgcn_readfirstlane(s_total);
+        if (total == 0 || (sp.max_iters > 0 && it >= sp.max_iters)) {
             if (blockIdx.x == 0 && tid == 0) {
-                ctrl->iters = done_iters;
+                ctrl->iters = it;
                 ctrl->done = total == 0 ? 1 : 0;
                 if (total != 0) ctrl->error = NP_ERR_NOT_CONVERGED;
             }
@@ -973,16 +974,16 @@ __global__ __launch_bounds__(WG) void k_persistent(DevState st, SchedDev sp) {
         if (SOLO && T == NO_WINDOW && !sp.trace && solo_fits(tb, total)) {
             __shared__ SoloBufs s_solo;
             int most = SOLO_ITERS;
-            if (sp.max_iters > 0 && sp.max_iters - done_iters < most) most = sp.max_iters - done_iters;
+            if (sp.max_iters > 0 && sp.max_iters - it < most) most = sp.max_iters - it;
             if (blockIdx.x == 0) {
                 const int k = solo_iterations<BATCH, UNIT>(st, tb, q_cur, s_solo, total, most);
                 if (tid == 0) st_coherent(&ctrl->solo, k);
             }
             if (!grid_sync(ctrl, nb, gen)) return;
-            extra += ld_coherent(&ctrl->solo) - 1;
+            it += __builtin_amdgcn_readfirstlane(ld_coherent(&ctrl->solo)) - 1;
             continue;
         }
-        Cfg cfg = decide(sp, tb.cnt, done_iters);
+        Cfg cfg = decide(sp, tb.cnt, it);
         if (tid < 64) build_tables(tb, cfg, TABLES_SINGLE, (long long)nb * WAVES);
         if (blockIdx.x == 0 && tid < 64) {
             if (tid == 0) ctrl->frontier_total += total;
@@ -2144,8 +2145,6 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
     int pass = 0, win = 0;
     for (int it = 0;; ++it) {
         const int tid = phase_tid();
-        int *cnt_cur = st.cnt + (it % 3) * NCLS;
-        int *cnt_zero = st.cnt + ((it + 2) % 3) * NCLS;
         int *q_cur = st.queue[it & 1];
         unsigned *qm_cur = st.qmask[it & 1];
         if (blockIdx.x == 0 && tid == 0) {
@@ -2153,8 +2152,10 @@ __global__ __launch_bounds__(WG) void k_pk_persistent(DevState st, SchedDev sp) 
             if (it > 0 && sp.trace && it - 1 < sp.trace_cap) sp.trace[it - 1].t_end = now;
             t_prev = now;
         }
-        if (blockIdx.x == 0 && tid < NCLS) st_coherent(cnt_zero + tid, 0);
         for (;;) {
+            // every pass has counters of its own, as in k_persistent
+            int *cnt_cur = st.cnt + (pass % 3) * NCLS;
+            if (blockIdx.x == 0 && tid < NCLS) st_coherent(st.cnt + ((pass + 1) % 3) * NCLS + tid, 0);
             // the sums of a window, or of a pass (held vertices); the next ones' were last read before
             // the previous barrier
             const int sums = st.deferred ? win : pass;
