@@ -527,11 +527,14 @@ def live_traffic(args, config, sch):
     """HBM bytes of one solve of schedule sch, measured in this run: two child processes build the
     same workload and run the solve under rocprofv3 --pmc, one for FETCH_SIZE and one for
     WRITE_SIZE.  Each counter is scaled by what it reads for a 1 GiB device-to-device copy in the
-    same child (a copy reads and writes exactly 1 GiB).  Returns (bytes, note) or (None, reason)."""
+    same child (a copy reads and writes exactly 1 GiB).  Not on the persistent drive.  Returns
+    (bytes, note) or (None, reason)."""
     import shutil
     import tempfile
     if any(k.startswith("ROCPROF") for k in os.environ):
         return None, "bench.py itself runs under rocprofv3"
+    if sch.drive == 0:  # persistent: rocprofv3 ends cooperative launches with a segmentation fault, or not at all
+        return None, "not measured live on the persistent drive"
     prof = shutil.which("rocprofv3") or "/opt/rocm/bin/rocprofv3"
     if not os.path.exists(prof):
         return None, "rocprofv3 not found"

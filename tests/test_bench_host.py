@@ -62,3 +62,12 @@ def test_sched_arg_round_trips(bench, npa):
     t = npa.Sched(level=v[0], log2_t_lo=v[1], log2_t_hi=v[2], wgs_per_cu=v[3], drive=v[4], delta=v[5],
                   pack_hold=v[6])
     assert repr(t) == repr(s)
+
+
+def test_no_live_traffic_on_the_persistent_drive(bench, npa, monkeypatch):
+    """No profiler is started for a cooperative launch."""
+    monkeypatch.setattr(bench, "_counter_pass", lambda *a: pytest.fail("profiled"))
+    for k in [k for k in os.environ if k.startswith("ROCPROF")]:
+        monkeypatch.delenv(k)
+    b, why = bench.live_traffic(None, "c5", npa.Sched(level=2, drive=npa.DRIVE_PERSISTENT, delta=2002))
+    assert b is None and "persistent" in why
